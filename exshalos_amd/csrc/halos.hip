@@ -21,16 +21,21 @@
 #include "kernels.hpp"
 #include "util.hpp"
 
+#include <algorithm>
+
 namespace exh {
 
 static constexpr int FLAG_FREE = -1;
 static constexpr int FLAG_REJECTED = -2;
 static constexpr int S_TAB_MAX = 1024;  // largest r^2 a halo may reach
 
-__device__ inline size_t cell_off(int ci, int cj, int ck, unsigned p, int n0, int n1, int n2) {
+// Cell at packed offset p from (ci, cj, ck), periodic; cells are below 2^30.
+__device__ inline unsigned cell_off(int ci, int cj, int ck, unsigned p, int n0, int n1, int n2) {
   int di = (int)(p & 255u) - 128, dj = (int)((p >> 8) & 255u) - 128,
       dk = (int)((p >> 16) & 255u) - 128;
-  return ((size_t)wrap1(ci, di, n0) * n1 + wrap1(cj, dj, n1)) * n2 + wrap1(ck, dk, n2);
+  return ((unsigned)wrap1(ci, di, n0) * (unsigned)n1 + (unsigned)wrap1(cj, dj, n1)) *
+             (unsigned)n2 +
+         (unsigned)wrap1(ck, dk, n2);
 }
 
 // ---------------------------------------------------------------------------
@@ -182,20 +187,6 @@ __global__ void k_cand_setup(const T* skey, const int* scell, long long np, long
   }
 }
 
-// Block counts of the non-negative entries of v (PK_TILE entries a block),
-// for the in-order compaction of the retry list.
-__global__ void k_nonneg_count(const int* v, const long long* dn, long long* bcnt) {
-  __shared__ long long sh[4];
-  const long long n = *dn;
-  long long base = (long long)blockIdx.x * PK_TILE + (long long)threadIdx.x * PK_ITEMS;
-  long long cnt = 0;
-  for (int q = 0; q < PK_ITEMS; q++)
-    if (base + q < n && v[base + q] >= 0) cnt++;
-  long long tot;
-  block_exclusive_256<long long>(cnt, sh, &tot);
-  if (threadIdx.x == 0) bcnt[blockIdx.x] = tot;
-}
-
 // Order of the first round: columns of BR x BR cells in (i, j) over all k
 // ("bricks"), one after the other, and within a brick by blocks of ORD_RB
 // consecutive ranks (similar densities, hence similar growth work per
@@ -204,6 +195,7 @@ __global__ void k_nonneg_count(const int* v, const long long* dn, long long* bcn
 static constexpr int ORD_RB = 4096;
 static constexpr int RT_RING = 16;   // device ring of per-round pending counts
 static constexpr int RT_BATCH = 4;   // rounds per host read after the first
+static constexpr int NXCD = 8;       // accelerator dies: lists of pending candidates
 static constexpr int ORD_MAXB = 8192;  // bricks (LDS ints)
 
 __device__ inline int brick_of(int cell, int n1, int n2, int bsh, int nby) {
@@ -262,44 +254,6 @@ __global__ void k_brick_scatter(const int* ccell, const T* cden, long long nc, i
   }
 }
 
-// In-order compaction of the candidates to retry (retry[t] >= 0), carrying
-// their cell and density along.
-template <typename T>
-__global__ void k_retry_write(const int* retry, const long long* dn, const long long* boff,
-                              long long nbk, const int* cell_in, const T* den_in, int* rank_out,
-                              int* cell_out, T* den_out, long long* dnext) {
-  __shared__ long long sh[4];
-  const long long n = *dn;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *dnext = boff[nbk];  // next round's count
-  long long base = (long long)blockIdx.x * PK_TILE + (long long)threadIdx.x * PK_ITEMS;
-  // the thread's entries, cells and densities are all loaded before the
-  // first store (which could alias them for the compiler)
-  int rv[PK_ITEMS], cv[PK_ITEMS];
-  T dv[PK_ITEMS];
-  long long cnt = 0;
-#pragma unroll
-  for (int q = 0; q < PK_ITEMS; q++) {
-    rv[q] = base + q < n ? retry[base + q] : -1;
-    cnt += rv[q] >= 0;
-  }
-#pragma unroll
-  for (int q = 0; q < PK_ITEMS; q++)
-    if (rv[q] >= 0) {
-      cv[q] = cell_in[base + q];
-      dv[q] = den_in[base + q];
-    }
-  long long tot;
-  long long o = block_exclusive_256<long long>(cnt, sh, &tot) + boff[blockIdx.x];
-#pragma unroll
-  for (int q = 0; q < PK_ITEMS; q++)
-    if (rv[q] >= 0) {
-      rank_out[o] = rv[q];
-      cell_out[o] = cv[q];
-      den_out[o] = dv[q];
-      o++;
-    }
-}
-
 // number of keys below Bmin (the first candidate's sorted position); *out
 // starts at zero
 template <typename T>
@@ -316,22 +270,10 @@ __global__ void k_count_below(const T* key, long long n, T Bmin, unsigned long l
     atomicAdd(out, (unsigned long long)(sh[0] + sh[1] + sh[2] + sh[3]));
 }
 
-__global__ void k_fill_i32(int* p, long long n, int v) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x)
-    p[i] = v;
-}
-
 __global__ void k_fill_u64(unsigned long long* p, long long n, unsigned long long v) {
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x)
     p[i] = v;
-}
-
-__global__ void k_iota(int* p, long long n) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x)
-    p[i] = (int)i;
 }
 
 // ---------------------------------------------------------------------------
@@ -373,210 +315,445 @@ __device__ inline void decode_cell(int cell, int n1, int n2, int& i, int& j, int
   i = r / n1;
 }
 
-// Workgroup w runs on XCD w mod 8: give each XCD a contiguous range of
-// blocks, so that a round's consecutive candidates (neighbours in space)
-// share one L2.
-__device__ inline int xcd_block(unsigned nb) {
-  const unsigned w = blockIdx.x;
-  const unsigned q = nb / 8, rem = nb % 8, x = w % 8;
-  return (int)(x * q + (x < rem ? x : rem) + w / 8);
+// A round's pending candidates stand in NXCD lists, list x at positions
+// [x cap, x cap + n_x) of the arrays by list position, with its count n_x on
+// the device.  Workgroup w, which runs on XCD w mod 8, takes CPB consecutive
+// candidates of list w mod 8: consecutive candidates (neighbours in space)
+// share one L2, and a candidate that must retry stays in its XCD's list, so
+// the next round keeps that.  The grid may be larger than the lists (sized by
+// an earlier round's counts); its extra blocks return.
+struct RoundLists {
+  const int* n;   // [NXCD] this round's counts
+  int* next;      // [NXCD] the next round's (zero on entry; k_commit adds)
+  int* clear;     // [NXCD] the round's after that, zeroed by k_grow
+  int cap;
+  int *rank_out, *cell_out;  // the next round's lists (densities in pden_out)
+};
+
+// A table that no kernel of the rounds writes, read through the scalar cache
+// where the index is uniform.
+__device__ __forceinline__ int table_at(const int* p, int i) {
+  return ((const int __attribute__((address_space(4)))*)(uintptr_t)p)[i];
 }
 
-// The round's count is read on the device (*dn): the grid may be larger
-// (sized by an earlier round's count) and its extra blocks return.
+// Value of lane E of the lane's row of 16 (row_newbcast).
+template <int E>
+__device__ __forceinline__ float row_lane(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + E, 0xf, 0xf, true));
+}
+template <int E>
+__device__ __forceinline__ double row_lane(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + E, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + E, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// s += v of lanes 0 .. nb - 1 of the row, in lane order (nb the same in the
+// whole wave).  The lanes past nb hold zeros, which leave s unchanged, so
+// four lanes are added at a time: one branch per four cells.
+template <int E, typename T>
+__device__ __forceinline__ void row_add(double& s, T v, int nb) {
+  if constexpr (E < 16) {
+    if (nb > E) {
+      s += (double)row_lane<E>(v);
+      s += (double)row_lane<E + 1>(v);
+      s += (double)row_lane<E + 2>(v);
+      s += (double)row_lane<E + 3>(v);
+      row_add<E + 4>(s, v, nb);
+    }
+  }
+}
+// s -= v of the row's lanes, in lane order, zeros past the last cell.
+template <int E, typename T>
+__device__ __forceinline__ void row_sub(double& s, T v) {
+  if constexpr (E < 16) {
+    s -= (double)row_lane<E>(v);
+    row_sub<E + 1>(s, v);
+  }
+}
+
+// The row's values of f at cells [o, min(o + 64, o1)) of the shell table,
+// 16 cells in each v[k], in lane order and zeros past o1.  The offsets of the first SH_LDS
+// cells are read from LDS: a load of theirs from memory would wait behind
+// the loads of values in flight.
+static constexpr int ROW_K = 4;
+static constexpr int SH_LDS = 1024;
+template <typename T>
+__device__ __forceinline__ void row_load(T (&v)[ROW_K], const T* f, const unsigned* lds_offs,
+                                         const unsigned* offs, int o, int o1, int lane, int ci,
+                                         int cj, int ck, int n0, int n1, int n2) {
+#pragma unroll
+  for (int k = 0; k < ROW_K; k++) {
+    if (o + 16 * k >= o1) break;
+    const int e = o + 16 * k + lane;
+    v[k] = 0;
+    if (e < o1) {
+      const unsigned p = o1 <= SH_LDS ? lds_offs[e] : offs[e];
+      v[k] = f[cell_off(ci, cj, ck, p, n0, n1, n2)];
+    }
+  }
+}
+
 // Claims are 64-bit (round tag << 32 | ~rank) or, with fewer than 2^24
 // candidates, 32-bit (round tag << 24 | (2^24 - 1 - rank)): atomicMax keeps
 // the densest claim of the current round, and any claim of the round beats
 // those of earlier rounds.
-template <typename T, bool C32>
-__global__ void k_grow(GrowArgs<T> a, const long long* dn, unsigned long long tag_hi) {
-  const int npend = (int)*dn;
-  const unsigned nba = (unsigned)((npend + 255) / 256);
-  if (blockIdx.x >= nba) return;
-  int t = xcd_block(nba) * blockDim.x + threadIdx.x;
-  if (t >= npend) return;
-  const int rank = a.prank[t];
-  const int cell = a.pcell[t];
-  if (a.flag[cell] != FLAG_FREE) {  // already inside a denser halo
-    a.pG[t] = -1;
-    a.kept[rank] = 0;
-    return;
-  }
-  int ci, cj, ck;
-  decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
-  const double Bmin = (double)a.Bmin;
-  double den = (double)a.pden[t], den_tmp = den;
-  int count = 0, count_tmp = 1, grows = 0, grows_tmp = 0;
-  while (den_tmp >= Bmin) {
-    if (count < count_tmp) grows = grows_tmp;
-    grows_tmp++;
-    if (grows_tmp >= a.sh.stab) {
-      atomicOr(a.err, 1);
-      a.pG[t] = -1;
-      return;
-    }
-    den = den_tmp;
-    count = count_tmp;
-    den_tmp = den * ((double)count);
-    // the shell's cells in cube order; loads issued in batches, summed in
-    // order (flagged cells hold -Mtot in eff, as the reference adds)
-    const int o0 = a.sh.start[grows_tmp], o1 = a.sh.start[grows_tmp + 1];
-    for (int ob = o0; ob < o1; ob += 8) {
-      T v[8];
-      const int nb = min(8, o1 - ob);
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (e < nb) v[e] = a.eff[cell_off(ci, cj, ck, a.sh.offs[ob + e], a.n0, a.n1, a.n2)];
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (e < nb) den_tmp += (double)v[e];
-      count_tmp += nb;
-    }
-    den_tmp = den_tmp / ((double)count_tmp);
-  }
-  const int G = grows_tmp;
-  for (;;) {
-    if (count >= a.nB) {
-      atomicOr(a.err, 2);
-      a.pG[t] = -1;
-      return;
-    }
-    if (!(den < (double)a.Bt[count] && count > 0)) break;
-    if (grows < 0) {  // cannot happen while count > 0 on an unclamped table
-      atomicOr(a.err, 32);
-      a.pG[t] = -1;
-      return;
-    }
-    den_tmp = den;
-    count_tmp = count;
-    den = den * ((double)count);
-    const int o0 = a.sh.start[grows], o1 = a.sh.start[grows + 1];
-    for (int ob = o0; ob < o1; ob += 8) {
-      T v[8];
-      const int nb = min(8, o1 - ob);
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (e < nb) v[e] = a.delta[cell_off(ci, cj, ck, a.sh.offs[ob + e], a.n0, a.n1, a.n2)];
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (e < nb) den -= (double)v[e];
-      count -= nb;
-    }
-    if (count > 0) den = den / ((double)count);
-    if (count < count_tmp) grows_tmp = grows;
-    grows--;
-  }
-  a.pG[t] = G;
-  a.pcnt[t] = count;
-  a.pr2[t] = grows_tmp;
-  // claim every cell the final halo could occupy (r^2 < G); the offsets
-  // of 8 cells are loaded before their atomics (which could alias them for
-  // the compiler)
-  const int oend = a.sh.start[G];
-  for (int ob = 0; ob < oend; ob += 8) {
-    const int nb = min(8, oend - ob);
-    unsigned off[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++)
-      if (e < nb) off[e] = a.sh.offs[ob + e];
-    if constexpr (C32) {
-      unsigned* cl = reinterpret_cast<unsigned*>(a.claim);
-      const unsigned tag = (unsigned)tag_hi | (0xffffffu - (unsigned)rank);
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (e < nb) atomicMax(&cl[cell_off(ci, cj, ck, off[e], a.n0, a.n1, a.n2)], tag);
-    } else {
-      const unsigned long long tag = tag_hi | (unsigned long long)(0xffffffffu - (unsigned)rank);
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (e < nb) atomicMax(&a.claim[cell_off(ci, cj, ck, off[e], a.n0, a.n1, a.n2)], tag);
-    }
+template <bool C32>
+__device__ __forceinline__ void claim_cell(unsigned long long* claim, unsigned id,
+                                           unsigned long long tag_hi, int rank) {
+  if constexpr (C32)
+    atomicMax(reinterpret_cast<unsigned*>(claim) + id,
+              (unsigned)tag_hi | (0xffffffu - (unsigned)rank));
+  else
+    atomicMax(claim + id, tag_hi | (unsigned long long)(0xffffffffu - (unsigned)rank));
+}
+
+// Whether a denser candidate has claimed cell id in this round.
+template <bool C32>
+__device__ __forceinline__ bool claimed(const unsigned long long* claim, unsigned id,
+                                        unsigned long long tag_hi, int rank) {
+  if constexpr (C32) {
+    const unsigned v = reinterpret_cast<const unsigned*>(claim)[id];
+    return (v & 0xff000000u) == (unsigned)tag_hi && (v & 0xffffffu) > 0xffffffu - (unsigned)rank;
+  } else {
+    const unsigned long long v = claim[id];
+    return (v & 0xffffffff00000000ull) == tag_hi &&
+           (unsigned)(v & 0xffffffffu) > 0xffffffffu - (unsigned)rank;
   }
 }
 
-// retry[t]: the rank again when candidate t must retry next round, else -1
-// (compacted in order, so the next round keeps this round's order).
-template <typename T, bool C32>
-__global__ void k_commit(GrowArgs<T> a, const long long* dn, unsigned long long tag_hi,
-                         int* retry, int tmax) {
-  const int npend = (int)*dn;
-  const unsigned nba = (unsigned)((npend + 255) / 256);
-  if (blockIdx.x >= nba) return;
-  int t = xcd_block(nba) * blockDim.x + threadIdx.x;
-  if (t >= npend) return;
-  const int rank = a.prank[t];
-  const int G = a.pG[t];
-  if (G < 0) {  // skipped or failed
-    retry[t] = -1;
-    return;
+// Growth of the round's candidates (find_halos.c:226-379), in two phases.
+//
+// One thread per candidate tests the flag and the first shell (6 cells).
+// Most candidates end there (81% of a 512^3 box's halos of 4 Mpc/h cells are
+// one cell), and they claim that cell.  The others go to a list in LDS, from
+// which each wave takes four at a time, one per row of 16 lanes: the row
+// loads a shell's cells in parallel, two shells ahead of the sum, and every
+// lane forms the reference's ordered double sum from the row's values
+// (row_newbcast moves).  A growth of n cells then waits for about one load
+// per shell and not for one per 8 cells, and a wave is held by the longest
+// of four growths and not of 64.
+template <typename T, bool C32, int CPB>
+__global__ __launch_bounds__(256) void k_grow(GrowArgs<T> a, RoundLists rl,
+                                              unsigned long long tag_hi) {
+  __shared__ double s_mean[CPB];
+  __shared__ int s_cell[CPB], s_rank[CPB];
+  __shared__ short s_at[CPB];
+  __shared__ unsigned s_offs[SH_LDS];
+  __shared__ int nlist, taken;
+  const int x = blockIdx.x % NXCD, t0 = (int)(blockIdx.x / NXCD) * CPB;
+  if (blockIdx.x < NXCD && threadIdx.x == 0) rl.clear[blockIdx.x] = 0;
+  const int n = rl.n[x];
+  if (t0 >= n) return;
+  const int base = x * rl.cap + t0, m = min(CPB, n - t0);
+  if (threadIdx.x == 0) {
+    nlist = 0;
+    taken = 0;
   }
-  const int cell = a.pcell[t];
-  int ci, cj, ck;
-  decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
-  // safe iff no denser pending candidate claims a cell of the read ball
-  const int oend = a.sh.start[G + 1];
-  bool blocked = false;
-  if constexpr (C32) {
-    const unsigned* cl = reinterpret_cast<const unsigned*>(a.claim);
-    const unsigned lim = 0xffffffu - (unsigned)rank, th = (unsigned)tag_hi;
-    for (int ob = 0; ob < oend && !blocked; ob += 8) {
-      unsigned v[8];
-      const int nb = min(8, oend - ob);
+  const int noffs = table_at(a.sh.start, a.sh.stab);
 #pragma unroll
-      for (int e = 0; e < 8; e++)
-        v[e] = e < nb ? cl[cell_off(ci, cj, ck, a.sh.offs[ob + e], a.n0, a.n1, a.n2)] : 0u;
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        blocked |= (v[e] & 0xff000000u) == th && (v[e] & 0xffffffu) > lim;
-    }
-  } else {
-    const unsigned lim = 0xffffffffu - (unsigned)rank;
-    for (int ob = 0; ob < oend && !blocked; ob += 8) {
-      unsigned long long v[8];
-      const int nb = min(8, oend - ob);
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        v[e] = e < nb ? a.claim[cell_off(ci, cj, ck, a.sh.offs[ob + e], a.n0, a.n1, a.n2)] : 0ull;
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        blocked |=
-            (v[e] & 0xffffffff00000000ull) == tag_hi && (unsigned)(v[e] & 0xffffffffu) > lim;
-    }
+  for (int q = 0; q < SH_LDS / 256; q++) {
+    const int e = (int)threadIdx.x + 256 * q;
+    s_offs[e] = e < noffs ? a.sh.offs[e] : 0u;
   }
-  retry[t] = blocked ? rank : -1;
-  if (blocked) return;
-  const int count = a.pcnt[t];
-  if (count == 0) {
-    a.kept[rank] = 0;
-    return;
-  }
-  const int R2 = a.pr2[t];
-  if (isqrt_floor(R2 - 1) > tmax) {  // flag sphere would wrap (reference writes past its cube)
-    atomicOr(a.err, 4);
-    a.kept[rank] = 0;
-    return;
-  }
-  bool keep = count >= a.Nmin;
-  int v = keep ? (rank << 1) : FLAG_REJECTED;
-  const int fend = a.sh.start[R2];
-  for (int ob = 0; ob < fend; ob += 8) {  // offsets of 8 cells before their stores
-    const int nb = min(8, fend - ob);
-    unsigned off[8];
+  __syncthreads();
+  const double Bmin = (double)a.Bmin;
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x < CPB) {
+    const int t = base + threadIdx.x;
+    bool more = false;
+    double mean = 0;
+    int rank = 0, cell = 0;
+    if ((int)threadIdx.x < m) {
+      rank = a.prank[t];
+      cell = a.pcell[t];
+      if (a.flag[cell] != FLAG_FREE) {  // already inside a denser halo
+        a.pG[t] = -1;
+        a.kept[rank] = 0;
+      } else {
+        int ci, cj, ck;
+        decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
+        T v[6];
 #pragma unroll
-    for (int e = 0; e < 8; e++)
-      if (e < nb) off[e] = a.sh.offs[ob + e];
+        for (int e = 0; e < 6; e++)
+          v[e] = a.eff[cell_off(ci, cj, ck, (unsigned)table_at((const int*)a.sh.offs, 1 + e),
+                                a.n0, a.n1, a.n2)];
+        double den = (double)a.pden[t];
+        mean = den * 1.0;
 #pragma unroll
-    for (int e = 0; e < 8; e++)
-      if (e < nb) {
-        const size_t id = cell_off(ci, cj, ck, off[e], a.n0, a.n1, a.n2);
-        a.flag[id] = v;
-        a.eff[id] = a.negMtot;
+        for (int e = 0; e < 6; e++) mean += (double)v[e];
+        mean = mean / 7.0;
+        more = mean >= Bmin;
+        if (!more) {
+          // one cell; below the barrier of one cell it shrinks to none
+          const bool one = !(den < (double)a.Bt[1]);
+          a.pG[t] = 1;
+          a.pcnt[t] = one ? 1 : 0;
+          a.pr2[t] = one ? 1 : 0;
+          claim_cell<C32>(a.claim, (unsigned)cell, tag_hi, rank);
+        }
       }
+    }
+    const unsigned long long bal = __ballot(more);
+    int at = 0;
+    if (bal && lane == 0) at = atomicAdd(&nlist, __popcll(bal));
+    at = __shfl(at, 0, 64) + __popcll(bal & lanemask_lt());
+    if (more) {
+      s_mean[at] = mean;
+      s_cell[at] = cell;
+      s_rank[at] = rank;
+      s_at[at] = (short)threadIdx.x;
+    }
   }
-  if (keep) a.flag[cell] = (rank << 1) | 1;
-  a.kept[rank] = keep ? 1 : 0;
-  a.cnt[rank] = count;
-  a.r2[rank] = R2;
+  __syncthreads();
+  const int nl = nlist, l16 = lane & 15, row = lane >> 4;
+  for (;;) {
+    int q = 0;
+    if (lane == 0) q = atomicAdd(&taken, 4);
+    q = __builtin_amdgcn_readfirstlane(q);
+    if (q >= nl) break;
+    const bool has = q + row < nl;
+    const int it = has ? q + row : q;  // an idle row follows the first one
+    const int cell = s_cell[it], rank = s_rank[it];
+    int ci, cj, ck;
+    decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
+    // growth from shell 2 on; count = start[s] cells lie inside shell s
+    double den = 0, mean = s_mean[it];
+    bool act = has;
+    int G = -1;
+    const int* start = a.sh.start;
+    T va[ROW_K], vb[ROW_K], vc[ROW_K];
+    int o0 = table_at(start, 2), o1 = table_at(start, 3), o2 = table_at(start, 4),
+        o3 = table_at(start, 5);
+    row_load(va, a.eff, s_offs, a.sh.offs, o0, o1, l16, ci, cj, ck, a.n0, a.n1, a.n2);
+    row_load(vb, a.eff, s_offs, a.sh.offs, o1, o2, l16, ci, cj, ck, a.n0, a.n1, a.n2);
+    for (int s = 2;; s++) {
+      if (s >= a.sh.stab) {  // rows still growing leave the table
+        if (act) atomicOr(a.err, 1);
+        break;
+      }
+      const int o4 = s + 3 < a.sh.stab ? table_at(start, s + 4) : o3;
+      row_load(vc, a.eff, s_offs, a.sh.offs, o2, o3, l16, ci, cj, ck, a.n0, a.n1, a.n2);
+      double sum = mean * (double)o0;
+#pragma unroll
+      for (int k = 0; k < ROW_K; k++)
+        if (o0 + 16 * k < o1) row_add<0>(sum, va[k], o1 - o0 - 16 * k);
+      for (int o = o0 + 16 * ROW_K; o < o1; o += 16 * ROW_K) {
+        row_load(va, a.eff, s_offs, a.sh.offs, o, o1, l16, ci, cj, ck, a.n0, a.n1, a.n2);
+#pragma unroll
+        for (int k = 0; k < ROW_K; k++)
+          if (o + 16 * k < o1) row_add<0>(sum, va[k], o1 - o - 16 * k);
+      }
+      sum = sum / (double)o1;
+      if (act) {
+        den = mean;
+        mean = sum;
+        if (!(mean >= Bmin)) {
+          act = false;
+          G = s;
+        }
+      }
+      if (!__ballot(act)) break;
+#pragma unroll
+      for (int k = 0; k < ROW_K; k++) {
+        va[k] = vb[k];
+        vb[k] = vc[k];
+      }
+      o0 = o1;
+      o1 = o2;
+      o2 = o3;
+      o3 = o4;
+    }
+    const int t = base + s_at[it];
+    if (G >= 0) {  // a row with a result: shrink it below the barrier
+      int grows = G - 1, grows_tmp = G, count = start[G];
+      while (start[grows + 1] == start[grows]) grows--;  // the last shell with cells
+      for (;;) {
+        if (count >= a.nB) {
+          if (l16 == 0) atomicOr(a.err, 2);
+          G = -1;
+          break;
+        }
+        if (!(den < (double)a.Bt[count] && count > 0)) break;
+        if (grows < 0) {  // cannot happen while count > 0 on an unclamped table
+          if (l16 == 0) atomicOr(a.err, 32);
+          G = -1;
+          break;
+        }
+        const int c1 = start[grows + 1], c0 = start[grows];
+        den = den * (double)count;
+        for (int o = c0; o < c1; o += 16 * ROW_K) {
+          row_load(va, a.delta, s_offs, a.sh.offs, o, c1, l16, ci, cj, ck, a.n0, a.n1, a.n2);
+#pragma unroll
+          for (int k = 0; k < ROW_K; k++)
+            if (o + 16 * k < c1) row_sub<0>(den, va[k]);
+        }
+        count -= c1 - c0;
+        if (count > 0) den = den / (double)count;
+        if (c1 > c0) grows_tmp = grows;
+        grows--;
+      }
+      if (G >= 0) {
+        if (l16 == 0) {
+          a.pcnt[t] = count;
+          a.pr2[t] = grows_tmp;
+        }
+        // claim every cell the final halo could occupy (r^2 < G)
+        const int oend = start[G];
+        for (int o = l16; o < oend; o += 16)
+          claim_cell<C32>(a.claim, cell_off(ci, cj, ck, a.sh.offs[o], a.n0, a.n1, a.n2), tag_hi,
+                          rank);
+      }
+    }
+    if (has && l16 == 0) a.pG[t] = G;
+  }
+}
+
+// Commit of the candidates that have seen their final flags: no denser
+// pending candidate claims a cell of their read ball (r^2 <= G).  As in
+// k_grow, one thread handles a candidate of one cell and a row of 16 lanes a
+// larger one.  The others are appended to their XCD's list of the next round
+// (in the order of the workgroups' atomics: the order of a list does not
+// change the result), in place of a count, a scan and a write pass (12 us a
+// round).  All rounds of the two boxes above: 283 -> 60 us, 2.6 -> 0.6 ms.
+template <typename T, bool C32, int CPB>
+__global__ __launch_bounds__(256) void k_commit(GrowArgs<T> a, RoundLists rl, T* pden_out,
+                                                unsigned long long tag_hi, int tmax) {
+  __shared__ short s_at[CPB];
+  __shared__ unsigned char s_retry[CPB];
+  __shared__ int nlist, taken, s_wave[4], s_base;
+  const int x = blockIdx.x % NXCD, t0 = (int)(blockIdx.x / NXCD) * CPB;
+  const int n = rl.n[x];
+  if (t0 >= n) return;
+  const int base = x * rl.cap + t0, m = min(CPB, n - t0);
+  if (threadIdx.x == 0) {
+    nlist = 0;
+    taken = 0;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x < CPB) {
+    const int t = base + threadIdx.x;
+    bool more = false, retry = false;
+    if ((int)threadIdx.x < m) {
+      const int G = a.pG[t];  // -1: skipped or failed
+      more = G > 1;
+      if (G == 1) {
+        const int rank = a.prank[t], cell = a.pcell[t], count = a.pcnt[t];
+        int ci, cj, ck;
+        decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
+#pragma unroll
+        for (int e = 0; e < 7; e++)
+          retry |= claimed<C32>(
+              a.claim,
+              cell_off(ci, cj, ck, (unsigned)table_at((const int*)a.sh.offs, e), a.n0, a.n1, a.n2),
+              tag_hi, rank);
+        if (!retry) {
+          const bool keep = count > 0 && count >= a.Nmin;
+          if (count > 0) {
+            a.flag[cell] = keep ? (rank << 1) | 1 : FLAG_REJECTED;
+            a.eff[cell] = a.negMtot;
+            a.cnt[rank] = count;
+            a.r2[rank] = 1;
+          }
+          a.kept[rank] = keep ? 1 : 0;
+        }
+      }
+    }
+    const unsigned long long bal = __ballot(more);
+    int at = 0;
+    if (bal && lane == 0) at = atomicAdd(&nlist, __popcll(bal));
+    at = __shfl(at, 0, 64) + __popcll(bal & lanemask_lt());
+    if (more) s_at[at] = (short)threadIdx.x;
+    s_retry[threadIdx.x] = retry;
+  }
+  __syncthreads();
+  const int nl = nlist, l16 = lane & 15, row = lane >> 4;
+  for (;;) {
+    int q = 0;
+    if (lane == 0) q = atomicAdd(&taken, 4);
+    q = __builtin_amdgcn_readfirstlane(q);
+    if (q >= nl) break;
+    if (q + row >= nl) continue;
+    const int at = s_at[q + row], t = base + at;
+    const int rank = a.prank[t], cell = a.pcell[t], G = a.pG[t], count = a.pcnt[t];
+    int ci, cj, ck;
+    decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
+    const int oend = a.sh.start[G + 1];
+    bool blocked = false;
+    for (int ob = 0; ob < oend && !blocked; ob += 64) {
+      unsigned p[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        p[k] = ob + 16 * k + l16 < oend ? a.sh.offs[ob + 16 * k + l16] : a.sh.offs[0];
+      bool hit = false;
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        hit |= claimed<C32>(a.claim, cell_off(ci, cj, ck, p[k], a.n0, a.n1, a.n2), tag_hi, rank);
+      blocked = ((__ballot(hit) >> (row * 16)) & 0xffffull) != 0;
+    }
+    if (blocked) {
+      if (l16 == 0) s_retry[at] = 1;
+      continue;
+    }
+    if (count == 0) {
+      if (l16 == 0) a.kept[rank] = 0;
+      continue;
+    }
+    const int R2 = a.pr2[t];
+    if (isqrt_floor(R2 - 1) > tmax) {  // flag sphere would wrap (reference writes past its cube)
+      if (l16 == 0) {
+        atomicOr(a.err, 4);
+        a.kept[rank] = 0;
+      }
+      continue;
+    }
+    const bool keep = count >= a.Nmin;
+    const int v = keep ? (rank << 1) : FLAG_REJECTED;
+    const int fend = a.sh.start[R2];
+    for (int o = l16; o < fend; o += 16) {  // cell 0 is the centre
+      const unsigned id = cell_off(ci, cj, ck, a.sh.offs[o], a.n0, a.n1, a.n2);
+      a.flag[id] = keep && o == 0 ? (rank << 1) | 1 : v;
+      a.eff[id] = a.negMtot;
+    }
+    if (l16 == 0) {
+      a.kept[rank] = keep ? 1 : 0;
+      a.cnt[rank] = count;
+      a.r2[rank] = R2;
+    }
+  }
+  __syncthreads();
+  // the candidates to retry, in this block's order
+  const bool retry = (int)threadIdx.x < m && s_retry[threadIdx.x % CPB] != 0;
+  const unsigned long long bal = __ballot(retry);
+  const int w = threadIdx.x >> 6;
+  if (lane == 0) s_wave[w] = __popcll(bal);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int tot = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+    s_base = tot ? atomicAdd(&rl.next[x], tot) : 0;
+  }
+  __syncthreads();
+  if (retry) {
+    int o = x * rl.cap + s_base + __popcll(bal & lanemask_lt());
+    for (int u = 0; u < w; u++) o += s_wave[u];
+    const int t = base + threadIdx.x;
+    const int rank = a.prank[t], cell = a.pcell[t];
+    const T den = a.pden[t];
+    rl.rank_out[o] = rank;
+    rl.cell_out[o] = cell;
+    pden_out[o] = den;
+  }
+}
+
+// Counts of the first round's lists (contiguous ranges of the candidates'
+// order) and the error flag after the ring.
+__global__ void k_round_init(int* rt, int nc, int cap) {
+  const int q = threadIdx.x;
+  if (q < NXCD) rt[q] = min(max(nc - q * cap, 0), cap);
+  if (q >= NXCD && q < 2 * NXCD) rt[q] = 0;
+  if (q == 2 * NXCD) rt[RT_RING * NXCD] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -724,55 +901,119 @@ __global__ void k_flag_out(const int* flag, long long ng, const long long* hidx,
   }
 }
 
-// halo displacement sums over the member sphere, in double
-template <typename T>
-__global__ void k_halo_posh(const int* hx, const int* hcount, const int* hr2, long long nh,
-                            ShellTab sh, int n0, int n1, int n2, const T* S, const T* V, T Lc,
-                            T L0, T L1, T L2, int lagrangian, T* posh, T* velh) {
-  for (long long h = blockIdx.x * (long long)blockDim.x + threadIdx.x; h < nh;
-       h += (long long)gridDim.x * blockDim.x) {
-    int ci = hx[3 * h], cj = hx[3 * h + 1], ck = hx[3 * h + 2];
+// Halo displacements: the mean over the member sphere, summed in double.  A
+// halo of one cell (81% of a 512^3 box's at 4 Mpc/h) takes one thread, a
+// larger one a row of 16 lanes that share its cells, so that no wave waits
+// for one thread's chain of loads through hundreds of cells.
+template <typename T, bool VEL>
+__device__ __forceinline__ void posh_store(const double* s, const double* v, int hc, int ci,
+                                           int cj, int ck, T Lc, T L0, T L1, T L2, T* posh,
+                                           T* velh, size_t h) {
+  const int q[3] = {ci, cj, ck};
+  const T L[3] = {L0, L1, L2};
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const T base = (T)((double)((T)q[a] * Lc) + (double)Lc / 2.0);
+    T r = base + (T)(s[a] / hc);
+    if (r >= L[a]) r -= L[a];
+    if (r < (T)0) r += L[a];
+    posh[3 * h + a] = r;
+    if constexpr (VEL) velh[3 * h + a] = (T)(v[a] / hc);
+  }
+}
+
+template <typename T, bool VEL>
+__global__ __launch_bounds__(256) void k_halo_posh(const int* hx, const int* hcount,
+                                                   const int* hr2, long long nh, ShellTab sh,
+                                                   int n0, int n1, int n2, const T* S, const T* V,
+                                                   T Lc, T L0, T L1, T L2, int lagrangian,
+                                                   T* posh, T* velh) {
+  __shared__ short s_at[256];
+  __shared__ int s_end[256];
+  __shared__ int nlist, taken;
+  using V3 = typename vec3<T>::type;
+  const long long h0 = blockIdx.x * 256ll, h = h0 + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) {
+    nlist = 0;
+    taken = 0;
+  }
+  __syncthreads();
+  int end = 0;
+  bool more = false;
+  if (h < nh) {
+    const int ci = hx[3 * h], cj = hx[3 * h + 1], ck = hx[3 * h + 2], hc = hcount[h];
+    end = lagrangian ? 0 : table_at(sh.start, hr2[h]);
+    more = end > 1;
+    if (!more) {
+      double s[3] = {0, 0, 0}, v[3] = {0, 0, 0};
+      if (end == 1) {
+        const size_t id = ((size_t)ci * n1 + cj) * n2 + ck;
+        const V3 a = *reinterpret_cast<const V3*>(S + 3 * id);
+        s[0] += (double)a.x;
+        s[1] += (double)a.y;
+        s[2] += (double)a.z;
+        if constexpr (VEL) {
+          const V3 u = *reinterpret_cast<const V3*>(V + 3 * id);
+          v[0] += (double)u.x;
+          v[1] += (double)u.y;
+          v[2] += (double)u.z;
+        }
+      }
+      posh_store<T, VEL>(s, v, hc, ci, cj, ck, Lc, L0, L1, L2, posh, velh, h);
+    }
+  }
+  const unsigned long long bal = __ballot(more);
+  int at = 0;
+  if (bal && lane == 0) at = atomicAdd(&nlist, __popcll(bal));
+  at = __shfl(at, 0, 64) + __popcll(bal & lanemask_lt());
+  if (more) {
+    s_at[at] = (short)threadIdx.x;
+    s_end[at] = end;
+  }
+  __syncthreads();
+  const int nl = nlist, l16 = lane & 15, row = lane >> 4;
+  for (;;) {
+    int q = 0;
+    if (lane == 0) q = atomicAdd(&taken, 4);
+    q = __builtin_amdgcn_readfirstlane(q);
+    if (q >= nl) break;
+    if (q + row >= nl) continue;
+    const size_t g = (size_t)h0 + s_at[q + row];
+    const int cells = s_end[q + row];
+    const int ci = hx[3 * g], cj = hx[3 * g + 1], ck = hx[3 * g + 2], hc = hcount[g];
     double s[3] = {0, 0, 0}, v[3] = {0, 0, 0};
-    if (!lagrangian) {
-      // cells in batches of 8, each cell's three components in one load,
-      // all of a batch's loads in flight before the sums, which keep the
-      // cell order per component
-      using V3 = typename vec3<T>::type;
-      const int end = sh.start[hr2[h]];
-      for (int ob = 0; ob < end; ob += 8) {
-        const int nb = min(8, end - ob);
-        V3 sv[8], vv[8];
+    for (int ob = l16; ob < cells; ob += 64) {
+      V3 sv[4], vv[4];
 #pragma unroll
-        for (int e = 0; e < 8; e++)
-          if (e < nb) {
-            const size_t id = cell_off(ci, cj, ck, sh.offs[ob + e], n0, n1, n2);
-            sv[e] = *reinterpret_cast<const V3*>(S + 3 * id);
-            if (V) vv[e] = *reinterpret_cast<const V3*>(V + 3 * id);
-          }
+      for (int k = 0; k < 4; k++)
+        if (ob + 16 * k < cells) {
+          const size_t id = cell_off(ci, cj, ck, sh.offs[ob + 16 * k], n0, n1, n2);
+          sv[k] = *reinterpret_cast<const V3*>(S + 3 * id);
+          if constexpr (VEL) vv[k] = *reinterpret_cast<const V3*>(V + 3 * id);
+        }
 #pragma unroll
-        for (int e = 0; e < 8; e++)
-          if (e < nb) {
-            s[0] += (double)sv[e].x;
-            s[1] += (double)sv[e].y;
-            s[2] += (double)sv[e].z;
-            if (V) {
-              v[0] += (double)vv[e].x;
-              v[1] += (double)vv[e].y;
-              v[2] += (double)vv[e].z;
-            }
+      for (int k = 0; k < 4; k++)
+        if (ob + 16 * k < cells) {
+          s[0] += (double)sv[k].x;
+          s[1] += (double)sv[k].y;
+          s[2] += (double)sv[k].z;
+          if constexpr (VEL) {
+            v[0] += (double)vv[k].x;
+            v[1] += (double)vv[k].y;
+            v[2] += (double)vv[k].z;
           }
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) {
+        s[a] += __shfl_xor(s[a], o, 16);
+        if constexpr (VEL) v[a] += __shfl_xor(v[a], o, 16);
       }
     }
-    int q[3] = {ci, cj, ck};
-    T L[3] = {L0, L1, L2};
-    for (int a = 0; a < 3; a++) {
-      T base = (T)((double)((T)q[a] * Lc) + (double)Lc / 2.0);
-      T r = base + (T)(s[a] / hcount[h]);
-      if (r >= L[a]) r -= L[a];
-      if (r < (T)0) r += L[a];
-      posh[3 * h + a] = r;
-      if (velh) velh[3 * h + a] = (T)(v[a] / hcount[h]);
-    }
+    if (l16 == 0) posh_store<T, VEL>(s, v, hc, ci, cj, ck, Lc, L0, L1, L2, posh, velh, g);
   }
 }
 
@@ -889,8 +1130,7 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   char* misc = (char*)ctx_buf(c, BUF_MISC, 256);
   const size_t o_cnt = 0;
   long long* dcnt = (long long*)(misc + o_cnt);  // [0..7] scratch counters
-  int* derr = (int*)(misc + o_cnt + 128);
-  long long* hbuf = (long long*)ctx_pinned(c, 256);
+  long long* hbuf = (long long*)ctx_pinned(c, 1024);
 
   // 1. peaks
   long long nblk = (ng + PK_TILE - 1) / PK_TILE;
@@ -943,7 +1183,7 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   long long nc = np > lb ? np - lb : 0;
   c->stat_candidates = nc;
 
-  // candidate state in BUF_CAND: G, cnt, r2 (int), kept (u8), pend x2, hidx
+  // candidate state in BUF_CAND: by rank, by list position, lists' counts
   size_t coff = 0;
   auto ctake = [&](size_t bytes) {
     size_t r = coff;
@@ -951,7 +1191,9 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
     return r;
   };
   size_t ncs = (size_t)std::max(nc, 1LL);
-  long long nblk_c = (nc + PK_TILE - 1) / PK_TILE;
+  // positions per XCD list of pending candidates
+  const long long lcap = ((nc + NXCD - 1) / NXCD + 255) / 256 * 256;
+  const size_t nls = (size_t)std::max(lcap * NXCD, 1LL);
   // first-round order: bricks of 2^bsh x 2^bsh cells (16 x 16, wider on big
   // grids so that the brick histogram fits in LDS)
   int bsh = 4;
@@ -960,21 +1202,20 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   const int nby = (n1 + (1 << bsh) - 1) >> bsh;
   const int nbr = ((n0 + (1 << bsh) - 1) >> bsh) * nby;
   const long long nblk_r = std::max((nc + ORD_RB - 1) / ORD_RB, 1LL);
-  size_t o_c = ctake(ncs * 4), o_r = ctake(ncs * 4), o_k = ctake(ncs),
-         o_p0 = ctake(ncs * 4), o_p1 = ctake(ncs * 4), o_kl = ctake((ncs + 1) * 8),
+  const size_t o_c = ctake(ncs * 4), o_r = ctake(ncs * 4), o_k = ctake(ncs),
+         o_p0 = ctake(nls * 4), o_p1 = ctake(nls * 4), o_kl = ctake((ncs + 1) * 8),
          o_hid = ctake((ncs + 1) * 8), o_cc = ctake(ncs * 4), o_cd = ctake(ncs * sizeof(T)),
-         o_bk = ctake(((size_t)nbr * nblk_r + 1) * 4), o_rf = ctake(ncs * 4),
-         o_pb2 = ctake((size_t)(2 * std::max(nblk_c, 1LL) + 2) * 8), o_pc0 = ctake(ncs * 4),
-         o_pc1 = ctake(ncs * 4), o_pd0 = ctake(ncs * sizeof(T)), o_pd1 = ctake(ncs * sizeof(T)),
-         o_pg = ctake(ncs * 4), o_pn = ctake(ncs * 4), o_pr = ctake(ncs * 4),
-         o_rt = ctake(RT_RING * 8);
+         o_bk = ctake(((size_t)nbr * nblk_r + 1) * 4), o_pc0 = ctake(nls * 4),
+         o_pc1 = ctake(nls * 4), o_pd0 = ctake(nls * sizeof(T)), o_pd1 = ctake(nls * sizeof(T)),
+         o_pg = ctake(nls * 4), o_pn = ctake(nls * 4), o_pr = ctake(nls * 4),
+         o_rt = ctake((RT_RING * NXCD + 1) * 4);
   char* cand = (char*)ctx_buf(c, BUF_CAND, coff);
   int* ccell = (int*)(cand + o_cc);
   T* cden = (T*)(cand + o_cd);
   // eff (delta) and the free flags were written by the peak passes
   S.flag = flag;
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, derr, 1, 0);
-  EXH_LAUNCH_CHECK();
+  int* rt = (int*)(cand + o_rt);
+  int* derr = rt + RT_RING * NXCD;
 
   GrowArgs<T> ga{};
   ga.n0 = n0;
@@ -1003,8 +1244,6 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   int* qcell_next = (int*)(cand + o_pc1);
   T* qden = (T*)(cand + o_pd0);
   T* qden_next = (T*)(cand + o_pd1);
-  int* retry = (int*)(cand + o_rf);
-  long long* pb2 = (long long*)(cand + o_pb2);
   {
     TimedScope ts(c, "halo_candidates");
     hipLaunchKernelGGL(k_cand_setup<T>, dim3(grid_for(nc, 256 * 4)), dim3(256), 0, c->stream,
@@ -1028,9 +1267,7 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   // sized by the last count the host read (counts only shrink), and the
   // host reads the counts and the error flag once per batch.  A round with
   // no pending candidate launches blocks that return at once.
-  long long* rt = (long long*)(cand + o_rt);
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->stream, (unsigned long long*)rt, 1,
-                     (unsigned long long)nc);
+  hipLaunchKernelGGL(k_round_init, dim3(1), dim3(64), 0, c->stream, rt, (int)nc, (int)lcap);
   EXH_LAUNCH_CHECK();
   // Claims carry their round's tag (an epoch counted over the context's
   // calls) above the inverted rank, so the claims of earlier rounds and
@@ -1052,16 +1289,25 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
     c->claim_gen = c->buf_gen[BUF_CLAIM];
     c->claim_mode = cmode;
   }
-  long long ub = nc;
+  // candidates per workgroup: 256, or 64 (16 rows for their long growths)
+  // where 256 would leave most CUs idle
+  long long ub = nc > 0 ? lcap : 0;  // the longest list
   int round = 0, launched = 0;
   {
     TimedScope ts(c, "halo_rounds");
     while (ub > 0) {
       const int batch = launched == 0 ? 1 : RT_BATCH;
       const int first = launched;
+      const int cpb = ub * NXCD > 256 * 512 ? 256 : 64;
+      const dim3 grid((unsigned)((ub + cpb - 1) / cpb) * NXCD);
       for (int q = 0; q < batch; q++) {
-        const long long* dn = rt + launched % RT_RING;
-        long long* dnext = rt + (launched + 1) % RT_RING;
+        RoundLists rl;
+        rl.n = rt + launched % RT_RING * NXCD;
+        rl.next = rt + (launched + 1) % RT_RING * NXCD;
+        rl.clear = rt + (launched + 2) % RT_RING * NXCD;
+        rl.cap = (int)lcap;
+        rl.rank_out = pnext;
+        rl.cell_out = qcell_next;
         launched++;
         if (c32 && c->claim_epoch >= 255) clear_claims();
         const unsigned long long ep = ++c->claim_epoch;
@@ -1069,44 +1315,39 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
         ga.prank = pend;
         ga.pcell = qcell;
         ga.pden = qden;
-        if (c32) {
-          hipLaunchKernelGGL((k_grow<T, true>), dim3(grid_for(ub, 256)), dim3(256), 0, c->stream,
-                             ga, dn, tag_hi);
-          hipLaunchKernelGGL((k_commit<T, true>), dim3(grid_for(ub, 256)), dim3(256), 0,
-                             c->stream, ga, dn, tag_hi, retry, tmax);
-        } else {
-          hipLaunchKernelGGL((k_grow<T, false>), dim3(grid_for(ub, 256)), dim3(256), 0, c->stream,
-                             ga, dn, tag_hi);
-          hipLaunchKernelGGL((k_commit<T, false>), dim3(grid_for(ub, 256)), dim3(256), 0,
-                             c->stream, ga, dn, tag_hi, retry, tmax);
-        }
-        EXH_LAUNCH_CHECK();
-        // candidates to retry, in this round's order
-        const long long nbk = (ub + PK_TILE - 1) / PK_TILE;
-        hipLaunchKernelGGL(k_nonneg_count, dim3((unsigned)nbk), dim3(256), 0, c->stream, retry,
-                           dn, pb2);
-        EXH_LAUNCH_CHECK();
-        exclusive_scan<long long>(c, pb2, pb2 + nbk + 1, nbk);
-        hipLaunchKernelGGL(k_retry_write<T>, dim3((unsigned)nbk), dim3(256), 0, c->stream, retry,
-                           dn, pb2 + nbk + 1, nbk, qcell, qden, pnext, qcell_next, qden_next,
-                           dnext);
+        auto go = [&](auto kg, auto kc) {
+          hipLaunchKernelGGL(kg, grid, dim3(256), 0, c->stream, ga, rl, tag_hi);
+          hipLaunchKernelGGL(kc, grid, dim3(256), 0, c->stream, ga, rl, qden_next, tag_hi, tmax);
+        };
+        if (c32 && cpb == 256)
+          go(k_grow<T, true, 256>, k_commit<T, true, 256>);
+        else if (c32)
+          go(k_grow<T, true, 64>, k_commit<T, true, 64>);
+        else if (cpb == 256)
+          go(k_grow<T, false, 256>, k_commit<T, false, 256>);
+        else
+          go(k_grow<T, false, 64>, k_commit<T, false, 64>);
         EXH_LAUNCH_CHECK();
         std::swap(pend, pnext);
         std::swap(qcell, qcell_next);
         std::swap(qden, qden_next);
       }
-      long long* hr = (long long*)hbuf + 4;  // the ring after the error word
-      EXH_CHECK_HIP(hipMemcpyAsync(hr, rt, RT_RING * 8, hipMemcpyDeviceToHost, c->stream));
-      EXH_CHECK_HIP(hipMemcpyAsync((int*)hbuf + 1, derr, 4, hipMemcpyDeviceToHost, c->stream));
+      int* hr = (int*)hbuf;  // the ring and the error flag
+      EXH_CHECK_HIP(hipMemcpyAsync(hr, rt, (RT_RING * NXCD + 1) * 4, hipMemcpyDeviceToHost,
+                                   c->stream));
       EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
-      int e = ((int*)hbuf)[1];
+      const int e = hr[RT_RING * NXCD];
       EXH_REQUIRE(e == 0, EXH_ERR_RANGE,
                   "halo growth left the supported range (code %d): radius^2 beyond %d, count "
                   "beyond the barrier table, or a sphere wider than half the box",
                   e, stab - 1);
+      auto longest = [&](int r) {
+        const int* h = hr + r % RT_RING * NXCD;
+        return (long long)*std::max_element(h, h + NXCD);
+      };
       for (int r = first; r < launched; r++)
-        if (hr[r % RT_RING] > 0) round++;
-      ub = hr[launched % RT_RING];
+        if (longest(r) > 0) round++;
+      ub = longest(launched);
       EXH_REQUIRE(launched < 1000000, EXH_ERR_INTERNAL, "halo rounds did not converge");
     }
   }
@@ -1185,9 +1426,10 @@ void run_halo_posh(exh_ctx* c, const exh_box* b, const T* S, const T* V, int lag
   HaloState& st = c->halo;
   if (c->nh <= 0) return;
   TimedScope ts(c, "halo_posh");
-  hipLaunchKernelGGL(k_halo_posh<T>, dim3(grid_for(c->nh, 256)), dim3(256), 0, c->stream, st.hx,
-                     st.hcount, st.hr2, c->nh, st.sh, b->nd[0], b->nd[1], b->nd[2], S, V,
-                     (T)b->Lc, (T)b->L[0], (T)b->L[1], (T)b->L[2], lagrangian, (T*)st.posh,
+  auto kern = V ? k_halo_posh<T, true> : k_halo_posh<T, false>;
+  hipLaunchKernelGGL(kern, dim3(grid_for(c->nh, 256)), dim3(256), 0, c->stream, st.hx, st.hcount,
+                     st.hr2, c->nh, st.sh, b->nd[0], b->nd[1], b->nd[2], S, V, (T)b->Lc,
+                     (T)b->L[0], (T)b->L[1], (T)b->L[2], lagrangian, (T*)st.posh,
                      V ? (T*)st.velh : nullptr);
   EXH_LAUNCH_CHECK();
 }

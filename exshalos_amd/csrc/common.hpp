@@ -60,7 +60,7 @@ enum Slot {
   BUF_V,        // velocity field [ng][3]
   BUF_FLAG,     // int32 halo flags
   BUF_CLAIM,    // uint64 per-cell claims used by the halo rounds
-  BUF_PEAK_IDX, // lexicographic peak indices (sort values)
+  BUF_PEAK_IDX, // peak index of every sorted position
   BUF_PEAK_CELL,// peak cell indices in lexicographic order
   BUF_PEAK_KEY, // peak densities
   BUF_SORT_K,   // sort ping-pong keys
@@ -115,11 +115,15 @@ struct Timing {
 };
 
 // Lattice offsets grouped by r^2: shell s occupies offs[start[s] ..
-// start[s+1]) in the reference's cube order.
+// start[s+1]) in the reference's cube order.  For 1 <= G <= ball_max the
+// start[G] offsets of r^2 < G stand in memory order (along k, then j, then i)
+// at balls[ball[G]].
 struct ShellTab {
   const int* start = nullptr;
   const unsigned* offs = nullptr;
-  int stab = 0;
+  const int* ball = nullptr;
+  const unsigned* balls = nullptr;
+  int stab = 0, ball_max = 0;
 };
 
 // Device arrays of the last halo run (views into context buffers).
@@ -130,7 +134,7 @@ struct HaloState {
   void* Mh = nullptr;
   void* posh = nullptr;
   void* velh = nullptr;
-  long long* hidx = nullptr;
+  int* hidx = nullptr;
   int* flag = nullptr;
   ShellTab sh;
   int sh_tmax = -1;

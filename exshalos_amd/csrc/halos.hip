@@ -10,9 +10,10 @@
 //    (thread per candidate, the reference's exact double-precision sum
 //    order) and claims the cells it could write (r^2 < G, G = first failing
 //    shell; more flags can only stop the growth earlier, so the final halo
-//    lies inside that ball).  A candidate whose read ball (r^2 <= G) holds
-//    no claim of a denser pending candidate has seen its final flags: it
-//    commits.  The densest pending candidate always commits, so the rounds
+//    lies inside that ball).  A candidate of one cell (G = 1) claims nothing:
+//    its centre's flag names its rank.  A candidate whose read ball
+//    (r^2 <= G) holds no claim and no centre of a denser pending candidate
+//    has seen its final flags: it commits.  The densest pending candidate always commits, so the rounds
 //    terminate; the result equals the sequential loop.
 // 4. masses: taus uniforms by GF(2) jump-ahead, Tinker-integral splines
 //    (find_halos.c:442-476);
@@ -25,17 +26,28 @@
 
 namespace exh {
 
+// Flags of the cells during the rounds: free, inside a rejected sphere, the
+// free centre of the pending candidate of rank r (FLAG_PENDING - r), or >= 0
+// in a halo.
 static constexpr int FLAG_FREE = -1;
 static constexpr int FLAG_REJECTED = -2;
+static constexpr int FLAG_PENDING = -3;
 static constexpr int S_TAB_MAX = 1024;  // largest r^2 a halo may reach
+static constexpr int BALL_MAX = 65;     // largest ball whose cells are tabled in memory order
+
+// x in [-n, 2n) wrapped into [0, n): of x, x + n and x - n the one that is
+// in range is the smallest as unsigned.
+__device__ __forceinline__ unsigned wrap_u(int x, int n) {
+  return min(min((unsigned)x, (unsigned)(x + n)), (unsigned)(x - n));
+}
 
 // Cell at packed offset p from (ci, cj, ck), periodic; cells are below 2^30.
-__device__ inline unsigned cell_off(int ci, int cj, int ck, unsigned p, int n0, int n1, int n2) {
-  int di = (int)(p & 255u) - 128, dj = (int)((p >> 8) & 255u) - 128,
-      dk = (int)((p >> 16) & 255u) - 128;
-  return ((unsigned)wrap1(ci, di, n0) * (unsigned)n1 + (unsigned)wrap1(cj, dj, n1)) *
-             (unsigned)n2 +
-         (unsigned)wrap1(ck, dk, n2);
+__device__ __forceinline__ unsigned cell_off(int ci, int cj, int ck, unsigned p, int n0, int n1,
+                                             int n2) {
+  const int di = (int)(p & 255u) - 128, dj = (int)((p >> 8) & 255u) - 128,
+            dk = (int)((p >> 16) & 255u) - 128;
+  return (wrap_u(ci + di, n0) * (unsigned)n1 + wrap_u(cj + dj, n1)) * (unsigned)n2 +
+         wrap_u(ck + dk, n2);
 }
 
 // ---------------------------------------------------------------------------
@@ -116,9 +128,11 @@ __device__ inline unsigned peak_bits(const T* d, unsigned c0, unsigned ng, const
 // neighbours again.
 template <typename T>
 __global__ __launch_bounds__(256) void k_peak_count(const T* d, PeakGeom g, long long* bcnt,
-                                                    T* eff, unsigned char* pbits) {
+                                                    T* eff, unsigned char* pbits,
+                                                    unsigned long long* below) {
   static_assert(PK_ITEMS == 8, "one byte of peak flags per thread");
   __shared__ int sh[4];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *below = 0;
   const unsigned ng = (unsigned)g.n0 * g.sx;
   const unsigned base = blockIdx.x * (unsigned)PK_TILE + threadIdx.x;
   const unsigned bits = peak_bits(d, base, ng, g, eff);
@@ -130,11 +144,15 @@ __global__ __launch_bounds__(256) void k_peak_count(const T* d, PeakGeom g, long
   if (threadIdx.x == 0) bcnt[blockIdx.x] = (long long)sh[0] + sh[1] + sh[2] + sh[3];
 }
 
+// It also counts the peaks below the smallest barrier, which are never
+// visited: their number is the first visited sorted position.
 template <typename T>
 __global__ __launch_bounds__(256) void k_peak_write(const T* d, PeakGeom g, const long long* boff,
-                                                    const unsigned char* pbits, T* key, int* cell,
-                                                    int* flag) {
+                                                    const unsigned char* pbits, T Bmin, T* key,
+                                                    int* cell, int* flag,
+                                                    unsigned long long* n_below) {
   __shared__ int wcnt[PK_ITEMS][4];
+  __shared__ int wlow[4];
   const unsigned ng = (unsigned)g.n0 * g.sx;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const unsigned base = blockIdx.x * (unsigned)PK_TILE + threadIdx.x;
@@ -156,7 +174,16 @@ __global__ __launch_bounds__(256) void k_peak_write(const T* d, PeakGeom g, cons
     bal[q] = __ballot((bits >> q) & 1u);
     if (lane == 0) wcnt[q][w] = __popcll(bal[q]);
   }
+  int low = 0;
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++)
+    low += __popcll(__ballot(((bits >> q) & 1u) && dv[q] < Bmin));
+  if (lane == 0) wlow[w] = low;
   __syncthreads();
+  if (threadIdx.x == 0) {
+    low = wlow[0] + wlow[1] + wlow[2] + wlow[3];
+    if (low) atomicAdd(n_below, (unsigned long long)low);
+  }
   long long o = boff[blockIdx.x];
   const unsigned long long below = lanemask_lt();
   for (int q = 0; q < PK_ITEMS; q++) {
@@ -172,102 +199,81 @@ __global__ __launch_bounds__(256) void k_peak_write(const T* d, PeakGeom g, cons
   }
 }
 
-// Candidates by rank (0 = densest): rank r <-> sorted position np-1-r,
-// kept for sorted positions >= lb (density >= the minimum barrier, and
-// never position 0, which the reference does not visit).  The sort carried
-// each peak's cell along with its density.
-template <typename T>
-__global__ void k_cand_setup(const T* skey, const int* scell, long long np, long long lb,
-                             int* ccell, T* cden) {
-  for (long long l = lb + blockIdx.x * (long long)blockDim.x + threadIdx.x; l < np;
-       l += (long long)gridDim.x * blockDim.x) {
-    const long long r = np - 1 - l;
-    ccell[r] = scell[l];
-    cden[r] = skey[l];
-  }
-}
-
-// Order of the first round: columns of BR x BR cells in (i, j) over all k
-// ("bricks"), one after the other, and within a brick by blocks of ORD_RB
-// consecutive ranks (similar densities, hence similar growth work per
-// wave).  A counting sort: per rank block, a histogram over bricks; one
-// exclusive scan over (brick, block); then each block scatters its ranks.
-static constexpr int ORD_RB = 4096;
+// Candidates: the peaks with density >= the smallest barrier, except the one
+// at sorted position 0, which the reference does not visit.  Rank r (0 =
+// densest) is sorted position np - 1 - r; perm gives each position's peak.
+// Writes each candidate's rank by peak.
 static constexpr int RT_RING = 16;   // device ring of per-round pending counts
 static constexpr int RT_BATCH = 4;   // rounds per host read after the first
 static constexpr int NXCD = 8;       // accelerator dies: lists of pending candidates
-static constexpr int ORD_MAXB = 8192;  // bricks (LDS ints)
 
-__device__ inline int brick_of(int cell, int n1, int n2, int bsh, int nby) {
-  const int r = cell / n2;
-  const int j = r % n1, i = r / n1;
-  return (i >> bsh) * nby + (j >> bsh);
-}
-
-__global__ void k_brick_hist(const int* ccell, long long nc, int n1, int n2, int bsh, int nby,
-                             int nbr, int nblk, int* counts) {
-  __shared__ int hist[ORD_MAXB];
-  for (int b = threadIdx.x; b < nbr; b += blockDim.x) hist[b] = 0;
-  __syncthreads();
-  const long long r0 = (long long)blockIdx.x * ORD_RB;
-  const long long r1 = r0 + ORD_RB < nc ? r0 + ORD_RB : nc;
-  for (long long r = r0 + threadIdx.x; r < r1; r += blockDim.x)
-    atomicAdd(&hist[brick_of(ccell[r], n1, n2, bsh, nby)], 1);
-  __syncthreads();
-  for (int b = threadIdx.x; b < nbr; b += blockDim.x)
-    counts[(long long)b * nblk + blockIdx.x] = hist[b];
-}
-
-template <typename T>
-__global__ void k_brick_scatter(const int* ccell, const T* cden, long long nc, int n1, int n2,
-                                int bsh, int nby, int nbr, int nblk, const int* offs, int* prank,
-                                int* pcell, T* pden) {
-  __shared__ int cur[ORD_MAXB];
-  for (int b = threadIdx.x; b < nbr; b += blockDim.x)
-    cur[b] = offs[(long long)b * nblk + blockIdx.x];
-  __syncthreads();
-  const long long r0 = (long long)blockIdx.x * ORD_RB;
-  const long long r1 = r0 + ORD_RB < nc ? r0 + ORD_RB : nc;
-  // the block's cells and densities first, all loads in flight together
-  // (the stores below could alias them for the compiler); then the ranks
-  // in the same order as a strided loop would take them
-  constexpr int PER = ORD_RB / 256;
-  int cells[PER];
-  T dens[PER];
+__global__ __launch_bounds__(256) void k_cand_ranks(const int* perm, int np, int below, int* rank,
+                                                    int* rt) {
+  if (blockIdx.x == 0 && threadIdx.x <= 2 * NXCD)  // the first two rounds' counts, the error flag
+    rt[threadIdx.x < 2 * NXCD ? threadIdx.x : RT_RING * NXCD] = 0;
+  const int l0 = below + (int)blockIdx.x * 1024 + (int)threadIdx.x;
+  int p[4];
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const long long r = r0 + threadIdx.x + 256 * q;
-    if (r < r1) {
-      cells[q] = ccell[r];
-      dens[q] = cden[r];
-    }
+  for (int q = 0; q < 4; q++) p[q] = l0 + 256 * q < np ? perm[l0 + 256 * q] : -1;
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    if (p[q] >= 0) rank[p[q]] = np - 1 - (l0 + 256 * q);
+}
+
+// The first round's lists: the candidates in the order of their cells, list
+// x the x-th eighth of the blocks of PK_TILE peaks.  Neighbours in the list
+// are neighbours in memory, and dense candidates (long growths) are spread
+// over the workgroups.  (Lists by bricks of 16 x 16 columns and density gave
+// a wave growths of similar length, but workgroups of long ones only: the
+// first round of a 256^3 grid of 2 Mpc/h cells took 2.3 ms with them.)
+// Clears the results by peak and flags the candidates' centres as pending.
+template <typename T>
+__global__ __launch_bounds__(256) void k_list_build(const T* key, const int* cell,
+                                                    const int* rank, int np, int nc, T Bmin,
+                                                    int cap, int* rt, int* prank, int* ppeak,
+                                                    unsigned short* res, int* flag) {
+  __shared__ int wcnt[PK_ITEMS][4];
+  __shared__ int s_base;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int p0 = (int)blockIdx.x * PK_TILE + (int)threadIdx.x;
+  int r[PK_ITEMS], c[PK_ITEMS];
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++) {
+    const int p = p0 + 256 * q;
+    c[q] = p < np ? cell[p] : 0;
+    r[q] = p < np && key[p] >= Bmin ? rank[p] : nc;
   }
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const long long r = r0 + threadIdx.x + 256 * q;
-    if (r < r1) {
-      const int pos = atomicAdd(&cur[brick_of(cells[q], n1, n2, bsh, nby)], 1);
-      prank[pos] = (int)r;
-      pcell[pos] = cells[q];
-      pden[pos] = dens[q];
-    }
+  for (int q = 0; q < PK_ITEMS; q++) {
+    if (p0 + 256 * q < np) res[p0 + 256 * q] = 0;
+    if (r[q] < nc) flag[c[q]] = FLAG_PENDING - r[q];
   }
-}
-
-// number of keys below Bmin (the first candidate's sorted position); *out
-// starts at zero
-template <typename T>
-__global__ void k_count_below(const T* key, long long n, T Bmin, unsigned long long* out) {
-  __shared__ unsigned sh[4];
-  unsigned cnt = 0;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x)
-    cnt += key[i] < Bmin;
-  for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = cnt;
+  unsigned long long bal[PK_ITEMS];
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++) {
+    bal[q] = __ballot(r[q] < nc);
+    if (lane == 0) wcnt[q][w] = __popcll(bal[q]);
+  }
   __syncthreads();
-  if (threadIdx.x == 0)
-    atomicAdd(out, (unsigned long long)(sh[0] + sh[1] + sh[2] + sh[3]));
+  const int x = (int)((long long)blockIdx.x * NXCD / gridDim.x);
+  if (threadIdx.x == 0) {
+    int tot = 0;
+    for (int q = 0; q < PK_ITEMS; q++) tot += wcnt[q][0] + wcnt[q][1] + wcnt[q][2] + wcnt[q][3];
+    s_base = atomicAdd(&rt[x], tot);
+  }
+  __syncthreads();
+  int o = x * cap + s_base;
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++) {
+    int ow = o;
+    for (int u = 0; u < w; u++) ow += wcnt[q][u];
+    if (r[q] < nc) {
+      const int at = ow + __popcll(bal[q] & lanemask_lt());
+      prank[at] = r[q];
+      ppeak[at] = p0 + 256 * q;
+    }
+    o += wcnt[q][0] + wcnt[q][1] + wcnt[q][2] + wcnt[q][3];
+  }
 }
 
 __global__ void k_fill_u64(unsigned long long* p, long long n, unsigned long long v) {
@@ -279,6 +285,8 @@ __global__ void k_fill_u64(unsigned long long* p, long long n, unsigned long lon
 // ---------------------------------------------------------------------------
 // growth rounds
 // ---------------------------------------------------------------------------
+static constexpr int PRES_BLOCKED = 1 << 30;
+
 template <typename T>
 struct GrowArgs {
   int n0, n1, n2;
@@ -292,18 +300,18 @@ struct GrowArgs {
   T Bmin;
   T negMtot;
   int Nmin;
-  // the round's candidates by list position: rank (0 = densest), centre
-  // cell and density, and the growth results handed from k_grow to k_commit
-  const int* prank;
+  // cell and density by peak
   const int* pcell;
-  const T* pden;
-  int* pG;         // first failing shell (read radius^2); -1 = skipped
-  int* pcnt;       // count
-  int* pr2;        // grows_tmp
-  // final results by rank
-  int* cnt;
-  int* r2;
-  unsigned char* kept;
+  const T* pkey;
+  // the round's candidates by list position: rank (0 = densest), peak, and
+  // the growth result handed from k_grow to k_commit: (G << 16 | R2), G the
+  // first failing shell (read radius^2) and R2 the final halo's shells (its
+  // cells are those of r^2 < R2, start[R2] of them), PRES_BLOCKED where the
+  // centre of a denser pending candidate lies in the read ball; -1 = skipped
+  const int* prank;
+  const int* ppeak;
+  int* pres;
+  unsigned short* res;  // final result by peak: R2, or 0 (no halo)
   int* err;
 };
 
@@ -327,7 +335,7 @@ struct RoundLists {
   int* next;      // [NXCD] the next round's (zero on entry; k_commit adds)
   int* clear;     // [NXCD] the round's after that, zeroed by k_grow
   int cap;
-  int *rank_out, *cell_out;  // the next round's lists (densities in pden_out)
+  int *rank_out, *peak_out;  // the next round's lists
 };
 
 // A table that no kernel of the rounds writes, read through the scalar cache
@@ -373,24 +381,58 @@ __device__ __forceinline__ void row_sub(double& s, T v) {
   }
 }
 
-// The row's values of f at cells [o, min(o + 64, o1)) of the shell table,
-// 16 cells in each v[k], in lane order and zeros past o1.  The offsets of the first SH_LDS
-// cells are read from LDS: a load of theirs from memory would wait behind
-// the loads of values in flight.
-static constexpr int ROW_K = 4;
-static constexpr int SH_LDS = 1024;
+// A row's centre and where its ball may wrap: with FLAT, cells within
+// sqrt(flat) of the centre need no wrap in i and j.
+struct Centre {
+  int i, j, k, ij;  // ij: the cell (i, j, 0)
+  int flat;
+};
+
 template <typename T>
-__device__ __forceinline__ void row_load(T (&v)[ROW_K], const T* f, const unsigned* lds_offs,
-                                         const unsigned* offs, int o, int o1, int lane, int ci,
-                                         int cj, int ck, int n0, int n1, int n2) {
+__device__ __forceinline__ Centre centre_of(const GrowArgs<T>& a, int i, int j, int k) {
+  Centre c;
+  c.i = i;
+  c.j = j;
+  c.k = k;
+  c.ij = (i * a.n1 + j) * a.n2;
+  const int d = min(min(i, a.n0 - 1 - i), min(j, a.n1 - 1 - j));
+  c.flat = d * d;
+  return c;
+}
+
+// The offsets of the first SH_LDS cells of the shell table, in LDS (a load
+// of theirs from memory would wait behind the loads of values in flight):
+// x = di n1 n2 + dj n2, y = the packed offset.
+static constexpr unsigned CENTRE_OFF = 0x808080u;  // packed offset (0, 0, 0)
+static constexpr int SH_LDS = 1024;
+static constexpr int ST_LDS = 256;  // shells whose starts are in LDS
+
+__device__ __forceinline__ unsigned table_cell(const int2& t, bool flat, const Centre& c, int n0,
+                                               int n1, int n2) {
+  if (flat)
+    return (unsigned)(c.ij + t.x) + wrap_u(c.k + (int)(((unsigned)t.y >> 16) & 255u) - 128, n2);
+  return cell_off(c.i, c.j, c.k, (unsigned)t.y, n0, n1, n2);
+}
+
+// The row's values of f at cells [o, min(o + 64, o1)) of the shell table,
+// 16 cells in each v[k], in lane order and zeros past o1.
+static constexpr int ROW_K = 4;
+template <typename T>
+__device__ __forceinline__ void row_load(T (&v)[ROW_K], const T* f, const int2* tab,
+                                         const GrowArgs<T>& a, int o, int o1, int lane, bool flat,
+                                         const Centre& c) {
 #pragma unroll
   for (int k = 0; k < ROW_K; k++) {
     if (o + 16 * k >= o1) break;
     const int e = o + 16 * k + lane;
     v[k] = 0;
     if (e < o1) {
-      const unsigned p = o1 <= SH_LDS ? lds_offs[e] : offs[e];
-      v[k] = f[cell_off(ci, cj, ck, p, n0, n1, n2)];
+      unsigned id;
+      if (o1 <= SH_LDS)
+        id = table_cell(tab[e], flat, c, a.n0, a.n1, a.n2);
+      else
+        id = cell_off(c.i, c.j, c.k, a.sh.offs[e], a.n0, a.n1, a.n2);
+      v[k] = f[id];
     }
   }
 }
@@ -427,86 +469,128 @@ __device__ __forceinline__ bool claimed(const unsigned long long* claim, unsigne
 //
 // One thread per candidate tests the flag and the first shell (6 cells).
 // Most candidates end there (81% of a 512^3 box's halos of 4 Mpc/h cells are
-// one cell), and they claim that cell.  The others go to a list in LDS, from
-// which each wave takes four at a time, one per row of 16 lanes: the row
-// loads a shell's cells in parallel, two shells ahead of the sum, and every
-// lane forms the reference's ordered double sum from the row's values
-// (row_newbcast moves).  A growth of n cells then waits for about one load
-// per shell and not for one per 8 cells, and a wave is held by the longest
-// of four growths and not of 64.
+// one cell); they claim nothing.  With 256 candidates a workgroup the
+// threads go on to the next shells while at least GROW_MIN of them grow: a
+// shell of n cells costs a wave about 20 n vector instructions for all of its
+// candidates, and a row (below) about 4 n for one.
+//
+// The others go to a list in LDS, from which each wave takes four at a time,
+// one per row of 16 lanes: the row loads a shell's cells in parallel, two
+// shells ahead of the sum, and every lane forms the reference's ordered
+// double sum from the row's values (row_newbcast moves).  A growth of n cells
+// then waits for about one load per shell and not for one per 8 cells, and a
+// wave is held by the longest of four growths and not of 64.  What bounds
+// the kernel is vector issue in large boxes and that chain of loads and
+// ordered additions in small ones.
+static constexpr int GROW_MIN = 56;
+static constexpr int GROW_SHELLS = 9;  // last shell of the threads
+
 template <typename T, bool C32, int CPB>
 __global__ __launch_bounds__(256) void k_grow(GrowArgs<T> a, RoundLists rl,
                                               unsigned long long tag_hi) {
   __shared__ double s_mean[CPB];
-  __shared__ int s_cell[CPB], s_rank[CPB];
-  __shared__ short s_at[CPB];
-  __shared__ unsigned s_offs[SH_LDS];
+  __shared__ int s_i[CPB], s_j[CPB], s_k[CPB], s_rank[CPB];
+  __shared__ short s_at[CPB], s_G[CPB];
+  __shared__ int2 s_tab[SH_LDS];
+  __shared__ int s_start[ST_LDS];
   __shared__ int nlist, taken;
   const int x = blockIdx.x % NXCD, t0 = (int)(blockIdx.x / NXCD) * CPB;
   if (blockIdx.x < NXCD && threadIdx.x == 0) rl.clear[blockIdx.x] = 0;
   const int n = rl.n[x];
   if (t0 >= n) return;
   const int base = x * rl.cap + t0, m = min(CPB, n - t0);
+  const int* start = a.sh.start;
   if (threadIdx.x == 0) {
     nlist = 0;
     taken = 0;
   }
-  const int noffs = table_at(a.sh.start, a.sh.stab);
+  const int noffs = table_at(start, a.sh.stab);
 #pragma unroll
   for (int q = 0; q < SH_LDS / 256; q++) {
     const int e = (int)threadIdx.x + 256 * q;
-    s_offs[e] = e < noffs ? a.sh.offs[e] : 0u;
+    const unsigned p = e < noffs ? a.sh.offs[e] : 0u;
+    const int di = (int)(p & 255u) - 128, dj = (int)((p >> 8) & 255u) - 128;
+    s_tab[e] = make_int2((di * a.n1 + dj) * a.n2, (int)p);
   }
+  s_start[threadIdx.x] = start[min((int)threadIdx.x, a.sh.stab)];
   __syncthreads();
   const double Bmin = (double)a.Bmin;
   const int lane = threadIdx.x & 63;
+  int s = 1;
   if (threadIdx.x < CPB) {
     const int t = base + threadIdx.x;
-    bool more = false;
-    double mean = 0;
-    int rank = 0, cell = 0;
+    bool mine = false, more;
+    double den = 0, mean = 0;
+    int rank = 0, cell = 0, G = 0;
+    Centre c = {0, 0, 0, 0, 0};
     if ((int)threadIdx.x < m) {
       rank = a.prank[t];
-      cell = a.pcell[t];
-      if (a.flag[cell] != FLAG_FREE) {  // already inside a denser halo
-        a.pG[t] = -1;
-        a.kept[rank] = 0;
-      } else {
-        int ci, cj, ck;
-        decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
-        T v[6];
+      const int p = a.ppeak[t];
+      cell = a.pcell[p];
+      mean = (double)a.pkey[p];
+      mine = a.flag[cell] <= FLAG_PENDING;
+      if (!mine) a.pres[t] = -1;  // already inside a denser halo
+      int i, j, k;
+      decode_cell<T>(cell, a.n1, a.n2, i, j, k);
+      c = centre_of(a, i, j, k);
+    }
+    more = mine;
+    const bool flat = __ballot(mine && c.flat < GROW_SHELLS) == 0;
+    // cell e of the table around the thread's candidate
+    auto at = [&](int e) {
+      const unsigned p = (unsigned)table_at((const int*)a.sh.offs, e);
+      if (!flat) return cell_off(c.i, c.j, c.k, p, a.n0, a.n1, a.n2);
+      const int di = (int)(p & 255u) - 128, dj = (int)((p >> 8) & 255u) - 128;
+      return (unsigned)(c.ij + (di * a.n1 + dj) * a.n2) +
+             wrap_u(c.k + (int)((p >> 16) & 255u) - 128, a.n2);
+    };
+    for (;;) {
+      const int o0 = table_at(start, s), o1 = table_at(start, s + 1);
+      if (more) {
+        // the shell's cells in cube order; loads issued in batches, summed
+        // in order (flagged cells hold -Mtot in eff, as the reference adds)
+        double sum = mean * (double)o0;
+        for (int ob = o0; ob < o1; ob += 6) {
+          T v[6];
 #pragma unroll
-        for (int e = 0; e < 6; e++)
-          v[e] = a.eff[cell_off(ci, cj, ck, (unsigned)table_at((const int*)a.sh.offs, 1 + e),
-                                a.n0, a.n1, a.n2)];
-        double den = (double)a.pden[t];
-        mean = den * 1.0;
+          for (int e = 0; e < 6; e++)
+            if (ob + e < o1) v[e] = a.eff[at(ob + e)];
 #pragma unroll
-        for (int e = 0; e < 6; e++) mean += (double)v[e];
-        mean = mean / 7.0;
-        more = mean >= Bmin;
-        if (!more) {
-          // one cell; below the barrier of one cell it shrinks to none
-          const bool one = !(den < (double)a.Bt[1]);
-          a.pG[t] = 1;
-          a.pcnt[t] = one ? 1 : 0;
-          a.pr2[t] = one ? 1 : 0;
-          claim_cell<C32>(a.claim, (unsigned)cell, tag_hi, rank);
+          for (int e = 0; e < 6; e++)
+            if (ob + e < o1) sum += (double)v[e];
+        }
+        sum = sum / (double)o1;
+        den = mean;
+        mean = sum;
+        if (!(mean >= Bmin)) {
+          more = false;
+          G = s;
         }
       }
+      s++;
+      if (CPB < 256 || s > GROW_SHELLS) break;
+      if (__builtin_amdgcn_readfirstlane(__syncthreads_count(more)) < GROW_MIN) break;
     }
-    const unsigned long long bal = __ballot(more);
-    int at = 0;
-    if (bal && lane == 0) at = atomicAdd(&nlist, __popcll(bal));
-    at = __shfl(at, 0, 64) + __popcll(bal & lanemask_lt());
-    if (more) {
-      s_mean[at] = mean;
-      s_cell[at] = cell;
-      s_rank[at] = rank;
-      s_at[at] = (short)threadIdx.x;
+    // grown out at one cell, which shrinks to none below its barrier; the
+    // others are left to a row
+    const bool row = more || G > 1;
+    if (G == 1) a.pres[t] = 1 << 16 | (den < (double)a.Bt[1] ? 0 : 1);
+    const unsigned long long bal = __ballot(row);
+    int o = 0;
+    if (bal && lane == 0) o = atomicAdd(&nlist, __popcll(bal));
+    o = __shfl(o, 0, 64) + __popcll(bal & lanemask_lt());
+    if (row) {
+      s_mean[o] = more ? mean : den;
+      s_G[o] = (short)G;
+      s_i[o] = c.i;
+      s_j[o] = c.j;
+      s_k[o] = c.k;
+      s_rank[o] = rank;
+      s_at[o] = (short)threadIdx.x;
     }
   }
   __syncthreads();
+  s = CPB < 256 ? 2 : __builtin_amdgcn_readfirstlane(s);  // the first shell of the rows
   const int nl = nlist, l16 = lane & 15, row = lane >> 4;
   for (;;) {
     int q = 0;
@@ -515,110 +599,155 @@ __global__ __launch_bounds__(256) void k_grow(GrowArgs<T> a, RoundLists rl,
     if (q >= nl) break;
     const bool has = q + row < nl;
     const int it = has ? q + row : q;  // an idle row follows the first one
-    const int cell = s_cell[it], rank = s_rank[it];
-    int ci, cj, ck;
-    decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
-    // growth from shell 2 on; count = start[s] cells lie inside shell s
-    double den = 0, mean = s_mean[it];
-    bool act = has;
-    int G = -1;
-    const int* start = a.sh.start;
+    const int rank = s_rank[it];
+    const Centre c = centre_of(a, s_i[it], s_j[it], s_k[it]);
+    // the rows that are to grow, from shell s on; count = start[sh] cells lie
+    // inside shell sh
+    int G = s_G[it];
+    double den = s_mean[it], mean = den;
+    bool act = has && G == 0;
+    if (G == 0) G = -1;
     T va[ROW_K], vb[ROW_K], vc[ROW_K];
-    int o0 = table_at(start, 2), o1 = table_at(start, 3), o2 = table_at(start, 4),
-        o3 = table_at(start, 5);
-    row_load(va, a.eff, s_offs, a.sh.offs, o0, o1, l16, ci, cj, ck, a.n0, a.n1, a.n2);
-    row_load(vb, a.eff, s_offs, a.sh.offs, o1, o2, l16, ci, cj, ck, a.n0, a.n1, a.n2);
-    for (int s = 2;; s++) {
-      if (s >= a.sh.stab) {  // rows still growing leave the table
-        if (act) atomicOr(a.err, 1);
-        break;
-      }
-      const int o4 = s + 3 < a.sh.stab ? table_at(start, s + 4) : o3;
-      row_load(vc, a.eff, s_offs, a.sh.offs, o2, o3, l16, ci, cj, ck, a.n0, a.n1, a.n2);
-      double sum = mean * (double)o0;
-#pragma unroll
-      for (int k = 0; k < ROW_K; k++)
-        if (o0 + 16 * k < o1) row_add<0>(sum, va[k], o1 - o0 - 16 * k);
-      for (int o = o0 + 16 * ROW_K; o < o1; o += 16 * ROW_K) {
-        row_load(va, a.eff, s_offs, a.sh.offs, o, o1, l16, ci, cj, ck, a.n0, a.n1, a.n2);
+    if (__ballot(act)) {
+      int fl = min(c.flat, __shfl_xor(c.flat, 16, 64));
+      fl = __builtin_amdgcn_readfirstlane(min(fl, __shfl_xor(fl, 32, 64)));
+      int o0 = table_at(start, s), o1 = table_at(start, s + 1), o2 = table_at(start, s + 2),
+          o3 = table_at(start, s + 3);
+      row_load(va, a.eff, s_tab, a, o0, o1, l16, s <= fl, c);
+      row_load(vb, a.eff, s_tab, a, o1, o2, l16, s + 1 <= fl, c);
+      for (int sh = s;; sh++) {
+        if (sh >= a.sh.stab) {  // rows still growing leave the table
+          if (act) atomicOr(a.err, 1);
+          break;
+        }
+        const int o4 = sh + 3 < a.sh.stab ? table_at(start, sh + 4) : o3;
+        row_load(vc, a.eff, s_tab, a, o2, o3, l16, sh + 2 <= fl, c);
+        double sum = mean * (double)o0;
 #pragma unroll
         for (int k = 0; k < ROW_K; k++)
-          if (o + 16 * k < o1) row_add<0>(sum, va[k], o1 - o - 16 * k);
-      }
-      sum = sum / (double)o1;
-      if (act) {
-        den = mean;
-        mean = sum;
-        if (!(mean >= Bmin)) {
-          act = false;
-          G = s;
-        }
-      }
-      if (!__ballot(act)) break;
-#pragma unroll
-      for (int k = 0; k < ROW_K; k++) {
-        va[k] = vb[k];
-        vb[k] = vc[k];
-      }
-      o0 = o1;
-      o1 = o2;
-      o2 = o3;
-      o3 = o4;
-    }
-    const int t = base + s_at[it];
-    if (G >= 0) {  // a row with a result: shrink it below the barrier
-      int grows = G - 1, grows_tmp = G, count = start[G];
-      while (start[grows + 1] == start[grows]) grows--;  // the last shell with cells
-      for (;;) {
-        if (count >= a.nB) {
-          if (l16 == 0) atomicOr(a.err, 2);
-          G = -1;
-          break;
-        }
-        if (!(den < (double)a.Bt[count] && count > 0)) break;
-        if (grows < 0) {  // cannot happen while count > 0 on an unclamped table
-          if (l16 == 0) atomicOr(a.err, 32);
-          G = -1;
-          break;
-        }
-        const int c1 = start[grows + 1], c0 = start[grows];
-        den = den * (double)count;
-        for (int o = c0; o < c1; o += 16 * ROW_K) {
-          row_load(va, a.delta, s_offs, a.sh.offs, o, c1, l16, ci, cj, ck, a.n0, a.n1, a.n2);
+          if (o0 + 16 * k < o1) row_add<0>(sum, va[k], o1 - o0 - 16 * k);
+        for (int o = o0 + 16 * ROW_K; o < o1; o += 16 * ROW_K) {
+          row_load(va, a.eff, s_tab, a, o, o1, l16, sh <= fl, c);
 #pragma unroll
           for (int k = 0; k < ROW_K; k++)
-            if (o + 16 * k < c1) row_sub<0>(den, va[k]);
+            if (o + 16 * k < o1) row_add<0>(sum, va[k], o1 - o - 16 * k);
         }
-        count -= c1 - c0;
-        if (count > 0) den = den / (double)count;
-        if (c1 > c0) grows_tmp = grows;
-        grows--;
-      }
-      if (G >= 0) {
-        if (l16 == 0) {
-          a.pcnt[t] = count;
-          a.pr2[t] = grows_tmp;
+        sum = sum / (double)o1;
+        if (act) {
+          den = mean;
+          mean = sum;
+          if (!(mean >= Bmin)) {
+            act = false;
+            G = sh;
+          }
         }
-        // claim every cell the final halo could occupy (r^2 < G)
-        const int oend = start[G];
-        for (int o = l16; o < oend; o += 16)
-          claim_cell<C32>(a.claim, cell_off(ci, cj, ck, a.sh.offs[o], a.n0, a.n1, a.n2), tag_hi,
-                          rank);
+        if (!__ballot(act)) break;
+#pragma unroll
+        for (int k = 0; k < ROW_K; k++) {
+          va[k] = vb[k];
+          vb[k] = vc[k];
+        }
+        o0 = o1;
+        o1 = o2;
+        o2 = o3;
+        o3 = o4;
       }
     }
-    if (has && l16 == 0) a.pG[t] = G;
+    const int t = base + s_at[it];
+    if (has && G >= 0) {  // a row with a result: shrink it below the barrier
+      auto start_of = [&](int sh) { return sh < ST_LDS ? s_start[sh] : start[sh]; };
+      int grows = G - 1, grows_tmp = G, count = start_of(G);
+      while (start_of(grows + 1) == start_of(grows)) grows--;  // the last shell with cells
+      if (count >= a.nB) {
+        if (l16 == 0) atomicOr(a.err, 2);
+        G = -1;
+      } else if (den < (double)a.Bt[count]) {
+        // shells come off from the outside in; each one's values and the
+        // barrier of the cells left are loaded one shell ahead
+        int c1 = start_of(grows + 1), c0 = start_of(grows);
+        T bt = a.Bt[c0];
+        row_load(va, a.delta, s_tab, a, c0, c1, l16, grows <= c.flat, c);
+        for (;;) {
+          const int cn = grows > 0 ? start_of(grows - 1) : 0;
+          T btn = 0;
+          if (grows > 0) {
+            btn = a.Bt[cn];
+            row_load(vb, a.delta, s_tab, a, cn, c0, l16, grows <= c.flat, c);
+          }
+          den = den * (double)count;
+#pragma unroll
+          for (int k = 0; k < ROW_K; k++)
+            if (c0 + 16 * k < c1) row_sub<0>(den, va[k]);
+          for (int o = c0 + 16 * ROW_K; o < c1; o += 16 * ROW_K) {
+            row_load(va, a.delta, s_tab, a, o, c1, l16, grows <= c.flat, c);
+#pragma unroll
+            for (int k = 0; k < ROW_K; k++)
+              if (o + 16 * k < c1) row_sub<0>(den, va[k]);
+          }
+          count -= c1 - c0;
+          if (count > 0) den = den / (double)count;
+          if (c1 > c0) grows_tmp = grows;
+          grows--;
+          if (!(den < (double)bt && count > 0)) break;
+          if (grows < 0) {  // cannot happen while count > 0 on an unclamped table
+            if (l16 == 0) atomicOr(a.err, 32);
+            G = -1;
+            break;
+          }
+          bt = btn;
+          c1 = c0;
+          c0 = cn;
+#pragma unroll
+          for (int k = 0; k < ROW_K; k++) va[k] = vb[k];
+        }
+      }
+      if (G >= 0) {
+        // the read ball r^2 <= G: claim its cells of r^2 < G and look for the
+        // centre of a denser pending candidate (flags change in k_commit
+        // only, so every candidate sees those of the round's start).  In
+        // memory order the atomics of a run along k share requests: global
+        // atomics run at 26 G requests of 64 bytes a second, whatever they
+        // touch.
+        const bool tabled = G < a.sh.ball_max;
+        const unsigned* offs = tabled ? a.sh.balls + a.sh.ball[G + 1] : a.sh.offs;
+        const int rend = start_of(G + 1);
+        bool hit = false;
+        for (int ob = l16; ob < rend; ob += 64) {
+          unsigned p[4];
+          int f[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) p[k] = ob + 16 * k < rend ? offs[ob + 16 * k] : CENTRE_OFF;
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            const unsigned id = cell_off(c.i, c.j, c.k, p[k], a.n0, a.n1, a.n2);
+            f[k] = a.flag[id];
+            const int di = (int)(p[k] & 255u) - 128, dj = (int)((p[k] >> 8) & 255u) - 128,
+                      dk = (int)((p[k] >> 16) & 255u) - 128;
+            if (ob + 16 * k < rend && di * di + dj * dj + dk * dk < G)
+              claim_cell<C32>(a.claim, id, tag_hi, rank);
+          }
+#pragma unroll
+          for (int k = 0; k < 4; k++) hit |= f[k] <= FLAG_PENDING && FLAG_PENDING - f[k] < rank;
+        }
+        const bool blocked = ((__ballot(hit) >> (row * 16)) & 0xffffull) != 0;
+        if (l16 == 0) a.pres[t] = G << 16 | grows_tmp | (blocked ? PRES_BLOCKED : 0);
+      }
+    }
+    if (has && G < 0 && l16 == 0) a.pres[t] = -1;
   }
 }
 
 // Commit of the candidates that have seen their final flags: no denser
-// pending candidate claims a cell of their read ball (r^2 <= G).  As in
+// pending candidate claims a cell of their read ball (r^2 <= G) or has its
+// centre there (k_grow has looked for those; no two centres are neighbours,
+// so a candidate of one cell has no other in its ball).  As in
 // k_grow, one thread handles a candidate of one cell and a row of 16 lanes a
 // larger one.  The others are appended to their XCD's list of the next round
 // (in the order of the workgroups' atomics: the order of a list does not
 // change the result), in place of a count, a scan and a write pass (12 us a
 // round).  All rounds of the two boxes above: 283 -> 60 us, 2.6 -> 0.6 ms.
 template <typename T, bool C32, int CPB>
-__global__ __launch_bounds__(256) void k_commit(GrowArgs<T> a, RoundLists rl, T* pden_out,
+__global__ __launch_bounds__(256) void k_commit(GrowArgs<T> a, RoundLists rl,
                                                 unsigned long long tag_hi, int tmax) {
   __shared__ short s_at[CPB];
   __shared__ unsigned char s_retry[CPB];
@@ -637,10 +766,11 @@ __global__ __launch_bounds__(256) void k_commit(GrowArgs<T> a, RoundLists rl, T*
     const int t = base + threadIdx.x;
     bool more = false, retry = false;
     if ((int)threadIdx.x < m) {
-      const int G = a.pG[t];  // -1: skipped or failed
-      more = G > 1;
+      const int pr = a.pres[t], G = pr >> 16;  // -1: skipped or failed
+      retry = pr > 0 && (pr & PRES_BLOCKED);
+      more = G > 1 && !retry;
       if (G == 1) {
-        const int rank = a.prank[t], cell = a.pcell[t], count = a.pcnt[t];
+        const int rank = a.prank[t], p = a.ppeak[t], cell = a.pcell[p];
         int ci, cj, ck;
         decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
 #pragma unroll
@@ -649,15 +779,12 @@ __global__ __launch_bounds__(256) void k_commit(GrowArgs<T> a, RoundLists rl, T*
               a.claim,
               cell_off(ci, cj, ck, (unsigned)table_at((const int*)a.sh.offs, e), a.n0, a.n1, a.n2),
               tag_hi, rank);
-        if (!retry) {
-          const bool keep = count > 0 && count >= a.Nmin;
-          if (count > 0) {
-            a.flag[cell] = keep ? (rank << 1) | 1 : FLAG_REJECTED;
-            a.eff[cell] = a.negMtot;
-            a.cnt[rank] = count;
-            a.r2[rank] = 1;
-          }
-          a.kept[rank] = keep ? 1 : 0;
+        if (!retry && (pr & 0xffff) == 0) a.flag[cell] = FLAG_FREE;  // no halo, pending no more
+        if (!retry && (pr & 0xffff)) {
+          const bool keep = 1 >= a.Nmin;
+          a.flag[cell] = keep ? (rank << 1) | 1 : FLAG_REJECTED;
+          a.eff[cell] = a.negMtot;
+          if (keep) a.res[p] = 1;
         }
       }
     }
@@ -677,51 +804,53 @@ __global__ __launch_bounds__(256) void k_commit(GrowArgs<T> a, RoundLists rl, T*
     if (q >= nl) break;
     if (q + row >= nl) continue;
     const int at = s_at[q + row], t = base + at;
-    const int rank = a.prank[t], cell = a.pcell[t], G = a.pG[t], count = a.pcnt[t];
+    const int rank = a.prank[t], p = a.ppeak[t], cell = a.pcell[p], pr = a.pres[t], G = pr >> 16;
     int ci, cj, ck;
     decode_cell<T>(cell, a.n1, a.n2, ci, cj, ck);
     const int oend = a.sh.start[G + 1];
+    const unsigned* offs = G < a.sh.ball_max ? a.sh.balls + a.sh.ball[G + 1] : a.sh.offs;
     bool blocked = false;
     for (int ob = 0; ob < oend && !blocked; ob += 64) {
-      unsigned p[4];
+      unsigned off[4];
 #pragma unroll
       for (int k = 0; k < 4; k++)
-        p[k] = ob + 16 * k + l16 < oend ? a.sh.offs[ob + 16 * k + l16] : a.sh.offs[0];
+        off[k] = ob + 16 * k + l16 < oend ? offs[ob + 16 * k + l16] : CENTRE_OFF;
       bool hit = false;
 #pragma unroll
       for (int k = 0; k < 4; k++)
-        hit |= claimed<C32>(a.claim, cell_off(ci, cj, ck, p[k], a.n0, a.n1, a.n2), tag_hi, rank);
+        hit |= claimed<C32>(a.claim, cell_off(ci, cj, ck, off[k], a.n0, a.n1, a.n2), tag_hi, rank);
       blocked = ((__ballot(hit) >> (row * 16)) & 0xffffull) != 0;
     }
     if (blocked) {
       if (l16 == 0) s_retry[at] = 1;
       continue;
     }
-    if (count == 0) {
-      if (l16 == 0) a.kept[rank] = 0;
+    const int R2 = pr & 0xffff;
+    if (R2 == 0) {  // shrunk to no cell: no halo, pending no more
+      if (l16 == 0) a.flag[cell] = FLAG_FREE;
       continue;
     }
-    const int R2 = a.pr2[t];
     if (isqrt_floor(R2 - 1) > tmax) {  // flag sphere would wrap (reference writes past its cube)
-      if (l16 == 0) {
-        atomicOr(a.err, 4);
-        a.kept[rank] = 0;
-      }
+      if (l16 == 0) atomicOr(a.err, 4);
       continue;
     }
-    const bool keep = count >= a.Nmin;
-    const int v = keep ? (rank << 1) : FLAG_REJECTED;
     const int fend = a.sh.start[R2];
-    for (int o = l16; o < fend; o += 16) {  // cell 0 is the centre
-      const unsigned id = cell_off(ci, cj, ck, a.sh.offs[o], a.n0, a.n1, a.n2);
-      a.flag[id] = keep && o == 0 ? (rank << 1) | 1 : v;
-      a.eff[id] = a.negMtot;
+    const bool keep = fend >= a.Nmin;
+    const int v = keep ? (rank << 1) : FLAG_REJECTED;
+    const unsigned* fo = R2 <= a.sh.ball_max ? a.sh.balls + a.sh.ball[R2] : a.sh.offs;
+    for (int ob = l16; ob < fend; ob += 64) {
+      unsigned off[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) off[k] = ob + 16 * k < fend ? fo[ob + 16 * k] : 0u;
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (ob + 16 * k < fend) {
+          const unsigned id = cell_off(ci, cj, ck, off[k], a.n0, a.n1, a.n2);
+          a.flag[id] = keep && off[k] == CENTRE_OFF ? (rank << 1) | 1 : v;
+          a.eff[id] = a.negMtot;
+        }
     }
-    if (l16 == 0) {
-      a.kept[rank] = keep ? 1 : 0;
-      a.cnt[rank] = count;
-      a.r2[rank] = R2;
-    }
+    if (keep && l16 == 0) a.res[p] = (unsigned short)R2;
   }
   __syncthreads();
   // the candidates to retry, in this block's order
@@ -739,48 +868,78 @@ __global__ __launch_bounds__(256) void k_commit(GrowArgs<T> a, RoundLists rl, T*
     int o = x * rl.cap + s_base + __popcll(bal & lanemask_lt());
     for (int u = 0; u < w; u++) o += s_wave[u];
     const int t = base + threadIdx.x;
-    const int rank = a.prank[t], cell = a.pcell[t];
-    const T den = a.pden[t];
+    const int rank = a.prank[t], p = a.ppeak[t];
     rl.rank_out[o] = rank;
-    rl.cell_out[o] = cell;
-    pden_out[o] = den;
+    rl.peak_out[o] = p;
   }
-}
-
-// Counts of the first round's lists (contiguous ranges of the candidates'
-// order) and the error flag after the ring.
-__global__ void k_round_init(int* rt, int nc, int cap) {
-  const int q = threadIdx.x;
-  if (q < NXCD) rt[q] = min(max(nc - q * cap, 0), cap);
-  if (q >= NXCD && q < 2 * NXCD) rt[q] = 0;
-  if (q == 2 * NXCD) rt[RT_RING * NXCD] = 0;
 }
 
 // ---------------------------------------------------------------------------
 // catalogue, masses, flags, positions
 // ---------------------------------------------------------------------------
-__global__ void k_kept_to_int(const unsigned char* kept, long long n, long long* out) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x)
-    out[i] = kept[i];
+// Halos in rank order: the results by rank and their counts per block of
+// PK_TILE ranks, then (after the counts' scan) the halos and each rank's halo
+// number.
+__global__ __launch_bounds__(256) void k_halo_count(const unsigned short* res, const int* perm,
+                                                    int np, int nc, unsigned short* rres,
+                                                    long long* bcnt) {
+  __shared__ int sh[4];
+  const int r0 = (int)blockIdx.x * PK_TILE + (int)threadIdx.x;
+  int p[PK_ITEMS], v[PK_ITEMS], cnt = 0;
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++) p[q] = r0 + 256 * q < nc ? perm[np - 1 - (r0 + 256 * q)] : -1;
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++) v[q] = p[q] >= 0 ? res[p[q]] : 0;
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++) {
+    if (p[q] >= 0) rres[r0 + 256 * q] = (unsigned short)v[q];
+    cnt += __popcll(__ballot(v[q] != 0));
+  }
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = cnt;
+  __syncthreads();
+  if (threadIdx.x == 0) bcnt[blockIdx.x] = (long long)sh[0] + sh[1] + sh[2] + sh[3];
 }
 
 template <typename T>
-__global__ void k_gather_halos(const unsigned char* kept, const long long* hidx, long long nc,
-                               const int* ccell, const int* cnt, const int* r2, int n1, int n2,
-                               int* hx, int* hcount, int* hr2) {
-  for (long long r = blockIdx.x * (long long)blockDim.x + threadIdx.x; r < nc;
-       r += (long long)gridDim.x * blockDim.x) {
-    if (!kept[r]) continue;
-    const long long h = hidx[r];
-    const int cell = ccell[r], hc = cnt[r], hr = r2[r];  // all loads before the stores
-    int i, j, k;
-    decode_cell<T>(cell, n1, n2, i, j, k);
-    hx[3 * h] = i;
-    hx[3 * h + 1] = j;
-    hx[3 * h + 2] = k;
-    hcount[h] = hc;
-    hr2[h] = hr;
+__global__ __launch_bounds__(256) void k_gather_halos(const unsigned short* res,
+                                                      const long long* boff, int nc,
+                                                      const int* perm, const int* pcell, int np,
+                                                      const int* start, int n1, int n2, int* hx,
+                                                      int* hcount, int* hr2, int* hidx) {
+  __shared__ int wcnt[PK_ITEMS][4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int r0 = (int)blockIdx.x * PK_TILE + (int)threadIdx.x;
+  int R2[PK_ITEMS], cell[PK_ITEMS];
+  unsigned long long bal[PK_ITEMS];
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++) {
+    const int r = r0 + 256 * q;
+    R2[q] = r < nc ? res[r] : 0;
+    cell[q] = R2[q] ? perm[np - 1 - r] : 0;
+    bal[q] = __ballot(R2[q] != 0);
+    if (lane == 0) wcnt[q][w] = __popcll(bal[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++)
+    if (R2[q]) cell[q] = pcell[cell[q]];
+  __syncthreads();
+  int o = (int)boff[blockIdx.x];
+#pragma unroll
+  for (int q = 0; q < PK_ITEMS; q++) {
+    int ow = o;
+    for (int u = 0; u < w; u++) ow += wcnt[q][u];
+    const int h = ow + __popcll(bal[q] & lanemask_lt()), r = r0 + 256 * q;
+    if (r < nc) hidx[r] = h;
+    if (R2[q]) {
+      int i, j, k;
+      decode_cell<T>(cell[q], n1, n2, i, j, k);
+      hx[3 * (size_t)h] = i;
+      hx[3 * (size_t)h + 1] = j;
+      hx[3 * (size_t)h + 2] = k;
+      hcount[h] = start[R2[q]];
+      hr2[h] = R2[q];
+    }
+    o += wcnt[q][0] + wcnt[q][1] + wcnt[q][2] + wcnt[q][3];
   }
 }
 
@@ -884,12 +1043,12 @@ __global__ void k_mass_table(const int* sphere, int nt, T Mcell, const double* M
   }
 }
 
-__global__ void k_flag_out(const int* flag, long long ng, const long long* hidx, long long* out) {
+__global__ void k_flag_out(const int* flag, long long ng, const int* hidx, long long* out) {
   for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < ng;
        c += (long long)gridDim.x * blockDim.x) {
     int v = flag[c];
     long long o;
-    if (v == FLAG_FREE)
+    if (v == FLAG_FREE || v <= FLAG_PENDING)
       o = ng;
     else if (v == FLAG_REJECTED)
       o = ng + 1;
@@ -904,7 +1063,9 @@ __global__ void k_flag_out(const int* flag, long long ng, const long long* hidx,
 // Halo displacements: the mean over the member sphere, summed in double.  A
 // halo of one cell (81% of a 512^3 box's at 4 Mpc/h) takes one thread, a
 // larger one a row of 16 lanes that share its cells, so that no wave waits
-// for one thread's chain of loads through hundreds of cells.
+// for one thread's chain of loads through hundreds of cells.  The halos stand
+// in order of density, so a workgroup's are of similar size: HPB = 16 of them
+// (one a row) where there are few halos, else 256.
 template <typename T, bool VEL>
 __device__ __forceinline__ void posh_store(const double* s, const double* v, int hc, int ci,
                                            int cj, int ck, T Lc, T L0, T L1, T L2, T* posh,
@@ -922,17 +1083,17 @@ __device__ __forceinline__ void posh_store(const double* s, const double* v, int
   }
 }
 
-template <typename T, bool VEL>
+template <typename T, bool VEL, int HPB>
 __global__ __launch_bounds__(256) void k_halo_posh(const int* hx, const int* hcount,
                                                    const int* hr2, long long nh, ShellTab sh,
                                                    int n0, int n1, int n2, const T* S, const T* V,
                                                    T Lc, T L0, T L1, T L2, int lagrangian,
                                                    T* posh, T* velh) {
-  __shared__ short s_at[256];
-  __shared__ int s_end[256];
+  __shared__ short s_at[HPB];
+  __shared__ int s_end[HPB];
   __shared__ int nlist, taken;
   using V3 = typename vec3<T>::type;
-  const long long h0 = blockIdx.x * 256ll, h = h0 + threadIdx.x;
+  const long long h0 = blockIdx.x * (long long)HPB, h = h0 + threadIdx.x;
   const int lane = threadIdx.x & 63;
   if (threadIdx.x == 0) {
     nlist = 0;
@@ -941,7 +1102,7 @@ __global__ __launch_bounds__(256) void k_halo_posh(const int* hx, const int* hco
   __syncthreads();
   int end = 0;
   bool more = false;
-  if (h < nh) {
+  if ((int)threadIdx.x < HPB && h < nh) {
     const int ci = hx[3 * h], cj = hx[3 * h + 1], ck = hx[3 * h + 2], hc = hcount[h];
     end = lagrangian ? 0 : table_at(sh.start, hr2[h]);
     more = end > 1;
@@ -1020,25 +1181,43 @@ __global__ __launch_bounds__(256) void k_halo_posh(const int* hx, const int* hco
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Upload the shell table for (stab, tmax) unless the context already holds
-// it; returns the number of offsets.
+// Upload the shell and ball tables for (stab, tmax) unless the context already
+// holds them; returns the number of offsets.  Offsets of r^2 < stab lie within
+// sqrt(stab - 1), so a larger tmax gives the same tables.
 static long long ensure_shells(exh_ctx* c, int stab, int tmax) {
   HaloState& S = c->halo;
+  tmax = std::min(tmax, isqrt_floor(stab - 1));
   if (S.sh.stab == stab && S.sh_tmax == tmax) return c->shell_noffs;
-  std::vector<int> start;
-  std::vector<unsigned> packed;
+  std::vector<int> start, ball(BALL_MAX + 1, 0);
+  std::vector<unsigned> packed, balls;
   shell_offsets(stab, tmax, start, packed);
-  size_t bytes = (start.size() + packed.size()) * 4;
-  int* d = (int*)ctx_buf(c, BUF_SHELL, bytes);
-  EXH_CHECK_HIP(hipMemcpyAsync(d, start.data(), start.size() * 4, hipMemcpyHostToDevice, c->stream));
-  EXH_CHECK_HIP(hipMemcpyAsync(d + start.size(), packed.data(), packed.size() * 4,
-                               hipMemcpyHostToDevice, c->stream));
+  const int bmax = std::min(BALL_MAX, stab);
+  for (int G = 1; G <= bmax; G++) {
+    ball[G] = (int)balls.size();
+    balls.insert(balls.end(), packed.begin(), packed.begin() + start[G]);
+    auto memory_order = [](unsigned p) {
+      return (p & 255u) << 16 | (p & 0xff00u) | p >> 16;
+    };
+    std::sort(balls.begin() + ball[G], balls.end(), [&](unsigned p, unsigned q) {
+      return memory_order(p) < memory_order(q);
+    });
+  }
+  const size_t ns = start.size(), nb = ball.size(), no = packed.size();
+  std::vector<unsigned> all(start.begin(), start.end());
+  all.insert(all.end(), ball.begin(), ball.end());
+  all.insert(all.end(), packed.begin(), packed.end());
+  all.insert(all.end(), balls.begin(), balls.end());
+  int* d = (int*)ctx_buf(c, BUF_SHELL, all.size() * 4);
+  EXH_CHECK_HIP(hipMemcpyAsync(d, all.data(), all.size() * 4, hipMemcpyHostToDevice, c->stream));
   EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
   S.sh.start = d;
-  S.sh.offs = (const unsigned*)(d + start.size());
+  S.sh.ball = d + ns;
+  S.sh.offs = (const unsigned*)(d + ns + nb);
+  S.sh.balls = (const unsigned*)(d + ns + nb + no);
   S.sh.stab = stab;
+  S.sh.ball_max = bmax;
   S.sh_tmax = tmax;
-  c->shell_noffs = (long long)packed.size();
+  c->shell_noffs = (long long)no;
   return c->shell_noffs;
 }
 
@@ -1127,11 +1306,8 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
     c->halotab_bmin = (double)Bt[Ncells - 1];
   }
   const int Ncells = c->halotab_ncells;
-  char* misc = (char*)ctx_buf(c, BUF_MISC, 256);
-  const size_t o_cnt = 0;
-  long long* dcnt = (long long*)(misc + o_cnt);  // [0..7] scratch counters
-  long long* hbuf = (long long*)ctx_pinned(c, 1024);
-
+  unsigned long long* below_d = (unsigned long long*)ctx_buf(c, BUF_MISC, 256);
+  const T Bmin = (T)c->halotab_bmin;
   // 1. peaks
   long long nblk = (ng + PK_TILE - 1) / PK_TILE;
   const PeakGeom pg{n0, n1, n2, (unsigned)((long long)n1 * n2), (unsigned)n2, fast_div(n2),
@@ -1147,10 +1323,11 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   {
     TimedScope ts(c, "peaks");
     hipLaunchKernelGGL(k_peak_count<T>, dim3((unsigned)nblk), dim3(256), 0, c->stream, delta, pg,
-                       bc, eff, pbits);
+                       bc, eff, pbits, below_d);
     EXH_LAUNCH_CHECK();
     exclusive_scan<long long>(c, bc, bc + nblk + 1, nblk);
   }
+  long long* hbuf = (long long*)ctx_pinned(c, 1024);
   EXH_CHECK_HIP(hipMemcpyAsync(hbuf, bc + nblk + 1 + nblk, 8, hipMemcpyDeviceToHost, c->stream));
   EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
   const long long np = hbuf[0];
@@ -1160,27 +1337,22 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   {
     TimedScope ts(c, "peaks_write");
     hipLaunchKernelGGL(k_peak_write<T>, dim3((unsigned)nblk), dim3(256), 0, c->stream, delta, pg,
-                       bc + nblk + 1, pbits, pkey, pcell, flag);
+                       bc + nblk + 1, pbits, Bmin, pkey, pcell, flag, below_d);
     EXH_LAUNCH_CHECK();
   }
-  // 2. sort (densities in lexicographic peak order; each peak's cell rides
-  // along as the value).  Peaks below the smallest barrier are never
-  // visited: their count is the first visited sorted position, and the
-  // sort leaves their order open.
-  const T Bmin = (T)c->halotab_bmin;
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->stream, (unsigned long long*)dcnt, 1,
-                     0ull);
-  hipLaunchKernelGGL(k_count_below<T>, dim3(grid_for(np, 256 * 16)), dim3(256), 0, c->stream,
-                     pkey, np, Bmin, (unsigned long long*)dcnt);
-  EXH_LAUNCH_CHECK();
-  lomuto_sort<T>(c, pkey, pcell, np, (double)Bmin);
+  // 2. sort (densities in lexicographic peak order).  Peaks below the smallest
+  // barrier are never visited: their count is the first visited sorted
+  // position, and the sort leaves their order open.
+  unsigned long long* below_h = (unsigned long long*)((char*)hbuf + 1016);
+  EXH_CHECK_HIP(hipMemcpyAsync(below_h, below_d, 8, hipMemcpyDeviceToHost, c->stream));
+  int* perm = (int*)ctx_buf(c, BUF_PEAK_IDX, (size_t)std::max(np, 1LL) * sizeof(int));
+  lomuto_sort<T>(c, pkey, perm, np, (double)Bmin);
   if (phase) phase(1);
 
-  // 3. candidates (the sort stages its state in the same pinned buffer)
-  EXH_CHECK_HIP(hipMemcpyAsync(hbuf, dcnt, 8, hipMemcpyDeviceToHost, c->stream));
-  EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
-  long long lb = std::max(hbuf[0], 1LL);
-  long long nc = np > lb ? np - lb : 0;
+  // 3. candidates (the sort has waited for the stream in its levels)
+  if (c->stat_sort_levels == 0) EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
+  const long long below = (long long)*below_h;
+  const long long nc = std::max(np - std::max(below, 1LL), 0LL);
   c->stat_candidates = nc;
 
   // candidate state in BUF_CAND: by rank, by list position, lists' counts
@@ -1190,28 +1362,19 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
     coff += (bytes + 255) & ~(size_t)255;
     return r;
   };
-  size_t ncs = (size_t)std::max(nc, 1LL);
-  // positions per XCD list of pending candidates
-  const long long lcap = ((nc + NXCD - 1) / NXCD + 255) / 256 * 256;
-  const size_t nls = (size_t)std::max(lcap * NXCD, 1LL);
-  // first-round order: bricks of 2^bsh x 2^bsh cells (16 x 16, wider on big
-  // grids so that the brick histogram fits in LDS)
-  int bsh = 4;
-  while ((long long)((n0 + (1 << bsh) - 1) >> bsh) * ((n1 + (1 << bsh) - 1) >> bsh) > ORD_MAXB)
-    bsh++;
-  const int nby = (n1 + (1 << bsh) - 1) >> bsh;
-  const int nbr = ((n0 + (1 << bsh) - 1) >> bsh) * nby;
-  const long long nblk_r = std::max((nc + ORD_RB - 1) / ORD_RB, 1LL);
-  const size_t o_c = ctake(ncs * 4), o_r = ctake(ncs * 4), o_k = ctake(ncs),
-         o_p0 = ctake(nls * 4), o_p1 = ctake(nls * 4), o_kl = ctake((ncs + 1) * 8),
-         o_hid = ctake((ncs + 1) * 8), o_cc = ctake(ncs * 4), o_cd = ctake(ncs * sizeof(T)),
-         o_bk = ctake(((size_t)nbr * nblk_r + 1) * 4), o_pc0 = ctake(nls * 4),
-         o_pc1 = ctake(nls * 4), o_pd0 = ctake(nls * sizeof(T)), o_pd1 = ctake(nls * sizeof(T)),
-         o_pg = ctake(nls * 4), o_pn = ctake(nls * 4), o_pr = ctake(nls * 4),
-         o_rt = ctake((RT_RING * NXCD + 1) * 4);
+  const size_t ncs = (size_t)std::max(nc, 1LL);
+  // list x may hold every peak of its blocks
+  const long long nblk_p = std::max((np + PK_TILE - 1) / PK_TILE, 1LL);
+  const long long lcap = (nblk_p + NXCD - 1) / NXCD * PK_TILE;
+  const size_t nls = (size_t)lcap * NXCD;
+  const long long nblk_c = (nc + PK_TILE - 1) / PK_TILE;
+  const size_t nps = (size_t)std::max(np, 1LL);
+  const size_t o_res = ctake(nps * 2), o_rres = ctake(ncs * 2), o_p0 = ctake(nls * 4),
+               o_p1 = ctake(nls * 4), o_rk = ctake(nps * 4), o_hid = ctake(ncs * 4),
+               o_pk0 = ctake(nls * 4), o_pk1 = ctake(nls * 4), o_pg = ctake(nls * 4),
+               o_hb = ctake((size_t)(2 * std::max(nblk_c, 1LL) + 2) * 8),
+               o_rt = ctake((RT_RING * NXCD + 1) * 4);
   char* cand = (char*)ctx_buf(c, BUF_CAND, coff);
-  int* ccell = (int*)(cand + o_cc);
-  T* cden = (T*)(cand + o_cd);
   // eff (delta) and the free flags were written by the peak passes
   S.flag = flag;
   int* rt = (int*)(cand + o_rt);
@@ -1231,34 +1394,24 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   ga.Bmin = Bmin;
   ga.negMtot = -(T)b->Mtot;
   ga.Nmin = o->Nmin;
-  ga.pG = (int*)(cand + o_pg);
-  ga.pcnt = (int*)(cand + o_pn);
-  ga.pr2 = (int*)(cand + o_pr);
-  ga.cnt = (int*)(cand + o_c);
-  ga.r2 = (int*)(cand + o_r);
-  ga.kept = (unsigned char*)(cand + o_k);
+  ga.pcell = pcell;
+  ga.pkey = pkey;
+  ga.pres = (int*)(cand + o_pg);
+  ga.res = (unsigned short*)(cand + o_res);
   ga.err = derr;
   int* pend = (int*)(cand + o_p0);
   int* pnext = (int*)(cand + o_p1);
-  int* qcell = (int*)(cand + o_pc0);
-  int* qcell_next = (int*)(cand + o_pc1);
-  T* qden = (T*)(cand + o_pd0);
-  T* qden_next = (T*)(cand + o_pd1);
+  int* qpeak = (int*)(cand + o_pk0);
+  int* qpeak_next = (int*)(cand + o_pk1);
   {
     TimedScope ts(c, "halo_candidates");
-    hipLaunchKernelGGL(k_cand_setup<T>, dim3(grid_for(nc, 256 * 4)), dim3(256), 0, c->stream,
-                       pkey, pcell, np, lb, ccell, cden);
-    EXH_LAUNCH_CHECK();
-    if (nc > 0) {
-      int* bk = (int*)(cand + o_bk);
-      hipLaunchKernelGGL(k_brick_hist, dim3((unsigned)nblk_r), dim3(256), 0, c->stream, ccell, nc,
-                         n1, n2, bsh, nby, nbr, (int)nblk_r, bk);
-      EXH_LAUNCH_CHECK();
-      exclusive_scan<int>(c, bk, bk, (long long)nbr * nblk_r);
-      hipLaunchKernelGGL(k_brick_scatter<T>, dim3((unsigned)nblk_r), dim3(256), 0, c->stream,
-                         ccell, cden, nc, n1, n2, bsh, nby, nbr, (int)nblk_r, bk, pend, qcell,
-                         qden);
-    }
+    int* rank = (int*)(cand + o_rk);
+    const long long nrk = std::max(np - below, 1LL);
+    hipLaunchKernelGGL(k_cand_ranks, dim3(grid_for(nrk, 1024)), dim3(256), 0, c->stream, perm,
+                       (int)np, (int)below, rank, rt);
+    hipLaunchKernelGGL(k_list_build<T>, dim3((unsigned)nblk_p), dim3(256), 0, c->stream, pkey,
+                       pcell, rank, (int)np, (int)nc, Bmin, (int)lcap, rt, pend, qpeak, ga.res,
+                       flag);
     EXH_LAUNCH_CHECK();
   }
   if (phase) phase(2);
@@ -1267,8 +1420,6 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   // sized by the last count the host read (counts only shrink), and the
   // host reads the counts and the error flag once per batch.  A round with
   // no pending candidate launches blocks that return at once.
-  hipLaunchKernelGGL(k_round_init, dim3(1), dim3(64), 0, c->stream, rt, (int)nc, (int)lcap);
-  EXH_LAUNCH_CHECK();
   // Claims carry their round's tag (an epoch counted over the context's
   // calls) above the inverted rank, so the claims of earlier rounds and
   // calls never match a later round: the array is cleared only when it is
@@ -1291,7 +1442,7 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   }
   // candidates per workgroup: 256, or 64 (16 rows for their long growths)
   // where 256 would leave most CUs idle
-  long long ub = nc > 0 ? lcap : 0;  // the longest list
+  long long ub = nc > 0 ? std::min(lcap, nc) : 0;  // bounds the longest list
   int round = 0, launched = 0;
   {
     TimedScope ts(c, "halo_rounds");
@@ -1307,17 +1458,16 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
         rl.clear = rt + (launched + 2) % RT_RING * NXCD;
         rl.cap = (int)lcap;
         rl.rank_out = pnext;
-        rl.cell_out = qcell_next;
+        rl.peak_out = qpeak_next;
         launched++;
         if (c32 && c->claim_epoch >= 255) clear_claims();
         const unsigned long long ep = ++c->claim_epoch;
         const unsigned long long tag_hi = c32 ? ep << 24 : ep << 32;
         ga.prank = pend;
-        ga.pcell = qcell;
-        ga.pden = qden;
+        ga.ppeak = qpeak;
         auto go = [&](auto kg, auto kc) {
           hipLaunchKernelGGL(kg, grid, dim3(256), 0, c->stream, ga, rl, tag_hi);
-          hipLaunchKernelGGL(kc, grid, dim3(256), 0, c->stream, ga, rl, qden_next, tag_hi, tmax);
+          hipLaunchKernelGGL(kc, grid, dim3(256), 0, c->stream, ga, rl, tag_hi, tmax);
         };
         if (c32 && cpb == 256)
           go(k_grow<T, true, 256>, k_commit<T, true, 256>);
@@ -1329,8 +1479,7 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
           go(k_grow<T, false, 64>, k_commit<T, false, 64>);
         EXH_LAUNCH_CHECK();
         std::swap(pend, pnext);
-        std::swap(qcell, qcell_next);
-        std::swap(qden, qden_next);
+        std::swap(qpeak, qpeak_next);
       }
       int* hr = (int*)hbuf;  // the ring and the error flag
       EXH_CHECK_HIP(hipMemcpyAsync(hr, rt, (RT_RING * NXCD + 1) * 4, hipMemcpyDeviceToHost,
@@ -1354,15 +1503,19 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   c->stat_rounds = round;
 
   // 4. catalogue
-  long long* kl = (long long*)(cand + o_kl);
-  long long* hidx = (long long*)(cand + o_hid);
-  hipLaunchKernelGGL(k_kept_to_int, dim3(grid_for(nc, 256 * 8)), dim3(256), 0, c->stream,
-                     ga.kept, nc, kl);
-  EXH_LAUNCH_CHECK();
-  exclusive_scan<long long>(c, kl, hidx, nc);
-  EXH_CHECK_HIP(hipMemcpyAsync(hbuf, hidx + nc, 8, hipMemcpyDeviceToHost, c->stream));
-  EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
-  const long long nh = hbuf[0];
+  long long* hb2 = (long long*)(cand + o_hb);
+  int* hidx = (int*)(cand + o_hid);
+  unsigned short* rres = (unsigned short*)(cand + o_rres);
+  long long nh = 0;
+  if (nc > 0) {
+    hipLaunchKernelGGL(k_halo_count, dim3((unsigned)nblk_c), dim3(256), 0, c->stream, ga.res,
+                       perm, (int)np, (int)nc, rres, hb2);
+    EXH_LAUNCH_CHECK();
+    exclusive_scan<long long>(c, hb2, hb2 + nblk_c + 1, nblk_c);
+    EXH_CHECK_HIP(hipMemcpyAsync(hbuf, hb2 + 2 * nblk_c + 1, 8, hipMemcpyDeviceToHost, c->stream));
+    EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
+    nh = hbuf[0];
+  }
   S.hidx = hidx;
   size_t hs = (size_t)std::max(nh, 1LL);
   size_t hoff = 0;
@@ -1385,8 +1538,10 @@ long long run_find_halos(exh_ctx* c, const exh_box* b, const T* delta, const exh
   S.Mh = hal + o_mh;
   S.posh = hal + o_ph;
   S.velh = hal + o_vh;
-  hipLaunchKernelGGL(k_gather_halos<T>, dim3(grid_for(nc, 256)), dim3(256), 0, c->stream,
-                     ga.kept, hidx, nc, ccell, ga.cnt, ga.r2, n1, n2, S.hx, S.hcount, S.hr2);
+  if (nh > 0)
+    hipLaunchKernelGGL(k_gather_halos<T>, dim3((unsigned)nblk_c), dim3(256), 0, c->stream, rres,
+                       hb2 + nblk_c + 1, (int)nc, perm, pcell, (int)np, S.sh.start, n1, n2, S.hx,
+                       S.hcount, S.hr2, hidx);
   EXH_LAUNCH_CHECK();
   // 5. masses
   if (nh > 0) {
@@ -1426,8 +1581,10 @@ void run_halo_posh(exh_ctx* c, const exh_box* b, const T* S, const T* V, int lag
   HaloState& st = c->halo;
   if (c->nh <= 0) return;
   TimedScope ts(c, "halo_posh");
-  auto kern = V ? k_halo_posh<T, true> : k_halo_posh<T, false>;
-  hipLaunchKernelGGL(kern, dim3(grid_for(c->nh, 256)), dim3(256), 0, c->stream, st.hx, st.hcount,
+  const bool few = c->nh < 256 * 1024;
+  auto kern = few ? (V ? k_halo_posh<T, true, 16> : k_halo_posh<T, false, 16>)
+                  : (V ? k_halo_posh<T, true, 256> : k_halo_posh<T, false, 256>);
+  hipLaunchKernelGGL(kern, dim3(grid_for(c->nh, few ? 16 : 256)), dim3(256), 0, c->stream, st.hx, st.hcount,
                      st.hr2, c->nh, st.sh, b->nd[0], b->nd[1], b->nd[2], S, V, (T)b->Lc,
                      (T)b->L[0], (T)b->L[1], (T)b->L[2], lagrangian, (T*)st.posh,
                      V ? (T*)st.velh : nullptr);

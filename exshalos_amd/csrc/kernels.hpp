@@ -40,12 +40,13 @@ template <typename T>
 void run_halo_posh(exh_ctx* c, const exh_box* b, const T* S, const T* V, int lagrangian);
 void run_halo_flag(exh_ctx* c, const exh_box* b, long long* flag_dev);
 
-// sort.hip: Lomuto quicksort emulation (ascending, "<=" left, pivot last).
+// sort.hip: Lomuto quicksort emulation (ascending, "<=" left, pivot last):
+// perm[l] = index of the key that the sort puts at position l.
 // With m keys below `floor`, positions m.. hold exactly what the full sort
 // puts there; positions below m are unspecified (segments of keys below
 // `floor` are not sorted further).
 template <typename K>
-void lomuto_sort(exh_ctx* c, K* keys, int* vals, long long n,
+void lomuto_sort(exh_ctx* c, const K* keys, int* perm, long long n,
                  double floor = -std::numeric_limits<double>::infinity());
 
 // spectrum.hip

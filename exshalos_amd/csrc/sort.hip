@@ -24,7 +24,10 @@
 //
 // Large segments (> SMALL) are processed level by level with tile kernels
 // across the whole device; segments of 2..SMALL elements are finished by one
-// wavefront each in LDS with the same partition rule.
+// workgroup each in LDS with the same partition rule.
+//
+// The result is the permutation alone: perm[l] is the index of the key that
+// the reference's sort puts at position l.  The keys are left as they are.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "util.hpp"
@@ -45,9 +48,10 @@ struct SegInfo {
 // ---------------------------------------------------------------------------
 // level kernels
 //
-// Keys and values move between two work buffers level by level (src ->
-// dst).  Elements whose place is final (pivots, children of one element)
-// are also written to the output array; segments of 2..SMALL elements are
+// Keys and indices move between two work buffers level by level (src ->
+// dst; the first level reads the input keys, whose indices are their
+// positions).  The indices of elements whose place is final (pivots, children
+// of one element) are also written to the output; segments of 2..SMALL elements are
 // queued with the buffer that holds them and finished by k_small_sort.
 // Children of more than SMALL elements become the next level's segments:
 // each reserves its list slot and its range of tiles with one packed 64-bit
@@ -109,6 +113,18 @@ __global__ void k_sort_init(long long* lo, long long* hi, long long* toff, unsig
     *st = LevelState{};
   }
 }
+
+// One small segment: the whole input.
+__global__ void k_small_init(long long* slo, long long* shi, int* sbuf, long long n) {
+  if (threadIdx.x == 0) {
+    slo[0] = 0;
+    shi[0] = n - 1;
+    sbuf[0] = 0;
+  }
+}
+
+// Index carried by element j (the first level's are their positions).
+__device__ inline int val_at(const int* vals, long long j) { return vals ? vals[j] : (int)j; }
 
 __device__ inline int find_seg(const long long* tile_off, int nseg, long long t) {
   int lo = 0, hi = nseg;  // tile_off[lo] <= t < tile_off[hi]
@@ -222,8 +238,7 @@ __device__ inline void push_child(const LevelBufs& b, long long cl, long long ch
 // queues the two children.
 template <typename K>
 __global__ __launch_bounds__(256) void k_tile_scatter(const K* keysA, const int* valsA, K* keysB,
-                                                      int* valsB, K* keysF, int* valsF,
-                                                      LevelBufs b, const long long* tile_pre,
+                                                      int* valsB, int* perm, LevelBufs b, const long long* tile_pre,
                                                       int* arot, int* s0) {
   __shared__ int shw[4];
   const long long t = blockIdx.x;
@@ -234,8 +249,7 @@ __global__ __launch_bounds__(256) void k_tile_scatter(const K* keysA, const int*
   if (t == g.first_tile && threadIdx.x == 0) {
     b.info[sg] = g;
     b.seg_need[sg] = 0;
-    keysF[g.lo + g.c] = pivot;
-    valsF[g.lo + g.c] = valsA[g.hi];
+    perm[g.lo + g.c] = val_at(valsA, g.hi);
     if (m > 0) arot[g.lo + g.r - 1] = (int)m;
     if (!((double)pivot < b.floor)) push_child(b, g.lo, g.lo + g.c - 1);
     push_child(b, g.lo + g.c + 1, g.hi);
@@ -257,7 +271,7 @@ __global__ __launch_bounds__(256) void k_tile_scatter(const K* keysA, const int*
   // alias them for the compiler)
   for (int q = 0; q < PER_THREAD; q++) {
     const long long j = base + q * 64 + lane;
-    vv[q] = (bal[q] >> lane) & 1ull ? valsA[j] : 0;
+    vv[q] = (bal[q] >> lane) & 1ull ? val_at(valsA, j) : 0;
   }
   if (lane == 0) shw[w] = wcnt;
   __syncthreads();
@@ -273,10 +287,7 @@ __global__ __launch_bounds__(256) void k_tile_scatter(const K* keysA, const int*
       if ((bal[q] >> lane) & 1ull) {
         keysB[g.lo + rank] = kv[q];
         valsB[g.lo + rank] = vv[q];
-        if (single_left) {
-          keysF[g.lo] = kv[q];
-          valsF[g.lo] = vv[q];
-        }
+        if (single_left) perm[g.lo] = vv[q];
         if (g.r > 0 && j > g.j0) arot[g.lo + rank - jlead] = (int)((j - g.lo) - rank);
       } else {
         const long long gt_before = (j - g.lo) - rank;
@@ -298,8 +309,7 @@ static constexpr int S0_DONE = 0x7fffffff;
 
 template <typename K>
 __global__ __launch_bounds__(256) void k_tile_chase(const K* keysA, const int* valsA, K* keysB,
-                                                    int* valsB, K* keysF, int* valsF,
-                                                    LevelBufs b, const int* arot, int* s0,
+                                                    int* valsB, int* perm, LevelBufs b, const int* arot, int* s0,
                                                     int* jmp, int cap) {
   const long long t = blockIdx.x;
   const int sg = b.tseg[t];
@@ -349,7 +359,7 @@ __global__ __launch_bounds__(256) void k_tile_chase(const K* keysA, const int* v
   int ld[PER_THREAD];
   for (int q = 0; q < PER_THREAD; q++) {
     const long long j = start + (long long)q * 256 + threadIdx.x;
-    ld[q] = !act[q] ? 0 : (s[q] < r ? A[s[q]] : valsA[j]);
+    ld[q] = !act[q] ? 0 : (s[q] < r ? A[s[q]] : val_at(valsA, j));
   }
   for (int q = 0; q < PER_THREAD; q++) {
     if (!act[q]) continue;
@@ -364,10 +374,7 @@ __global__ __launch_bounds__(256) void k_tile_chase(const K* keysA, const int* v
     const long long dst = g.lo + g.c + 1 + (s[q] - r);
     keysB[dst] = kv[q];
     valsB[dst] = ld[q];
-    if (single_right) {
-      keysF[dst] = kv[q];
-      valsF[dst] = ld[q];
-    }
+    if (single_right) perm[dst] = ld[q];
   }
   __shared__ unsigned long long sh_rem[4];
   for (int o = 32; o > 0; o >>= 1) rem = max(rem, (unsigned long long)__shfl_xor(rem, o, 64));
@@ -412,8 +419,7 @@ static int chase_cap() {
 // converged, since every pointer leads forward along its own chain.
 template <typename K>
 __global__ __launch_bounds__(256) void k_double_walk(const K* keysA, const int* valsA, K* keysB,
-                                                     int* valsB, K* keysF, int* valsF, LevelBufs b,
-                                                     int* jmp, const int* s0, int guard) {
+                                                     int* valsB, int* perm, LevelBufs b, int* jmp, const int* s0, int guard) {
   const long long t = blockIdx.x;
   const int sg = b.tseg[t];
   if (!b.seg_need[sg]) return;
@@ -464,11 +470,9 @@ __global__ __launch_bounds__(256) void k_double_walk(const K* keysA, const int* 
     }
     const long long dst = g.lo + g.c + 1 + (s - g.r);
     keysB[dst] = keysA[j];
-    valsB[dst] = valsA[j];
-    if (single_right) {
-      keysF[dst] = keysA[j];
-      valsF[dst] = valsA[j];
-    }
+    const int v = val_at(valsA, j);
+    valsB[dst] = v;
+    if (single_right) perm[dst] = v;
   }
   if (open) atomicExch(&b.st->async_open, 1ull);
 }
@@ -510,8 +514,8 @@ __global__ __launch_bounds__(256) void k_double_round(LevelBufs b, int* jmp, int
 // converged or not.  Walks left short set async_open (strict = 0: the host
 // then runs the synchronous rounds and this kernel again) or err (strict).
 template <typename K>
-__global__ void k_tile_chase2(const K* keysA, const int* valsA, K* keysB, int* valsB, K* keysF,
-                              int* valsF, LevelBufs b, const int* jmp, const int* s0,
+__global__ void k_tile_chase2(const K* keysA, const int* valsA, K* keysB, int* valsB, int* perm,
+                              LevelBufs b, const int* jmp, const int* s0,
                               int strict) {
   const long long t = blockIdx.x;
   const int sg = b.tseg[t];
@@ -533,11 +537,9 @@ __global__ void k_tile_chase2(const K* keysA, const int* valsA, K* keysB, int* v
     }
     const long long dst = g.lo + g.c + 1 + (s - g.r);
     keysB[dst] = keysA[j];
-    valsB[dst] = valsA[j];
-    if (single_right) {
-      keysF[dst] = keysA[j];
-      valsF[dst] = valsA[j];
-    }
+    const int v = val_at(valsA, j);
+    valsB[dst] = v;
+    if (single_right) perm[dst] = v;
   }
 }
 
@@ -685,7 +687,7 @@ static constexpr int SMALL_BATCH = 1024;  // segments per small-sort launch, at 
 
 template <typename K, int SMALL>
 __global__ __launch_bounds__(64 * SMALL_WAVES) void k_small_sort(
-    K* keys, int* vals, const K* keys1, const int* vals1, const K* keys2, const int* vals2,
+    int* perm, const K* keys, const K* keys1, const int* vals1, const K* keys2, const int* vals2,
     const long long* seg_lo, const long long* seg_hi, const int* seg_buf) {
   static_assert(SMALL <= 32767, "LDS indices are 16-bit");
   constexpr int NT = 64 * SMALL_WAVES;
@@ -705,10 +707,10 @@ __global__ __launch_bounds__(64 * SMALL_WAVES) void k_small_sort(
   const int n = (int)(seg_hi[blockIdx.x] - base + 1);
   const int buf = seg_buf[blockIdx.x];
   const K* srck = buf == 0 ? keys : (buf == 1 ? keys1 : keys2);
-  const int* srcv = buf == 0 ? vals : (buf == 1 ? vals1 : vals2);
+  const int* srcv = buf == 0 ? nullptr : (buf == 1 ? vals1 : vals2);
   for (int i = tid; i < n; i += NT) {
     sk[i] = srck[base + i];
-    sv[i] = srcv[base + i];
+    sv[i] = val_at(srcv, base + i);
   }
   if (tid == 0) {
     ntiny = 0;
@@ -881,10 +883,7 @@ __global__ __launch_bounds__(64 * SMALL_WAVES) void k_small_sort(
   __syncthreads();
   for (int q = tid; q < ntiny; q += NT) lane_quicksort<K>(sk, sv, tl_lo[q], tl_hi[q]);
   __syncthreads();
-  for (int i = tid; i < n; i += NT) {
-    keys[base + i] = sk[i];
-    vals[base + i] = sv[i];
-  }
+  for (int i = tid; i < n; i += NT) perm[base + i] = sv[i];
 }
 
 template <typename K>
@@ -899,13 +898,13 @@ struct SmallCfg<double> {
 };
 
 template <typename K>
-void lomuto_sort(exh_ctx* c, K* keys, int* vals, long long n, double floor) {
+void lomuto_sort(exh_ctx* c, const K* keys, int* perm, long long n, double floor) {
   TimedScope ts(c, "peak_sort");
   constexpr int SMALL = SmallCfg<K>::N;
   c->stat_sort_levels = 0;
   c->stat_sort_doubling = 0;
   c->stat_sort_async_open = 0;
-  if (n < 2) return;
+  if (n < 1) return;
   // scratch layout in BUF_SORT_AUX
   const long long maxseg = n / (SMALL + 1) * 2 + 4;
   const long long maxtiles = n / TILE + maxseg + 4;
@@ -931,7 +930,7 @@ void lomuto_sort(exh_ctx* c, K* keys, int* vals, long long n, double floor) {
                o_need = take(maxseg * 4 + 64), o_jmp = take((size_t)n * 4 + 64),
                o_tseg = take((maxtiles + 1) * 4);
   char* aux = (char*)ctx_buf(c, BUF_SORT_AUX, bytes);
-  // work buffers: 1 = B, 2 = C; the output (0) is `keys`/`vals`
+  // work buffers: 1 = B, 2 = C; 0 is the input
   K* kB = (K*)ctx_buf(c, BUF_SORT_K, (size_t)n * sizeof(K));
   int* vB = (int*)ctx_buf(c, BUF_SORT_V, (size_t)n * sizeof(int));
   K* kC = (K*)ctx_buf(c, BUF_SORT_K2, (size_t)n * sizeof(K));
@@ -989,25 +988,16 @@ void lomuto_sort(exh_ctx* c, K* keys, int* vals, long long n, double floor) {
     EXH_CHECK_HIP(hipStreamWaitEvent(c->side, c->ev_side_fork, 0));
     join.used = true;
     hipLaunchKernelGGL((k_small_sort<K, SMALL>), dim3((unsigned)(nsmall_host - nsmall_done)),
-                       dim3(64 * SMALL_WAVES), 0, c->side, keys, vals, kB, vB, kC, vC,
+                       dim3(64 * SMALL_WAVES), 0, c->side, perm, keys, kB, vB, kC, vC,
                        b.slo + nsmall_done, b.shi + nsmall_done, b.sbuf + nsmall_done);
     EXH_LAUNCH_CHECK();
     nsmall_done = nsmall_host;
   };
   if (n <= SMALL) {
-    long long init[2] = {0, n - 1};
-    int zero = 0;
-    EXH_CHECK_HIP(hipMemcpyAsync(b.slo, &init[0], 8, hipMemcpyHostToDevice, c->stream));
-    EXH_CHECK_HIP(hipMemcpyAsync(b.shi, &init[1], 8, hipMemcpyHostToDevice, c->stream));
-    EXH_CHECK_HIP(hipMemcpyAsync(b.sbuf, &zero, 4, hipMemcpyHostToDevice, c->stream));
-    EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
+    hipLaunchKernelGGL(k_small_init, dim3(1), dim3(64), 0, c->stream, b.slo, b.shi, b.sbuf, n);
+    EXH_LAUNCH_CHECK();
     nsmall_host = 1;
   } else {
-    // level 0 reads a copy, so pivots can be written to the output at once
-    EXH_CHECK_HIP(hipMemcpyAsync(kC, keys, (size_t)n * sizeof(K), hipMemcpyDeviceToDevice,
-                                 c->stream));
-    EXH_CHECK_HIP(hipMemcpyAsync(vC, vals, (size_t)n * sizeof(int), hipMemcpyDeviceToDevice,
-                                 c->stream));
     hipLaunchKernelGGL(k_sort_init, dim3(1), dim3(64), 0, c->stream,
                        (long long*)(aux + o_lo[0]), (long long*)(aux + o_hi[0]),
                        (long long*)(aux + o_toff[0]), (unsigned long long*)(aux + o_j0[0]), st, n);
@@ -1015,13 +1005,13 @@ void lomuto_sort(exh_ctx* c, K* keys, int* vals, long long n, double floor) {
     b.nseg = 1;
     b.ntiles = (n - 1 + TILE - 1) / TILE;
   }
-  // src/dst work buffers of the current level (ids 2 and 1 at level 0)
-  int src_id = 2;
+  // src/dst buffers of the current level (the input and 1 at level 0)
+  int src_id = 0;
   while (b.nseg > 0) {
     c->stat_sort_levels++;
-    const int dst_id = 3 - src_id;
-    K* ks = src_id == 1 ? kB : kC;
-    int* vs = src_id == 1 ? vB : vC;
+    const int dst_id = src_id == 1 ? 2 : 1;
+    const K* ks = src_id == 0 ? keys : (src_id == 1 ? kB : kC);
+    const int* vs = src_id == 0 ? nullptr : (src_id == 1 ? vB : vC);
     K* kd = dst_id == 1 ? kB : kC;
     int* vd = dst_id == 1 ? vB : vC;
     b.lo = (const long long*)(aux + o_lo[cur]);
@@ -1040,16 +1030,16 @@ void lomuto_sort(exh_ctx* c, K* keys, int* vals, long long n, double floor) {
     EXH_LAUNCH_CHECK();
     exclusive_scan<long long>(c, tle, tpre, b.ntiles);
     hipLaunchKernelGGL(k_tile_scatter<K>, dim3(nt), dim3(256), 0, c->stream, ks, vs, kd, vd,
-                       keys, vals, b, tpre, arot, s0);
+                       perm, b, tpre, arot, s0);
     EXH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_tile_chase<K>, dim3(nt), dim3(256), 0, c->stream, ks, vs, kd, vd, keys,
-                       vals, b, arot, s0, jmp, chase_cap());
+    hipLaunchKernelGGL(k_tile_chase<K>, dim3(nt), dim3(256), 0, c->stream, ks, vs, kd, vd, perm,
+                       b, arot, s0, jmp, chase_cap());
     EXH_LAUNCH_CHECK();
     // long chains (segments the chase flagged; the others return at once):
     // asynchronous pointer jumping, then the walk to the slots, before the
     // level's one host read
-    hipLaunchKernelGGL(k_double_walk<K>, dim3(nt), dim3(256), 0, c->stream, ks, vs, kd, vd, keys,
-                       vals, b, jmp, s0, 64);
+    hipLaunchKernelGGL(k_double_walk<K>, dim3(nt), dim3(256), 0, c->stream, ks, vs, kd, vd, perm,
+                       b, jmp, s0, 64);
     EXH_LAUNCH_CHECK();
     EXH_CHECK_HIP(hipMemcpyAsync(hs, st, sizeof(LevelState), hipMemcpyDeviceToHost, c->stream));
     EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
@@ -1068,7 +1058,7 @@ void lomuto_sort(exh_ctx* c, K* keys, int* vals, long long n, double floor) {
                            round_open, k);
       EXH_LAUNCH_CHECK();
       hipLaunchKernelGGL(k_tile_chase2<K>, dim3(nt), dim3(256), 0, c->stream, ks, vs, kd, vd,
-                         keys, vals, b, jmp, s0, 1);
+                         perm, b, jmp, s0, 1);
       EXH_LAUNCH_CHECK();
     }
     const int nseg_next = (int)(hs->pk >> 32);
@@ -1090,7 +1080,7 @@ void lomuto_sort(exh_ctx* c, K* keys, int* vals, long long n, double floor) {
   }
 }
 
-template void lomuto_sort<float>(exh_ctx*, float*, int*, long long, double);
-template void lomuto_sort<double>(exh_ctx*, double*, int*, long long, double);
+template void lomuto_sort<float>(exh_ctx*, const float*, int*, long long, double);
+template void lomuto_sort<double>(exh_ctx*, const double*, int*, long long, double);
 
 }  // namespace exh

@@ -34,6 +34,9 @@ def _field(bbks, nd, Lc, prec, bumps):
     (64, 4.0, (1.0, 0.0, 0.0), 1, [((0, 0, 0), 8.0, 2.6)]),
     # the same shrunk back below an ellipsoidal barrier, small halos rejected
     (64, 2.0, (0.8, 0.4, 0.6), 8, [((63, 1, 30), 9.0, 5.0), ((20, 40, 12), 6.0, 4.0)]),
+    # a high barrier of few cells: most growths shrink to no cell, and their
+    # centres must not keep later candidates waiting
+    (48, 2.75, (1.2, 0.6, 0.6), 1, [((10, 47, 5), 9.0, 3.5)]),
     # no row in use: isolated cells only
     (32, 4.0, (1.0, 0.0, 0.0), 1, None),
     # more than 131072 candidates: 256 of them a workgroup

@@ -26,6 +26,7 @@
 #include <array>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
 
 namespace exh {
@@ -2064,51 +2065,133 @@ __global__ void k_shell_fill(const typename cplx<T>::type* gk, const short* shel
   }
 }
 
-// Sums over the cells of products of two or three shell fields, one double
-// per product ("term": fields fa, fb and fc, fc < 0 for a pair).  A block
-// stages BS_CH cells of every field in LDS, then each thread runs its
-// terms over those cells (all lanes read the same cell: LDS broadcast).
-static constexpr int BS_TPT = 4;  // terms per thread
+// Sums over the cells of products of two or three shell fields, as a matrix
+// product on the FP64 matrix cores: row r of the left factor holds the
+// products A_r B_r of two fields, a column of the right factor a third field,
+// and the sum over the cells is the contraction.  A job is one 16 x 16 tile
+// of (rows, columns); the columns a row needs are a range, so only the tiles
+// that hold a wanted triple are listed.  The pair sums are the sums of a row
+// (a job with y set adds up its rows).
+//
+// A workgroup stages `ch` cells of every field in LDS; each wave runs its
+// jobs over them, four cells a lane (one 16-byte LDS read per operand) and
+// four v_mfma_f64_16x16x4 per job and 16 cells.  Lane l holds row (and
+// column) l % 16 and cells 4 (l / 16) .. + 3; the result's row 4 v + l / 16,
+// column l % 16 stands in accumulator v.  The products of two fields are
+// exact to double's rounding, the third factor enters by a fused
+// multiply-add.  What bounds it is the matrix cores' rate (128 flop per clock
+// and CU; 0.31 ms of it) and the conversions and products beside: 20 shells
+// of a 128^3 grid take 0.64 ms, and took 7.29 ms with one thread per product
+// reading all its factors from LDS.
+static constexpr int BS_JPW = 8;  // jobs per wave
+typedef double bs_d4 __attribute__((ext_vector_type(4)));
 
 template <typename T>
+struct BsVec;
+template <>
+struct BsVec<float> {
+  static constexpr int PAD = 4;
+  using V = float4;
+  static constexpr int W = 4;  // values per 16 bytes
+};
+template <>
+struct BsVec<double> {
+  static constexpr int PAD = 2;
+  using V = double2;
+  static constexpr int W = 2;
+};
+
+__device__ __forceinline__ void bs_read(const float* p, double (&v)[4]) {
+  const float4 x = *reinterpret_cast<const float4*>(p);
+  v[0] = x.x;
+  v[1] = x.y;
+  v[2] = x.z;
+  v[3] = x.w;
+}
+__device__ __forceinline__ void bs_read(const double* p, double (&v)[4]) {
+  const double2 x = reinterpret_cast<const double2*>(p)[0];
+  const double2 y = reinterpret_cast<const double2*>(p)[1];
+  v[0] = x.x;
+  v[1] = x.y;
+  v[2] = y.x;
+  v[3] = y.y;
+}
+
+// rows: the two fields of each row, cols: each column's field, jobs: first
+// row, first column, row sums wanted.  `split` waves share a job (few jobs).
+template <typename T>
 __global__ __launch_bounds__(256) void k_shell_products(const T* fields, int nfield, size_t ng,
-                                                        int ch, const int4* terms, int nterm,
-                                                        double* sums) {
+                                                        int chs, const short2* rows,
+                                                        const short* cols, const int4* jobs,
+                                                        int njob, int per_wave, int split,
+                                                        double* out, double* rowsum) {
   extern __shared__ __align__(16) unsigned char bs_raw[];
-  T* lf = (T*)bs_raw;  // [nfield][ch]
-  int4 tm[BS_TPT];
-  double acc[BS_TPT];
-  for (int q = 0; q < BS_TPT; q++) {
-    const int t = blockIdx.y * 256 * BS_TPT + q * 256 + threadIdx.x;
-    tm[q] = t < nterm ? terms[t] : make_int4(-1, 0, 0, 0);
-    acc[q] = 0.0;
-  }
-  const size_t nch = (ng + ch - 1) / ch;
-  for (size_t chunk = blockIdx.x; chunk < nch; chunk += gridDim.x) {
-    const size_t x0 = chunk * ch;
-    const int nx = (int)min((size_t)ch, ng - x0);
-    __syncthreads();
-    for (int f = 0; f < nfield; f++)
-      for (int c = threadIdx.x; c < ch; c += 256)
-        lf[f * ch + c] = c < nx ? fields[(size_t)f * ng + x0 + c] : (T)0;
-    __syncthreads();
+  T* lf = (T*)bs_raw;  // [nfield][ch + PAD]
+  using V = typename BsVec<T>::V;
+  constexpr int W = BsVec<T>::W;
+  const int ch = 1 << chs, pitch = ch + BsVec<T>::PAD;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, kk = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j0 = ((int)blockIdx.y * 4 + w) / split * per_wave;
+  const int nj = max(0, min(per_wave, njob - j0)), phase = w % split;
+  int oa[BS_JPW], ob[BS_JPW], oc[BS_JPW];
+  bool rsum[BS_JPW];
+  bs_d4 acc[BS_JPW];
+  double rs[BS_JPW];
 #pragma unroll
-    for (int q = 0; q < BS_TPT; q++) {
-      if (tm[q].x < 0) continue;
-      const T* A = lf + tm[q].x * ch;
-      const T* B = lf + tm[q].y * ch;
-      double s = 0.0;
-      if (tm[q].z >= 0) {
-        const T* Cf = lf + tm[q].z * ch;
-        for (int c = 0; c < nx; c++) s += (double)A[c] * (double)B[c] * (double)Cf[c];
-      } else {
-        for (int c = 0; c < nx; c++) s += (double)A[c] * (double)B[c];
+  for (int q = 0; q < BS_JPW; q++) {
+    const int4 job = jobs[q < nj ? j0 + q : 0];
+    const short2 r = rows[job.x + l16];
+    oa[q] = r.x * pitch + 4 * kk;
+    ob[q] = r.y * pitch + 4 * kk;
+    oc[q] = cols[job.y + l16] * pitch + 4 * kk;
+    rsum[q] = job.z != 0;
+    acc[q] = bs_d4{0.0, 0.0, 0.0, 0.0};
+    rs[q] = 0.0;
+  }
+  const size_t nch = (ng + ch - 1) >> chs;
+  const int vsh = chs - (W == 4 ? 2 : 1);  // log2 of the 16-byte vectors per field
+  for (size_t chunk = blockIdx.x; chunk < nch; chunk += gridDim.x) {
+    const size_t x0 = chunk << chs;
+    const int nv = (int)(min((size_t)ch, ng - x0) / W);  // ng is a multiple of 8
+    __syncthreads();
+    for (int e = threadIdx.x; e < nfield << vsh; e += 256) {
+      const int f = e >> vsh, v = e & ((1 << vsh) - 1);
+      V x = {};
+      if (v < nv) x = reinterpret_cast<const V*>(fields + (size_t)f * ng + x0)[v];
+      *reinterpret_cast<V*>(lf + f * pitch + v * W) = x;
+    }
+    __syncthreads();
+    for (int x = 16 * phase; x < ch; x += 16 * split) {
+#pragma unroll
+      for (int q = 0; q < BS_JPW; q++) {
+        if (q >= nj) break;
+        double va[4], vb[4], vc[4];
+        bs_read(lf + oa[q] + x, va);
+        bs_read(lf + ob[q] + x, vb);
+        bs_read(lf + oc[q] + x, vc);
+#pragma unroll
+        for (int e = 0; e < 4; e++) va[e] *= vb[e];
+        if (rsum[q]) rs[q] += (va[0] + va[1]) + (va[2] + va[3]);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[e], vc[e], acc[q], 0, 0, 0);
       }
-      acc[q] += s;
     }
   }
-  for (int q = 0; q < BS_TPT; q++)
-    if (tm[q].x >= 0) atomicAdd(&sums[blockIdx.y * 256 * BS_TPT + q * 256 + threadIdx.x], acc[q]);
+#pragma unroll
+  for (int q = 0; q < BS_JPW; q++) {
+    if (q >= nj) break;
+    double* o = out + (size_t)(j0 + q) * 256;
+#pragma unroll
+    for (int v = 0; v < 4; v++) atomicAdd(&o[(4 * v + kk) * 16 + l16], acc[q][v]);
+    if (rsum[q]) {
+      double t = rs[q];
+      t += __shfl_xor(t, 16, 64);
+      t += __shfl_xor(t, 32, 64);
+      if (kk == 0) atomicAdd(&rowsum[jobs[j0 + q].x + l16], t);
+    }
+  }
 }
 
 // Configuration order of bimodule.c:49-317.
@@ -2205,79 +2288,143 @@ int run_bispectrum(exh_ctx* c, const T* grid, int ntype, int nd, double L, int w
     }
   }
   // 3. the products: per configuration ntype^3 triples and the indicator's,
-  // per shell the ntype (ntype+1)/2 pairs and the indicator's square
-  const int NBs = ntype * ntype * ntype, NPs = ntype * (ntype + 1) / 2;
-  std::vector<int4> terms;
+  // per shell the ntype (ntype+1)/2 pairs and the indicator's square.  Rows:
+  // the pairs of shells (a, b) of the configurations, times ntype^2 for the
+  // tracers, then once for the indicators; columns: the tracers' shells, then
+  // the indicators'.
+  const int NBs = ntype * ntype * ntype, NPs = ntype * (ntype + 1) / 2, nt2 = ntype * ntype;
+  std::vector<int> pid((size_t)Nk * Nk, -1);
+  std::vector<std::array<int, 2>> pairs;
   for (const auto& t : tri) {
-    for (int f1 = 0; f1 < ntype; f1++)
-      for (int f2 = 0; f2 < ntype; f2++)
-        for (int f3 = 0; f3 < ntype; f3++)
-          terms.push_back(make_int4(t[0] * nf + f1, t[1] * nf + f2, t[2] * nf + f3, 0));
-    terms.push_back(make_int4(t[0] * nf + ntype, t[1] * nf + ntype, t[2] * nf + ntype, 0));
+    int& id = pid[(size_t)t[0] * Nk + t[1]];
+    if (id < 0) {
+      id = (int)pairs.size();
+      pairs.push_back({t[0], t[1]});
+    }
   }
-  const size_t tri_terms = terms.size();
+  auto up16 = [](int n) { return (n + 15) & ~15; };
+  const int np = (int)pairs.size();
+  const int irow = up16(np * nt2), nrow = irow + up16(np);
+  const int icol = up16(Nk * ntype), ncol = icol + up16(Nk);
+  std::vector<short2> rows(nrow, make_short2(0, 0));
+  std::vector<short> cols(ncol, 0);
+  for (int p = 0; p < np; p++) {
+    for (int f = 0; f < nt2; f++)
+      rows[p * nt2 + f] = make_short2((short)(pairs[p][0] * nf + f / ntype),
+                                      (short)(pairs[p][1] * nf + f % ntype));
+    rows[irow + p] =
+        make_short2((short)(pairs[p][0] * nf + ntype), (short)(pairs[p][1] * nf + ntype));
+  }
   for (int s = 0; s < Nk; s++) {
-    for (int f1 = 0; f1 < ntype; f1++)
-      for (int f2 = 0; f2 <= f1; f2++) terms.push_back(make_int4(s * nf + f1, s * nf + f2, -1, 0));
-    terms.push_back(make_int4(s * nf + ntype, s * nf + ntype, -1, 0));
+    for (int f = 0; f < ntype; f++) cols[f * Nk + s] = (short)(s * nf + f);
+    cols[icol + s] = (short)(s * nf + ntype);
   }
-  const int nterm = (int)terms.size();
+  // the tiles that hold a wanted triple
+  const int ntr = nrow / 16, ntc = ncol / 16;
+  std::vector<int> tile((size_t)ntr * ntc, -1);
+  auto want = [&](int r, int c) { tile[(size_t)(r / 16) * ntc + c / 16] = 0; };
+  for (const auto& t : tri) {
+    const int p = pid[(size_t)t[0] * Nk + t[1]];
+    for (int f = 0; f < nt2; f++)
+      for (int f3 = 0; f3 < ntype; f3++) want(p * nt2 + f, f3 * Nk + t[2]);
+    want(irow + p, icol + t[2]);
+  }
+  std::vector<int4> jobs;
+  for (int r = 0; r < ntr; r++) {
+    bool first = true;
+    for (int q = 0; q < ntc; q++) {
+      int& id = tile[(size_t)r * ntc + q];
+      if (id < 0) continue;
+      id = (int)jobs.size();
+      jobs.push_back(make_int4(r * 16, q * 16, first ? 1 : 0, 0));
+      first = false;
+    }
+  }
+  const int njob = (int)jobs.size();
   size_t toff = 0;
   auto ttake = [&](size_t b) {
     size_t r = toff;
     toff += (b + 255) & ~(size_t)255;
     return r;
   };
-  const size_t o_terms = ttake((size_t)nterm * sizeof(int4)), o_sums = ttake((size_t)nterm * 8);
+  // one upload: jobs, rows, columns; then the sums
+  const size_t o_jobs = ttake((size_t)njob * sizeof(int4)),
+               o_rows = ttake((size_t)nrow * sizeof(short2)),
+               o_cols = ttake((size_t)ncol * sizeof(short)), up_bytes = toff,
+               o_out = ttake(((size_t)njob * 256 + nrow) * 8);
+  std::vector<char> up(up_bytes);
+  std::memcpy(up.data() + o_jobs, jobs.data(), (size_t)njob * sizeof(int4));
+  std::memcpy(up.data() + o_rows, rows.data(), (size_t)nrow * sizeof(short2));
+  std::memcpy(up.data() + o_cols, cols.data(), (size_t)ncol * sizeof(short));
   char* tb = (char*)ctx_buf(c, BUF_PART, toff);
-  int4* dterms = (int4*)(tb + o_terms);
-  double* dsums = (double*)(tb + o_sums);
-  EXH_CHECK_HIP(hipMemcpyAsync(dterms, terms.data(), (size_t)nterm * sizeof(int4),
-                               hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_zero<double>, dim3(grid_for(nterm, 256)), dim3(256), 0, c->stream, dsums,
-                     (size_t)nterm);
+  double* dout = (double*)(tb + o_out);
+  double* drow = dout + (size_t)njob * 256;
+  const size_t nout = (size_t)njob * 256 + nrow;
+  EXH_CHECK_HIP(hipMemcpyAsync(tb, up.data(), up_bytes, hipMemcpyHostToDevice, c->stream));
+  hipLaunchKernelGGL(k_zero<double>, dim3(grid_for(nout, 256)), dim3(256), 0, c->stream, dout,
+                     nout);
   const int nfield = Nk * nf;
-  int ch = 256;
-  while (ch > 16 && (size_t)nfield * ch * sizeof(T) > 96 * 1024) ch >>= 1;
-  EXH_REQUIRE((size_t)nfield * ch * sizeof(T) <= 96 * 1024, EXH_ERR_UNSUPPORTED,
+  // cells per chunk: the most that let two workgroups share a CU's LDS, at
+  // least 16
+  int chs = 8;
+  auto lds_of = [&](int sh) {
+    return (size_t)nfield * ((1 << sh) + BsVec<T>::PAD) * sizeof(T);
+  };
+  while (chs > 4 && lds_of(chs) > 72 * 1024) chs--;
+  EXH_REQUIRE((size_t)nfield * 16 * sizeof(T) <= 96 * 1024, EXH_ERR_UNSUPPORTED,
               "bispectrum: %d shell fields exceed the LDS staging", nfield);
   {
     TimedScope ts(c, "bispec_products");
     const T* fields = (const T*)c->buf[BUF_SHELLS];
-    const int lds = nfield * ch * (int)sizeof(T);
+    const int lds = (int)lds_of(chs);
     EXH_CHECK_HIP(hipFuncSetAttribute((const void*)k_shell_products<T>,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    const unsigned ty = (unsigned)((nterm + 256 * BS_TPT - 1) / (256 * BS_TPT));
-    const size_t nch = (ng + ch - 1) / ch;
-    const unsigned tx = (unsigned)std::max<size_t>(1, std::min<size_t>(nch, 2048 / ty + 1));
+    const int ty = (njob + 4 * BS_JPW - 1) / (4 * BS_JPW);
+    const int split = njob <= 1 ? 4 : (njob == 2 ? 2 : 1);
+    const int per_wave = split > 1 ? 1 : (njob + 4 * ty - 1) / (4 * ty);
+    const size_t nch = (ng + (1 << chs) - 1) >> chs;
+    // three workgroups a CU, all resident (two: 0.68 ms; 513 workgroups, one
+    // more than two a CU: 0.87 ms)
+    const unsigned tx = (unsigned)std::max<size_t>(1, std::min<size_t>(nch, 768 / ty));
     hipLaunchKernelGGL(k_shell_products<T>, dim3(tx, ty), dim3(256), lds, c->stream, fields,
-                       nfield, ng, ch, dterms, nterm, dsums);
+                       nfield, ng, chs, (const short2*)(tb + o_rows), (const short*)(tb + o_cols),
+                       (const int4*)(tb + o_jobs), njob, per_wave, split, dout, drow);
     EXH_LAUNCH_CHECK();
   }
-  std::vector<double> hs(nterm), hks(Nk);
+  std::vector<double> hs(nout), hks(Nk);
   std::vector<unsigned long long> hkc(Nk);
-  EXH_CHECK_HIP(hipMemcpyAsync(hs.data(), dsums, (size_t)nterm * 8, hipMemcpyDeviceToHost,
-                               c->stream));
+  EXH_CHECK_HIP(hipMemcpyAsync(hs.data(), dout, nout * 8, hipMemcpyDeviceToHost, c->stream));
   EXH_CHECK_HIP(hipMemcpyAsync(hks.data(), ksum, (size_t)Nk * 8, hipMemcpyDeviceToHost,
                                c->stream));
   EXH_CHECK_HIP(hipMemcpyAsync(hkc.data(), kcnt, (size_t)Nk * 8, hipMemcpyDeviceToHost,
                                c->stream));
   EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
+  const double* hrow = hs.data() + (size_t)njob * 256;
+  auto triple = [&](int r, int q) {
+    return hs[(size_t)tile[(size_t)(r / 16) * ntc + q / 16] * 256 + (r % 16) * 16 + q % 16];
+  };
   // 4. normalisation (bimodule.c:356-370) and outputs in T (spectrum.c:368-383)
   std::vector<double> km(Nk);
   for (int s = 0; s < Nk; s++) km[s] = (double)(T)(hkc[s] ? hks[s] / (double)hkc[s] : NAN);
   const double L15 = std::pow((double)Lr, 1.5);
   for (long long n = 0; n < ntri; n++) {
-    const double* v = hs.data() + (size_t)n * (NBs + 1);
-    const double IB = v[NBs];
-    for (int j = 0; j < NBs; j++) Bk[(size_t)j * ntri + n] = (double)(T)(v[j] / IB * L15);
+    const auto& t = tri[n];
+    const int p = pid[(size_t)t[0] * Nk + t[1]];
+    const double IB = triple(irow + p, icol + t[2]);
+    for (int j = 0; j < NBs; j++) {
+      const double v = triple(p * nt2 + j / ntype, (j % ntype) * Nk + t[2]);
+      Bk[(size_t)j * ntri + n] = (double)(T)(v / IB * L15);
+    }
     Ntri_out[n] = (double)(T)(IB / (double)ng);
-    for (int q = 0; q < 3; q++) kB[(size_t)q * ntri + n] = km[tri[n][q]];
+    for (int q = 0; q < 3; q++) kB[(size_t)q * ntri + n] = km[t[q]];
   }
   for (int s = 0; s < Nk; s++) {
-    const double* v = hs.data() + tri_terms + (size_t)s * (NPs + 1);
-    const double IP = v[NPs];
-    for (int j = 0; j < NPs; j++) Pk[(size_t)j * Nk + s] = (double)(T)(v[j] / IP);
+    const int p = pid[(size_t)s * Nk + s];
+    const double IP = hrow[irow + p];
+    int j = 0;
+    for (int f1 = 0; f1 < ntype; f1++)
+      for (int f2 = 0; f2 <= f1; f2++, j++)
+        Pk[(size_t)j * Nk + s] = (double)(T)(hrow[p * nt2 + f1 * ntype + f2] / IP);
     Nk_out[s] = (double)(T)(IP / (double)ng);
     kP[s] = km[s];
   }

@@ -37,12 +37,17 @@ namespace exh {
 // Periodic wrap into [0, L).  Values within one box length of the range
 // take the reference's subtract/add loop (spectrum_h.c:18-28); farther
 // values are reduced with floor first, so that the loop is bounded (the
-// reference's loop does not terminate for huge or infinite values).
+// reference's loop does not terminate for huge or infinite values).  Where L
+// is below the rounding of x / L * L (|x| beyond 1e7 boxes in float), the
+// difference may lie anywhere and says nothing of the position: 0 is taken.
 // Non-finite input returns -1, which the callers skip.
 template <typename T>
 __device__ inline T wrap_while(T x, T L) {
   if (!isfinite(x)) return (T)-1;
-  if (x >= (T)2 * L || x < -L) x = x - floor(x / L) * L;
+  if (x >= (T)2 * L || x < -L) {
+    const T r = x - floor(x / L) * L;
+    x = r >= -L && r < (T)2 * L ? r : (T)0;
+  }
   while (x >= L) x -= L;
   while (x < (T)0) x += L;
   return x;

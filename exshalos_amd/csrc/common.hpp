@@ -79,6 +79,9 @@ enum Slot {
   BUF_HALOTAB,  // halo finder tables (barrier, mass function, spheres, taus)
   BUF_PTAB,     // power spectrum phase and window tables
   BUF_GCNT,     // tracer counts of the grid deposit
+  BUF_BINS,     // binned deposit: counts, offsets, places
+  BUF_BIN_SCAN, // binned deposit: scan partials (may run beside the halo finder's scans)
+  BUF_BIN_ENT,  // binned deposit: entries and the parts' sums
   BUF_SHELLS,   // bispectrum: real fields of every k shell and tracer
   BUF_SHELLK,   // bispectrum: combined modes, shell index per mode, shell work grids
   BUF_EFF,      // halo growth: delta with flagged cells set to -Mtot

@@ -82,7 +82,7 @@ static void scan_rec(exh_ctx* c, const T* in, T* out, long long n, T* scratch) {
 }
 
 template <typename T>
-void exclusive_scan(exh_ctx* c, const T* in, T* out, long long n) {
+void exclusive_scan(exh_ctx* c, const T* in, T* out, long long n, Slot slot) {
   if (n <= 0) {
     hipLaunchKernelGGL(k_scan_apply<T>, dim3(1), dim3(256), 0, c->stream, in, 0LL,
                        (const T*)nullptr, out);
@@ -97,11 +97,11 @@ void exclusive_scan(exh_ctx* c, const T* in, T* out, long long n) {
   // scratch: geometric series of levels, < 3 * n / SCAN_TILE + 64 entries
   long long need = 64;
   for (long long m = n; m > 1; m = (m + SCAN_TILE - 1) / SCAN_TILE) need += 2 * ((m + SCAN_TILE - 1) / SCAN_TILE) + 2;
-  T* scratch = (T*)ctx_buf(c, BUF_SCAN, (size_t)need * sizeof(T));
+  T* scratch = (T*)ctx_buf(c, slot, (size_t)need * sizeof(T));
   scan_rec<T>(c, in, out, n, scratch);
 }
 
-template void exclusive_scan<int>(exh_ctx*, const int*, int*, long long);
-template void exclusive_scan<long long>(exh_ctx*, const long long*, long long*, long long);
+template void exclusive_scan<int>(exh_ctx*, const int*, int*, long long, Slot);
+template void exclusive_scan<long long>(exh_ctx*, const long long*, long long*, long long, Slot);
 
 }  // namespace exh

@@ -6,9 +6,11 @@
 namespace exh {
 
 // out[0..n] = exclusive prefix sums of in[0..n-1]; out[n] = total.
-// `in` and `out` may not alias.  Uses BUF_SCAN scratch (or `scratch`).
+// `in` and `out` may not alias.  The partial sums of long inputs
+// go to buffer `slot`: scans that may run at once on two streams of a context
+// take two slots.
 template <typename T>
-void exclusive_scan(exh_ctx* c, const T* in, T* out, long long n);
+void exclusive_scan(exh_ctx* c, const T* in, T* out, long long n, Slot slot = BUF_SCAN);
 
 // Exclusive prefix of `v` over the 256 threads of a block; returns this
 // thread's prefix and writes the block total to *total.  `sh` must hold

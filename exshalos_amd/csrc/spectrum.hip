@@ -517,35 +517,74 @@ static constexpr int WIN_HALO = 4;  // default margin h
 // 32-bit fixed point with 22 fraction bits (ds_add_u32; integer sums are
 // exact, so the window does not depend on the order of the adds).  Fixed
 // point serves unweighted deposits only, whose weights lie in [0, 1]: a
-// cell holds 1023 particles' weight before the sum would wrap.  Every add
-// checks the value it replaced, so the add that wraps is seen; its tile
-// then deposits straight to the grid instead of through the window.
+// cell holds 1023 particles' weight before the sum would wrap.  The adds
+// return nothing; what a thread added is summed beside them, and the window's
+// own total is compared with it.  Where they differ a cell wrapped, and the
+// window is filled again with adds that return the old value: one that wraps
+// carries 1024, exactly, to the grid's cell.
 template <typename ACC>
 struct WinAcc {
+  static constexpr float SCALE = 1.f;
   template <typename T>
-  __device__ static ACC to(T v) {
-    return (ACC)v;
+  __device__ static ACC to(T a, T w) {
+    return (ACC)(a * w);
   }
-  __device__ static double from(ACC a) { return (double)a; }
-  // add v to *p; true if the sum wrapped
-  __device__ static bool add(ACC* p, ACC v) {
-    atomicAdd(p, v);
-    return false;
+  template <typename T>
+  __device__ static T from(ACC a) {
+    return (T)a;
   }
 };
 template <>
 struct WinAcc<unsigned> {
+  static constexpr float SCALE = 4194304.f;  // of the weights passed to `to`
+  // a w, to the nearest
   template <typename T>
-  __device__ static unsigned to(T v) {
-    return (unsigned)((float)v * 4194304.0f + 0.5f);
+  __device__ static unsigned to(T a, T w) {
+    return (unsigned)fmaf((float)a, (float)w, 0.5f);
   }
-  __device__ static double from(unsigned a) { return (double)a * (1.0 / 4194304.0); }
-  __device__ static bool add(unsigned* p, unsigned v) {
-    const unsigned old = atomicAdd(p, v);
-    return old + v < old;
+  template <typename T>
+  __device__ static T from(unsigned a) {
+    return (T)a * (T)(1.0 / 4194304.0);
   }
 };
 
+// First cell (possibly -1) and weights of the window along one axis: the
+// values of stencil_q, in cell order.  CIC and TSC scale by the reciprocal of
+// the cell size (their weights are continuous in the position, so the
+// rounding of x / Ld against x * (1 / Ld) moves them by an ulp); NGP divides
+// as the reference does.
+template <typename T, int WIN>
+__device__ __forceinline__ int axis_window(T x, T Ld, T inv, double invd, int nd, T* w) {
+  if constexpr (WIN == 1) {
+    const int xt = (int)floor(x / Ld);
+    w[0] = (T)1;
+    return xt == nd ? xt - 1 : xt;
+  } else if constexpr (WIN == 2) {
+    const T q = x * inv;
+    int xt = (int)floor(q);
+    if (xt == nd) xt -= 1;
+    const T dx = q - ((T)xt + (T)0.5);
+    const T far = dx >= (T)0 ? dx : -dx, near = (T)1 - far;
+    w[0] = dx >= (T)0 ? near : far;
+    w[1] = dx >= (T)0 ? far : near;
+    return dx >= (T)0 ? xt : xt - 1;
+  } else {
+    const double u = (double)x * invd - 0.5;
+    const double cf = floor(u + 0.5);
+    const double d = u - cf;
+    w[0] = (T)(0.5 * (0.5 - d) * (0.5 - d));
+    w[1] = (T)(0.75 - d * d);
+    w[2] = (T)(0.5 * (0.5 + d) * (0.5 + d));
+    return (int)cf - 1;
+  }
+}
+
+// Bound by vector instructions (204 a particle and sub-grid for TSC) and LDS
+// adds (6 cycles each with conflicts), with the flush's atomics close behind.
+// One cell and one range test per axis, the fixed-point scale folded into the
+// weights, adds without return values, the double division of TSC as a
+// product, and 64 registers in place of more than 64 (two workgroups per CU
+// instead of one): 775 -> 637 us for 256^3 particles, TSC, interlaced, FP32.
 template <typename T, int WIN, typename ACC, int PX, int PY, int PZ>
 __device__ __forceinline__ void deposit_window_tile(
     int tile, const T* pos, const T* vel, const T* mass, int nL, int nd, int Wx, int Wy, int Wz,
@@ -558,6 +597,7 @@ __device__ __forceinline__ void deposit_window_tile(
   ACC* box = (ACC*)lds_raw;
   __shared__ float samp[3][NWAVE];
   __shared__ int wo_s[3];
+  __shared__ long long diff_s[NWAVE];
   __shared__ unsigned long long nvalid;
   const size_t ng = (size_t)nd * nd * nd;
   const T Ld = L / (T)nd;
@@ -568,33 +608,37 @@ __device__ __forceinline__ void deposit_window_tile(
   // tile centre in grid cells: the middle of the grid tile of the same index
   const int qc[3] = {tx * Wx + Wx / 2, ty * Wy + Wy / 2, tz * Wz + Wz / 2};
   if (threadIdx.x == 0) nvalid = 0;
-  T xs[PPT][3];
-  T ms[PPT];
-  bool ok[PPT];
-  unsigned long long myvalid = 0;
-#pragma unroll
-  for (int p = 0; p < PPT; p++) {
+  // particle p of this thread, after the redshift-space shift.  Positions are
+  // read again for every filling (48 KB a tile, from the L2): kept in registers
+  // they cost the second workgroup of a CU.
+  auto load = [&](int p, T* x, T& m) {
     const int lin = threadIdx.x + p * WIN_THREADS;
     const int c = lin % PZ, b = (lin / PZ) % PY, a = lin / (PZ * PY);
     const size_t j = ((size_t)(tx * PX + a) * nL + (ty * PY + b)) * nL + (tz * PZ + c);
-    T x[3] = {pos[3 * j], pos[3 * j + 1], pos[3 * j + 2]};
-    if (direction >= 0) x[direction] = wrap_while<T>(x[direction] + vel[3 * j + direction] * rsd, L);
-    ok[p] = isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]);
 #pragma unroll
-    for (int q = 0; q < 3; q++) xs[p][q] = x[q];
-    ms[p] = mass ? mass[j] : (T)1;
-    myvalid += ok[p];
-  }
+    for (int q = 0; q < 3; q++) x[q] = pos[3 * j + q];
+    if (direction >= 0) {
+      const T v = vel[3 * j + direction] * rsd;
+#pragma unroll
+      for (int q = 0; q < 3; q++)
+        if (q == direction) x[q] = wrap_while<T>(x[q] + v, L);
+    }
+    m = mass ? mass[j] : (T)1;
+  };
+  auto valid = [](const T* x) { return isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]); };
+  unsigned myvalid = 0;
   // displacement (in cells) of each wave's first particle: its cell relative
   // to the tile centre minus its lattice point's offset from the centre
   if ((threadIdx.x & 63) == 0) {
     const int lin = threadIdx.x;
     const int lat[3] = {lin / (PZ * PY), (lin / PZ) % PY, lin % PZ};
+    T x[3], m;
+    load(0, x, m);
 #pragma unroll
     for (int q = 0; q < 3; q++) {
       float r = 1e30f;
-      if (ok[0]) {
-        int cc = (int)floor(wrap_while<T>(xs[0][q], L) / Ld);
+      if (valid(x)) {
+        int cc = (int)floor(wrap_while<T>(x[q], L) / Ld);
         cc = cc < nd ? cc : nd - 1;
         r = (float)rel_cell(cc, qc[q], nd) -
             ((lat[q] + 0.5f) * (float)nd / (float)nL - 0.5f * (float)W[q]);
@@ -618,107 +662,107 @@ __device__ __forceinline__ void deposit_window_tile(
   }
   __syncthreads();
   const int wo[3] = {wo_s[0], wo_s[1], wo_s[2]};
-  const int E[3] = {Ex, Ey, Ez};
   const int vol = Ex * sx;
   const T shift = (T)(-(double)Lb / 2.0);
-  // CIC scales by the reciprocal of the cell size (its weights are
-  // continuous in the position, so the rounding of x / Ld against x * (1 /
-  // Ld) moves them by an ulp); NGP and TSC divide as the reference does
   const T invLd = (T)1 / Ld;
+  const double invd = 1.0 / (double)Ld;
+  // the window's first cell, in [0, nd)
+  int org[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    org[q] = (qc[q] + wo[q]) % nd;
+    org[q] += org[q] < 0 ? nd : 0;
+  }
+  constexpr bool FIXED = std::is_same<ACC, unsigned>::value;
   for (int s = 0; s < nsub; s++) {
     T* g = grid + (size_t)s * ng;
-    for (int v = threadIdx.x; v < vol; v += WIN_THREADS) box[v] = (ACC)0;
-    __syncthreads();
-    bool wrapped = false;
-#pragma unroll
-    for (int p = 0; p < PPT; p++) {
-      if (!ok[p]) continue;
-      int cell[3][3], off[3][3];
-      T w[3][3];
-      bool in = true;
-#pragma unroll
-      for (int q = 0; q < 3; q++) {
-        const T pa = wrap_while<T>(s == 0 ? xs[p][q] : xs[p][q] + shift, L);
-        if constexpr (WIN == 2)
-          stencil_q<T, WIN>(pa * invLd, nd, cell[q], w[q]);
-        else
-          stencil_q<T, WIN>(scale_q<T, WIN>(pa, Ld), nd, cell[q], w[q]);
-        const int st = q == 0 ? sx : (q == 1 ? Ez : 1);
-#pragma unroll
-        for (int u = 0; u < NW; u++) {
-          const int l = rel_cell(cell[q][u], qc[q], nd) - wo[q];
-          in = in && (unsigned)l < (unsigned)E[q];
-          off[q][u] = l * st;
-        }
-      }
-      if (in) {
-#pragma unroll
-        for (int u = 0; u < NW; u++) {
-#pragma unroll
-          for (int b = 0; b < NW; b++) {
-            const T wab = ms[p] * w[0][u] * w[1][b];
-            const int o = off[0][u] + off[1][b];
-#pragma unroll
-            for (int c = 0; c < NW; c++)
-              wrapped |= WinAcc<ACC>::add(&box[o + off[2][c]], WinAcc<ACC>::to(wab * w[2][c]));
-          }
-        }
-      } else {
-        for (int u = 0; u < NW; u++)
-          for (int b = 0; b < NW; b++) {
-            const T wab = ms[p] * w[0][u] * w[1][b];
-            for (int c = 0; c < NW; c++)
-              atomic_add_t(g + ((size_t)cell[0][u] * nd + cell[1][b]) * nd + cell[2][c],
-                           wab * w[2][c]);
-          }
-      }
-    }
-    if (__syncthreads_or(wrapped)) {
-      // a fixed-point window cell wrapped: the window is void; every
-      // in-window stencil of the tile goes to the grid directly instead
-      // (the out-of-window ones already did)
-#pragma unroll
+    unsigned added = 0;  // fixed point: this thread's sum, < 5 * 2^22 * PPT
+    // the tile's particles into the window; `again`: the second filling, which
+    // carries and leaves out what lies outside
+    auto fill = [&](auto again) {
+      for (int v = threadIdx.x; v < vol; v += WIN_THREADS) box[v] = (ACC)0;
+      __syncthreads();
+      T x[3], m;
+      load(0, x, m);
+#pragma unroll 1
       for (int p = 0; p < PPT; p++) {
-        if (!ok[p]) continue;
-        int cell[3][3];
-        T w[3][3];
-        bool in = true;
+        const T px[3] = {x[0], x[1], x[2]}, pm = m;
+        if (p + 1 < PPT) load(p + 1, x, m);
+        if (!valid(px)) continue;
+        if constexpr (!decltype(again)::value) myvalid += s == 0;
+        int b[3], l[3];
+        T w[3][NW];
 #pragma unroll
         for (int q = 0; q < 3; q++) {
-          const T pa = wrap_while<T>(s == 0 ? xs[p][q] : xs[p][q] + shift, L);
-          // the stencil of the window pass, so that `in` matches it
-          if constexpr (WIN == 2)
-            stencil_q<T, WIN>(pa * invLd, nd, cell[q], w[q]);
-          else
-            stencil_q<T, WIN>(scale_q<T, WIN>(pa, Ld), nd, cell[q], w[q]);
-          for (int u = 0; u < NW; u++) {
-            const int l = rel_cell(cell[q][u], qc[q], nd) - wo[q];
-            in = in && (unsigned)l < (unsigned)E[q];
-          }
+          T pa = s == 0 ? px[q] : px[q] + shift;
+          if (!(pa >= (T)0 && pa < L)) pa = wrap_while<T>(pa, L);
+          b[q] = axis_window<T, WIN>(pa, Ld, invLd, invd, nd, w[q]);
+          l[q] = b[q] - org[q];
+          l[q] += l[q] < 0 ? nd : 0;
         }
-        if (!in) continue;
-        for (int u = 0; u < NW; u++)
-          for (int b = 0; b < NW; b++) {
-            const T wab = ms[p] * w[0][u] * w[1][b];
-            for (int c = 0; c < NW; c++)
-              atomic_add_t(g + ((size_t)cell[0][u] * nd + cell[1][b]) * nd + cell[2][c],
-                           wab * w[2][c]);
+        if (l[0] + NW <= Ex && l[1] + NW <= Ey && l[2] + NW <= Ez) {
+          ACC* row = box + l[0] * sx + l[1] * Ez + l[2];
+#pragma unroll
+          for (int u = 0; u < NW; u++) {
+#pragma unroll
+            for (int v = 0; v < NW; v++) {
+              const T wab = pm * w[0][u] * w[1][v] * (T)WinAcc<ACC>::SCALE;
+              ACC* r = row + u * sx + v * Ez;
+#pragma unroll
+              for (int k = 0; k < NW; k++) {
+                const ACC val = WinAcc<ACC>::to(wab, w[2][k]);
+                if constexpr (decltype(again)::value) {
+                  const ACC old = atomicAdd(&r[k], val);
+                  if (old + val < old)
+                    atomic_add_t(g + ((size_t)wrap_cell(b[0] + u, nd) * nd +
+                                      wrap_cell(b[1] + v, nd)) * nd + wrap_cell(b[2] + k, nd),
+                                 (T)1024);
+                } else {
+                  atomicAdd(&r[k], val);
+                  if constexpr (FIXED) added += val;
+                }
+              }
+            }
           }
+        } else if constexpr (!decltype(again)::value) {
+          for (int u = 0; u < NW; u++)
+            for (int v = 0; v < NW; v++) {
+              const T wab = pm * w[0][u] * w[1][v];
+              for (int k = 0; k < NW; k++)
+                atomic_add_t(g + ((size_t)wrap_cell(b[0] + u, nd) * nd +
+                                  wrap_cell(b[1] + v, nd)) * nd + wrap_cell(b[2] + k, nd),
+                             wab * w[2][k]);
+            }
+        }
       }
-      continue;
+      __syncthreads();
+    };
+    fill(std::false_type{});
+    if constexpr (FIXED) {
+      // the window's total less what was added; a multiple of 2^32 wrapped
+      long long diff = -(long long)added;
+      for (int v = threadIdx.x; v < vol; v += WIN_THREADS) diff += box[v];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) diff += __shfl_xor(diff, o, 64);
+      if ((threadIdx.x & 63) == 0) diff_s[threadIdx.x >> 6] = diff;
+      __syncthreads();
+      long long all = 0;
+#pragma unroll
+      for (int w = 0; w < NWAVE; w++) all += diff_s[w];
+      if (all != 0) fill(std::true_type{});
     }
     // flush: (y, z) rows over the threads, z fastest in 32-lane groups
     const int lz0 = threadIdx.x & 31;
     for (int ly = threadIdx.x >> 5; ly < Ey; ly += WIN_THREADS / 32) {
-      const int cy = wrap_cell(qc[1] + wo[1] + ly, nd);
+      const int cy = wrap_cell(org[1] + ly, nd);
       for (int lz = lz0; lz < Ez; lz += 32) {
-        const int cz = wrap_cell(qc[2] + wo[2] + lz, nd);
+        const int cz = wrap_cell(org[2] + lz, nd);
         const ACC* bp = box + ly * Ez + lz;
-        int cx = wrap_cell(qc[0] + wo[0], nd);
+        int cx = org[0];
         for (int lx = 0; lx < Ex; lx++) {
           const ACC val = bp[lx * sx];
           if (val != (ACC)0)
-            atomic_add_t(g + ((size_t)cx * nd + cy) * nd + cz, (T)WinAcc<ACC>::from(val));
+            atomic_add_t(g + ((size_t)cx * nd + cy) * nd + cz, WinAcc<ACC>::template from<T>(val));
           cx = cx + 1 == nd ? 0 : cx + 1;
         }
       }
@@ -726,7 +770,7 @@ __device__ __forceinline__ void deposit_window_tile(
     __syncthreads();
   }
   if (!mass && counts) {
-    atomicAdd(&nvalid, myvalid);
+    atomicAdd(&nvalid, (unsigned long long)myvalid);
     __syncthreads();
     if (threadIdx.x == 0) atomicAdd(&counts[0], nvalid);
   }
@@ -735,7 +779,7 @@ __device__ __forceinline__ void deposit_window_tile(
 // One workgroup per tile, or (EXH_DEPOSIT_WG) fewer workgroups that walk the
 // tiles, leaving CUs to the kernels of other streams.
 template <typename T, int WIN, typename ACC, int PX, int PY, int PZ>
-__global__ __launch_bounds__(WIN_THREADS) void k_deposit_window(
+__global__ __launch_bounds__(WIN_THREADS, sizeof(ACC) == 4 ? 8 : 4) void k_deposit_window(
     const T* pos, const T* vel, const T* mass, int nL, int nd, int Wx, int Wy, int Wz, int wh,
     T L, T Lb, int direction, T rsd, int nsub, T* grid, unsigned long long* counts, int ntiles) {
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
@@ -1198,14 +1242,14 @@ void* noalloc_grid_scratch(int device) {
 // Tile shape of the window deposit (EXH_DEPOSIT_TILE: 16 = 16^3 particles,
 // the default; 3216 = 32 x 16 x 16; 32 = 32 x 32 x 16) and its
 // accumulator (EXH_DEPOSIT_ACC: 1 fixed point, the default for float grids
-// without masses; 8 double; 4 float).  At nd = nL = 512 (CIC, interlaced),
-// alone: 3.18 ms for 32 x 16 x 16 in fixed point, 3.06 ms for 32 x 32 x 16,
-// 3.63 ms for 16^3, 3.89 ms for 16^3 in double, 12.6 ms for 16^3 in float
-// (ds_add_f32 runs far slower than ds_add_u32 or ds_add_f64 here).  Beside
-// the halo finder's sort the 32 x 32 x 16 workgroups (153 KB of LDS each)
-// hold CUs long enough to slow the sort by 2.6 ms; the 16^3 workgroups
-// (55 KB, two per CU) leave it most room: the fused nd = 512 step runs
-// 26.85-26.99 ms with them against 27.21-27.27 ms with 32 x 16 x 16.
+// without masses; 8 double; 4 float).  Two 16^3 workgroups of 55 KB and 64
+// registers share a CU.  The whole call (zero, deposit, normalise) at nd = nL
+// = 512, CIC, interlaced, takes 3.28 ms with 16^3 tiles; longer ones in z,
+// which issue up to a third fewer atomics, take 3.41 (16 x 16 x 32, one
+// workgroup per CU), 3.74 (16 x 8 x 32) and 3.84 ms (8 x 8 x 64).  Float sums
+// are no choice: ds_add_f32 runs far slower than ds_add_u32 or ds_add_f64
+// here (16^3: 12.6 ms against 3.6).  Beside the halo finder's sort larger
+// workgroups hold CUs long enough to slow the sort.
 struct WinShape {
   int px, py, pz;
 };
@@ -1259,7 +1303,11 @@ static void launch_window(exh_ctx* c, unsigned nwg, int lds, const DepositWinArg
 template <typename T, int WN>
 static void launch_window_shape(exh_ctx* c, int acc, const WinShape& ws, unsigned nwg, int lds,
                                 const DepositWinArgs<T>& a) {
-  if (ws.px == 32 && ws.py == 32) {
+  if constexpr (sizeof(T) == 8) {
+    if (ws.px == 32 && ws.py == 32) launch_window<T, WN, double, 32, 32, 16>(c, nwg, lds, a);
+    else if (ws.px == 32) launch_window<T, WN, double, 32, 16, 16>(c, nwg, lds, a);
+    else launch_window<T, WN, double, 16, 16, 16>(c, nwg, lds, a);
+  } else if (ws.px == 32 && ws.py == 32) {
     if (acc == 1) launch_window<T, WN, unsigned, 32, 32, 16>(c, nwg, lds, a);
     else if (acc == 4) launch_window<T, WN, float, 32, 32, 16>(c, nwg, lds, a);
     else launch_window<T, WN, double, 32, 32, 16>(c, nwg, lds, a);

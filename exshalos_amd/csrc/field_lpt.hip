@@ -496,8 +496,12 @@ struct HaloStage {
 __device__ inline int wrapi(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
 // Gradient of a scalar field phi: MODE 1 writes S = -D phi / (60 Lc) and
-// V = f1 S (lpt.c:56-93); MODE 2 adds -3/7 Omz^(-1/143) D phi2 / (60 Lc) to
-// S and f2 times it to V (lpt.c:182-223; coef carries the prefactor).
+// V = f1 S (lpt.c:56-93); MODE 2 adds S2 = -3/7 Omz^(-1/143) D phi2 / (60 Lc)
+// to S and writes V = f1 S1 + f2 S2 (lpt.c:182-223; coef carries the
+// prefactor).  Bound by memory: before a second pass MODE 1 leaves V out, and
+// MODE 2 takes f1 S1 from the S it reads, the product that MODE 1 would have
+// rounded and stored (256^3, FP64: 206 + 359 us with V through memory, 130 +
+// 296 without).
 // Positions written by the last gradient pass: q + S wrapped into the box
 // (Compute_Pos, lpt.c:229-255): the lattice point (q + 1/2) Lc in the
 // field's precision, plus S, wrapped once.
@@ -525,7 +529,7 @@ __device__ inline T lattice_pos(int q, T Lc, T s, T L) {
 template <typename T, int MODE, bool FULL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, MODE == 2 ? 4 : 8))) void
 k_grad_tiles(TileGeom g, const T* phi, double inv60,
-                                                    double coef, T* S, T* V, T fv,
+                                                    double coef, T* S, T* V, T f1, T f2,
                                                     PosOut<T> po) {
   __shared__ T pl[ST_PJ * ST_PK];
   int i0, j0, k0;
@@ -550,21 +554,19 @@ k_grad_tiles(TileGeom g, const T* phi, double inv60,
     ps.load(phi + (size_t)i * plane, hv);
     const T* pp = phi + (size_t)wrapi(i + 3, g.n0) * plane;
     for (int q = 0; q < ST_Q; q++) win[q][6] = pp[wo[q]];
-    // the second-order pass adds to S (and V): for float fields on full
-    // tiles the plane's values of the thread's cells are loaded here, before
-    // any store of the plane (which could alias them for the compiler); the
-    // other variants keep their registers (and occupancy) and load them
-    // below
+    // the second-order pass adds to S: for float fields on full tiles the
+    // plane's values of the thread's cells are loaded here, before any store
+    // of the plane (which could alias them for the compiler); the other
+    // variants keep their registers (and occupancy) and load them below
     using V3 = typename vec3<T>::type;
     constexpr bool PRE = MODE == 2 && sizeof(T) == 4 && FULL;
-    V3 s_old[PRE ? ST_Q : 1], v_old[PRE ? ST_Q : 1];
+    V3 s_old[PRE ? ST_Q : 1];
     if (PRE)
       for (int q = 0; q < ST_Q; q++) {
         const int j = j0 + ty + 4 * q;
         if (kin && j < g.n1) {
           const size_t c = ((size_t)i * g.n1 + j) * g.n2 + k;
           s_old[q] = *reinterpret_cast<const V3*>(S + 3 * c);
-          if (V) v_old[q] = *reinterpret_cast<const V3*>(V + 3 * c);
         }
       }
     __syncthreads();  // previous plane's readers are done
@@ -590,21 +592,21 @@ k_grad_tiles(TileGeom g, const T* phi, double inv60,
           const T sx = (T)(-gx * inv60), sy = (T)(-gy * inv60), sz = (T)(-gz * inv60);
           snew = V3{sx, sy, sz};
           *Sp = snew;
-          if (Vp) *Vp = V3{fv * sx, fv * sy, fv * sz};
+          if (Vp) *Vp = V3{f1 * sx, f1 * sy, f1 * sz};
         } else {
           const T sx = (T)(coef * gx * inv60), sy = (T)(coef * gy * inv60),
                   sz = (T)(coef * gz * inv60);
           V3 o = PRE ? s_old[PRE ? q : 0] : *Sp;
+          V3 u = {f1 * o.x, f1 * o.y, f1 * o.z};
           o.x += sx;
           o.y += sy;
           o.z += sz;
           *Sp = o;
           snew = o;
           if (Vp) {
-            V3 u = PRE ? v_old[PRE ? q : 0] : *Vp;
-            u.x += fv * sx;
-            u.y += fv * sy;
-            u.z += fv * sz;
+            u.x += f2 * sx;
+            u.y += f2 * sy;
+            u.z += f2 * sz;
             *Vp = u;
           }
         }
@@ -681,16 +683,17 @@ __global__ __launch_bounds__(256) void k_source_tiles(TileGeom g, const T* S, do
   }
 }
 
-// The same source for float fields whose tiles are all full (n1 a
+// The same source for grids whose tiles are all full (n1 a
 // multiple of 16, n2 of 64): each thread keeps its own four cells of planes
 // i .. i + 3 in registers (one 12-byte load per cell and plane, made three
 // planes ahead for the x difference), writes them into the staged plane
 // from there, and loads only the plane's halo cells (516 of the 22 x 70).
 // The separate strided load of S_x at plane i + 3, whose lines were fetched
-// again when the plane was staged, goes away.
-__global__ __launch_bounds__(256) void k_source_full(TileGeom g, const float* S, double inv60,
-                                                     float* src) {
-  __shared__ float pl[3 * ST_PJ * ST_PK];  // [pj][pk][component]
+// again when the plane was staged, goes away (256^3, FP64: 260 -> 152 us).
+template <typename T>
+__global__ __launch_bounds__(256) void k_source_full(TileGeom g, const T* S, double inv60,
+                                                     T* src) {
+  __shared__ T pl[3 * ST_PJ * ST_PK];  // [pj][pk][component]
   int i0, j0, k0;
   tile_origin(g, i0, j0, k0);
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
@@ -699,15 +702,15 @@ __global__ __launch_bounds__(256) void k_source_full(TileGeom g, const float* S,
   const size_t plane = (size_t)g.n1 * g.n2 * 3;
   int co[ST_Q];  // the thread's cells within a plane of S
   for (int q = 0; q < ST_Q; q++) co[q] = ((j0 + ty + 4 * q) * g.n2 + k0 + tx) * 3;
-  using V3 = float3;
+  using V3 = typename vec3<T>::type;
   V3 cur[ST_Q][4];     // S at planes i .. i + 3, the thread's cells
-  float xo[ST_Q][3];   // S_x at planes i - 3 .. i - 1
+  T xo[ST_Q][3];   // S_x at planes i - 3 .. i - 1
   for (int d = 0; d < 3; d++) {
-    const float* pp = S + (size_t)wrapi(i0 - 3 + d, g.n0) * plane;
+    const T* pp = S + (size_t)wrapi(i0 - 3 + d, g.n0) * plane;
     for (int q = 0; q < ST_Q; q++) xo[q][d] = pp[co[q]];
   }
   for (int d = 0; d < 3; d++) {
-    const float* pp = S + (size_t)wrapi(i0 + d, g.n0) * plane;
+    const T* pp = S + (size_t)wrapi(i0 + d, g.n0) * plane;
     for (int q = 0; q < ST_Q; q++) cur[q][d] = *reinterpret_cast<const V3*>(pp + co[q]);
   }
   constexpr int DY = 3 * ST_PK, DZ = 3;
@@ -715,17 +718,17 @@ __global__ __launch_bounds__(256) void k_source_full(TileGeom g, const float* S,
   for (int i = i0; i < i1; i++) {
     // every load of the plane is in flight before the first wait: the halo
     // values (an unused slot reads the plane's first value), then plane i + 3
-    float hv[HaloStage<3>::NE];
+    T hv[HaloStage<3>::NE];
     {
       hs.load(S + (size_t)i * plane, hv);
-      const float* pp = S + (size_t)wrapi(i + 3, g.n0) * plane;
+      const T* pp = S + (size_t)wrapi(i + 3, g.n0) * plane;
       for (int q = 0; q < ST_Q; q++) cur[q][3] = *reinterpret_cast<const V3*>(pp + co[q]);
     }
     __syncthreads();  // previous plane's readers are done
     {
       hs.store(hv, pl);
       for (int q = 0; q < ST_Q; q++) {
-        float* o = pl + ((ty + 4 * q + ST_H) * ST_PK + tx + ST_H) * 3;
+        T* o = pl + ((ty + 4 * q + ST_H) * ST_PK + tx + ST_H) * 3;
         o[0] = cur[q][0].x;
         o[1] = cur[q][0].y;
         o[2] = cur[q][0].z;
@@ -734,25 +737,25 @@ __global__ __launch_bounds__(256) void k_source_full(TileGeom g, const float* S,
     __syncthreads();
     for (int q = 0; q < ST_Q; q++) {
       const int jl = ty + 4 * q, j = j0 + jl;
-      const float* x = pl + ((jl + ST_H) * ST_PK + tx + ST_H) * 3;
-      const float* y = x + 1;
-      const float* z = x + 2;
-      const float sxx = (float)(d6w(xo[q][0], xo[q][1], xo[q][2], cur[q][1].x, cur[q][2].x,
+      const T* x = pl + ((jl + ST_H) * ST_PK + tx + ST_H) * 3;
+      const T* y = x + 1;
+      const T* z = x + 2;
+      const T sxx = (T)(d6w(xo[q][0], xo[q][1], xo[q][2], cur[q][1].x, cur[q][2].x,
                                     cur[q][3].x) * inv60);
-      const float sxy =
-          (float)(d6w(x[-3 * DY], x[-2 * DY], x[-DY], x[DY], x[2 * DY], x[3 * DY]) * inv60);
-      const float sxz =
-          (float)(d6w(x[-3 * DZ], x[-2 * DZ], x[-DZ], x[DZ], x[2 * DZ], x[3 * DZ]) * inv60);
-      const float syy =
-          (float)(d6w(y[-3 * DY], y[-2 * DY], y[-DY], y[DY], y[2 * DY], y[3 * DY]) * inv60);
-      const float syz =
-          (float)(d6w(y[-3 * DZ], y[-2 * DZ], y[-DZ], y[DZ], y[2 * DZ], y[3 * DZ]) * inv60);
-      const float szz =
-          (float)(d6w(z[-3 * DZ], z[-2 * DZ], z[-DZ], z[DZ], z[2 * DZ], z[3 * DZ]) * inv60);
-      const float t3 = sxx * syy + sxx * szz + syy * szz;
+      const T sxy =
+          (T)(d6w(x[-3 * DY], x[-2 * DY], x[-DY], x[DY], x[2 * DY], x[3 * DY]) * inv60);
+      const T sxz =
+          (T)(d6w(x[-3 * DZ], x[-2 * DZ], x[-DZ], x[DZ], x[2 * DZ], x[3 * DZ]) * inv60);
+      const T syy =
+          (T)(d6w(y[-3 * DY], y[-2 * DY], y[-DY], y[DY], y[2 * DY], y[3 * DY]) * inv60);
+      const T syz =
+          (T)(d6w(y[-3 * DZ], y[-2 * DZ], y[-DZ], y[DZ], y[2 * DZ], y[3 * DZ]) * inv60);
+      const T szz =
+          (T)(d6w(z[-3 * DZ], z[-2 * DZ], z[-DZ], z[DZ], z[2 * DZ], z[3 * DZ]) * inv60);
+      const T t3 = sxx * syy + sxx * szz + syy * szz;
       const double v = (double)t3 - (double)sxy * (double)sxy - (double)sxz * (double)sxz -
                        (double)syz * (double)syz;
-      src[((size_t)i * g.n1 + j) * g.n2 + k0 + tx] = (float)v;
+      src[((size_t)i * g.n1 + j) * g.n2 + k0 + tx] = (T)v;
     }
     for (int q = 0; q < ST_Q; q++) {
       xo[q][0] = xo[q][1];
@@ -980,19 +983,21 @@ void launch_lpt(exh_ctx* c, const exh_box* b, const exh_field_src* s, double k_s
     TimedScope ts(c, "lpt1_grad");
     if (full)
       hipLaunchKernelGGL((k_grad_tiles<T, 1, true>), dim3(tblocks), dim3(256), 0, c->stream, tg,
-                         phi, inv60, 1.0, S, V, f1, do_2lpt ? none : pos);
+                         phi, inv60, 1.0, S, do_2lpt ? nullptr : V, f1, f1,
+                         do_2lpt ? none : pos);
     else
       hipLaunchKernelGGL((k_grad_tiles<T, 1, false>), dim3(tblocks), dim3(256), 0, c->stream, tg,
-                         phi, inv60, 1.0, S, V, f1, do_2lpt ? none : pos);
+                         phi, inv60, 1.0, S, do_2lpt ? nullptr : V, f1, f1,
+                         do_2lpt ? none : pos);
     EXH_LAUNCH_CHECK();
   }
   if (do_2lpt) {
     T* src = (T*)ctx_buf(c, BUF_R1, ng * sizeof(T));
     {
       TimedScope ts(c, "lpt2_source");
-      if (sizeof(T) == 4 && full)
-        hipLaunchKernelGGL(k_source_full, dim3(tblocks), dim3(256), 0, c->stream, tg,
-                           (const float*)S, inv60, (float*)src);
+      if (full)
+        hipLaunchKernelGGL(k_source_full<T>, dim3(tblocks), dim3(256), 0, c->stream, tg, S, inv60,
+                           src);
       else
         hipLaunchKernelGGL(k_source_tiles<T>, dim3(tblocks), dim3(256), 0, c->stream, tg, S,
                            inv60, src);
@@ -1007,10 +1012,10 @@ void launch_lpt(exh_ctx* c, const exh_box* b, const exh_field_src* s, double k_s
       TimedScope ts(c, "lpt2_grad");
       if (full)
         hipLaunchKernelGGL((k_grad_tiles<T, 2, true>), dim3(tblocks), dim3(256), 0, c->stream,
-                           tg, src, inv60, coef, S, V, f2, pos);
+                           tg, src, inv60, coef, S, V, f1, f2, pos);
       else
         hipLaunchKernelGGL((k_grad_tiles<T, 2, false>), dim3(tblocks), dim3(256), 0, c->stream,
-                           tg, src, inv60, coef, S, V, f2, pos);
+                           tg, src, inv60, coef, S, V, f1, f2, pos);
       EXH_LAUNCH_CHECK();
     }
   }

@@ -1738,16 +1738,178 @@ __device__ inline T window_r(const PowerArgs& a, int fi, int fj, int fk) {
   return (T)exp((double)(-kmod * R * R) / 2.0);
 }
 
-// ONE: one tracer and the monopole only (two values per mode: P, |k|), with
-// the counts fixed at compile time so the per-tracer arrays stay in
-// registers; the arithmetic is the general path's.
-template <typename T, bool ONE>
+// The waves' LDS sums and counts added in a fixed order: one partial per block.
+__device__ __forceinline__ void power_block_sums(const double* lds, int nw, int Nk, int NV,
+                                                 double* part, unsigned* pcnt) {
+  __syncthreads();
+  double* out = part + (size_t)blockIdx.x * Nk * NV;
+  unsigned* cout = pcnt + (size_t)blockIdx.x * Nk;
+  for (int q = threadIdx.x; q < Nk * NV; q += blockDim.x) {
+    double s = 0.0;
+    for (int w = 0; w < nw; w++) s += lds[(size_t)w * Nk * NV + q];
+    out[q] = s;
+  }
+  for (int q = threadIdx.x; q < Nk; q += blockDim.x) {
+    unsigned s = 0;
+    const unsigned* cbase = (const unsigned*)(lds + (size_t)nw * Nk * NV);
+    for (int w = 0; w < nw; w++) s += cbase[(size_t)w * Nk + q];
+    cout[q] = s;
+  }
+}
+
+// One tracer's combined, deconvolved mode, (f1 + f2 e^{-i theta}) / 2 over the
+// window: for the monopole of a float grid in float (the grid's precision),
+// else in double.
+template <typename T, bool FLT, bool RWIN>
+__device__ __forceinline__ void power_mode(const PowerArgs& a, int i, int j, int k,
+                                           const double2& e1d, const double2& e2d,
+                                           const double2& e3d,
+                                           const typename cplx<T>::type& f1,
+                                           const typename cplx<T>::type& f2, double& dr,
+                                           double& di) {
+  const int nd = a.nd;
+  const int fi = (2 * i < nd) ? i : i - nd, fj = (2 * j < nd) ? j : j - nd;
+  const int fk = (2 * k < nd) ? k : k - nd;
+  if constexpr (FLT) {
+    const float2 e1 = make_float2((float)e1d.x, (float)e1d.y);
+    const float2 e2 = make_float2((float)e2d.x, (float)e2d.y);
+    const float2 e3 = make_float2((float)e3d.x, (float)e3d.y);
+    const float wk = RWIN && a.rwin ? (float)(a.Normk / (double)window_r<T>(a, fi, fj, fk))
+                            : (float)a.wx[i] * (float)a.wx[j] * (float)a.wz[k] * (float)a.Normk;
+    const float pr = e1.x * e2.x - e1.y * e2.y, pi = e1.x * e2.y + e1.y * e2.x;
+    const float er = pr * e3.x - pi * e3.y, ei = pr * e3.y + pi * e3.x;
+    float re = (float)f1.x, im = (float)f1.y;
+    if (a.nsub == 2) {
+      re = (re + ((float)f2.x * er - (float)f2.y * ei)) * 0.5f;
+      im = (im + ((float)f2.x * ei + (float)f2.y * er)) * 0.5f;
+    }
+    dr = (double)(re * wk);
+    di = (double)(im * wk);
+  } else {
+    const double wk = RWIN && a.rwin ? a.Normk / (double)window_r<T>(a, fi, fj, fk)
+                             : a.wx[i] * a.wx[j] * a.wz[k] * a.Normk;
+    // e^{-i theta} = e1 e2 e3
+    const double pr = e1d.x * e2d.x - e1d.y * e2d.y, pi = e1d.x * e2d.y + e1d.y * e2d.x;
+    const double er = pr * e3d.x - pi * e3d.y, ei = pr * e3d.y + pi * e3d.x;
+    double re = (double)f1.x, im = (double)f1.y;
+    if (a.nsub == 2) {
+      re = (re + ((double)f2.x * er - (double)f2.y * ei)) / 2.0;
+      im = (im + ((double)f2.x * ei + (double)f2.y * er)) / 2.0;
+    }
+    dr = re * wk;
+    di = im * wk;
+  }
+}
+
+// One tracer, LS multipoles, a window that is a product over the axes; KB is
+// the binning's precision.  Bound by vector instructions: with a segmented
+// sum of every 64 modes and value (k_power_bins) the sums took most of them.
+// Here a lane keeps one k and steps along j, sums the modes of its current bin
+// in registers (a bin holds a few steps) and adds them to its wave's LDS sums
+// when the bin changes; a wave's sums are its own, so the order of the adds
+// does not depend on timing.  A wave takes 64 neighbouring k and `jlen` steps;
+// the nz % 64 last k share a wave `rpw` rows at a time.  512^3, FP32,
+// interlaced: monopole, binned in double, 620 -> 464 us; l_max = 4, binned in
+// float, 1158 -> 520 us.
+struct PowerLines {
+  int jlen, kfull, rem, rpw, njs, njr;
+};
+template <typename T, int LS, int KB>
+__global__ __launch_bounds__(256) void k_power_lines(PowerArgs a, PowerLines g,
+                                                     const typename cplx<T>::type* gk,
+                                                     double* part, unsigned* pcnt) {
+  extern __shared__ double lds[];
+  using C2 = typename cplx<T>::type;
+  constexpr int NV = LS + 1, U = 4;
+  constexpr bool FLT = LS == 1 && sizeof(T) == 4;
+  a.kbin = KB;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int Nk = a.Nk, nd = a.nd, nz = a.nz;
+  double* acc = lds + (size_t)wave * Nk * NV;
+  unsigned* cacc = (unsigned*)(lds + (size_t)nw * Nk * NV) + (size_t)wave * Nk;
+  for (int q = lane; q < Nk * NV; q += 64) acc[q] = 0.0;
+  for (int q = lane; q < Nk; q += 64) cacc[q] = 0;
+  __syncthreads();
+  const size_t nh = (size_t)nd * nd * nz;
+  const long long nfull = (long long)nd * g.kfull * g.njs;
+  const long long ntask = nfull + (g.rem ? (long long)nd * g.njr : 0);
+  const long long gw = (long long)blockIdx.x * nw + wave, tw = (long long)gridDim.x * nw;
+  for (long long t = gw; t < ntask; t += tw) {
+    int i, j, k, dj, jend;
+    if (t < nfull) {
+      const int r = (int)(t / g.kfull);
+      k = (int)(t - (long long)r * g.kfull) * 64 + lane;
+      i = r / g.njs;
+      j = (r - i * g.njs) * g.jlen;
+      dj = 1;
+      jend = min(j + g.jlen, nd);
+    } else {
+      const int r = (int)(t - nfull), row = lane / g.rem;
+      k = g.kfull * 64 + lane - row * g.rem;
+      i = r / g.njr;
+      const int j0 = (r - i * g.njr) * g.jlen * g.rpw;
+      dj = g.rpw;
+      jend = min(j0 + g.jlen * g.rpw, nd);
+      j = row < g.rpw ? j0 + row : jend;
+    }
+    const double2 e1 = a.ex[i], e3 = a.ez[k];
+    int cb = -1;  // the lane's bin and its sums
+    unsigned cn = 0;
+    double cs[NV];
+    auto flush = [&]() {
+      if (cb >= 0) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) atomicAdd(&acc[(size_t)cb * NV + v], cs[v]);
+        atomicAdd(&cacc[cb], cn);
+      }
+    };
+    const C2* p = gk + ((size_t)i * nd + j) * nz + k;
+    const size_t dp = (size_t)dj * nz;
+    for (; j < jend; j += U * dj, p += U * dp) {
+      C2 f1[U], f2[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const bool in = j + u * dj < jend;
+        const C2* q = in ? p + u * dp : p;
+        f1[u] = q[0];
+        f2[u] = a.nsub == 2 ? q[nh] : f1[u];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int ju = j + u * dj;
+        if (ju >= jend) break;
+        double kmod = 0, mu = 0;
+        const int b = mode_bin(a, i, ju, k, kmod, mu);
+        if (b != cb) {
+          flush();
+          cb = b;
+          cn = 0;
+#pragma unroll
+          for (int v = 0; v < NV; v++) cs[v] = 0.0;
+        }
+        if (b < 0) continue;
+        double dr, di;
+        power_mode<T, FLT, false>(a, i, ju, k, e1, a.ex[ju], e3, f1[u], f2[u], dr, di);
+        const double P = dr * dr + di * di;
+#pragma unroll
+        for (int l = 0; l < LS; l++) cs[l] += P * legendre_d(2 * l, mu);
+        cs[LS] += kmod;
+        cn++;
+      }
+    }
+    flush();
+  }
+  power_block_sums(lds, nw, Nk, NV, part, pcnt);
+}
+
+// Several tracers, more multipoles, or a window of |k|: segmented sums of 64 modes at a time.
+template <typename T>
 __global__ void k_power_bins(PowerArgs a, const typename cplx<T>::type* gk, double* part,
                              unsigned* pcnt) {
   extern __shared__ double lds[];
   using C2 = typename cplx<T>::type;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int NV = ONE ? 2 : a.NV, Nk = a.Nk, LS = ONE ? 1 : a.ls;
+  const int NV = a.NV, Nk = a.Nk, LS = a.ls;
   double* acc = lds + (size_t)wave * Nk * NV;
   unsigned* cacc = (unsigned*)(lds + (size_t)nw * Nk * NV) + (size_t)wave * Nk;
   for (int q = lane; q < Nk * NV; q += 64) acc[q] = 0.0;
@@ -1786,7 +1948,6 @@ __global__ void k_power_bins(PowerArgs a, const typename cplx<T>::type* gk, doub
       const long long row0 = __shfl(row, 0, 64);
       const int part = (int)(row - row0);
       const int nparts = (int)(__shfl(row, 63, 64) - row0) + 1;
-      const int fi = (2 * i < nd) ? i : i - nd, fj = (2 * j < nd) ? j : j - nd;
       double kmod = 0, mu = 0;
       const int b = k < nz ? mode_bin(a, i, j, k, kmod, mu) : -1;
       const bool valid = b >= 0;
@@ -1800,47 +1961,12 @@ __global__ void k_power_bins(PowerArgs a, const typename cplx<T>::type* gk, doub
       const bool tail = valid && (lane == 63 || bnext != b);
       // combined modes of every tracer
       double dr[8], di[8];
-      const int nt = ONE ? 1 : a.ntype;
-      if constexpr (ONE && sizeof(T) == 4) {
-        // one float tracer: the combine and deconvolution in float (the
-        // grid's precision), |delta|^2 summed in double below
-        if (valid) {
-          const double2 e1d = a.ex[i], e2d = a.ex[j], e3d = a.ez[k];
-          const float2 e1 = make_float2((float)e1d.x, (float)e1d.y);
-          const float2 e2 = make_float2((float)e2d.x, (float)e2d.y);
-          const float2 e3 = make_float2((float)e3d.x, (float)e3d.y);
-          const float wk = a.rwin ? (float)(a.Normk / (double)window_r<T>(a, fi, fj,
-                                                                           (2 * k < nd) ? k : k - nd))
-                                  : (float)a.wx[i] * (float)a.wx[j] * (float)a.wz[k] * (float)a.Normk;
-          const float pr = e1.x * e2.x - e1.y * e2.y, pi = e1.x * e2.y + e1.y * e2.x;
-          const float er = pr * e3.x - pi * e3.y, ei = pr * e3.y + pi * e3.x;
-          const C2 f1 = gk[id];
-          float re = (float)f1.x, im = (float)f1.y;
-          if (a.nsub == 2) {
-            const C2 f2 = gk[nh + id];
-            re = (re + ((float)f2.x * er - (float)f2.y * ei)) * 0.5f;
-            im = (im + ((float)f2.x * ei + (float)f2.y * er)) * 0.5f;
-          }
-          dr[0] = (double)(re * wk);
-          di[0] = (double)(im * wk);
-        }
-      } else if (valid) {
+      if (valid) {
         const double2 e1 = a.ex[i], e2 = a.ex[j], e3 = a.ez[k];
-        const double wk = a.rwin ? a.Normk / (double)window_r<T>(a, fi, fj, (2 * k < nd) ? k : k - nd)
-                                 : a.wx[i] * a.wx[j] * a.wz[k] * a.Normk;
-        // e^{-i theta} = e1 e2 e3
-        double pr = e1.x * e2.x - e1.y * e2.y, pi = e1.x * e2.y + e1.y * e2.x;
-        double er = pr * e3.x - pi * e3.y, ei = pr * e3.y + pi * e3.x;
-        for (int t = 0; t < nt; t++) {
-          const C2 f1 = gk[(size_t)(t * a.nsub) * nh + id];
-          double re = (double)f1.x, im = (double)f1.y;
-          if (a.nsub == 2) {
-            const C2 f2 = gk[(size_t)(t * a.nsub + 1) * nh + id];
-            re = (re + ((double)f2.x * er - (double)f2.y * ei)) / 2.0;
-            im = (im + ((double)f2.x * ei + (double)f2.y * er)) / 2.0;
-          }
-          dr[t] = re * wk;
-          di[t] = im * wk;
+        for (int t = 0; t < a.ntype; t++) {
+          const C2* f = gk + (size_t)(t * a.nsub) * nh + id;
+          power_mode<T, false, true>(a, i, j, k, e1, e2, e3, f[0], a.nsub == 2 ? f[nh] : f[0], dr[t],
+                               di[t]);
         }
       }
       // values: pair products x P_2l(mu), then |k|
@@ -1866,21 +1992,7 @@ __global__ void k_power_bins(PowerArgs a, const typename cplx<T>::type* gk, doub
         if (tail && part == p) cacc[b] += (unsigned)(lane - sstart + 1);
     }
   }
-  __syncthreads();
-  // fixed-order reduction over waves, one partial per block
-  double* out = part + (size_t)blockIdx.x * Nk * NV;
-  unsigned* cout = pcnt + (size_t)blockIdx.x * Nk;
-  for (int q = threadIdx.x; q < Nk * NV; q += blockDim.x) {
-    double s = 0.0;
-    for (int w = 0; w < nw; w++) s += lds[(size_t)w * Nk * NV + q];
-    out[q] = s;
-  }
-  for (int q = threadIdx.x; q < Nk; q += blockDim.x) {
-    unsigned s = 0;
-    unsigned* cbase = (unsigned*)(lds + (size_t)nw * Nk * NV);
-    for (int w = 0; w < nw; w++) s += cbase[(size_t)w * Nk + q];
-    cout[q] = s;
-  }
+  power_block_sums(lds, nw, Nk, NV, part, pcnt);
 }
 
 // One block per output value: 256 threads stride over the block partials,
@@ -2035,7 +2147,21 @@ void run_power(exh_ctx* c, const T* grid, int ntype, int nd, double L, int windo
   while (waves > 1 && per_wave * waves > 60 * 1024) waves--;
   EXH_REQUIRE(per_wave <= 60 * 1024, EXH_ERR_UNSUPPORTED,
               "Nk x spectra x multipoles too large for the LDS accumulator (%zu bytes)", per_wave);
+  // one tracer up to l = 4, no window of |k|: lines along j, at least 8 steps each and about one
+  // for each of 8192 waves
+  const bool lines = ntype == 1 && ls <= 3 && !a.rwin;
+  PowerLines g{};
   long long nrows = (long long)nd * nd;
+  if (lines) {
+    g.kfull = nz / 64;
+    g.rem = nz % 64;
+    g.rpw = g.rem ? 64 / g.rem : 0;
+    g.jlen = (int)std::min<long long>(std::max<long long>(8, nrows * std::max(g.kfull, 1) / 8192),
+                                      128);
+    g.njs = (nd + g.jlen - 1) / g.jlen;
+    g.njr = g.rem ? (nd + g.jlen * g.rpw - 1) / (g.jlen * g.rpw) : 0;
+    nrows = (long long)nd * (g.kfull * g.njs + g.njr);  // waves' tasks
+  }
   int nblocks = (int)std::min<long long>((nrows + waves - 1) / waves, 2048);
   size_t poff = 0;
   auto ptake = [&](size_t bytes) {
@@ -2052,12 +2178,16 @@ void run_power(exh_ctx* c, const T* grid, int ntype, int nd, double L, int windo
   unsigned long long* cnt = (unsigned long long*)(pbuf + o_cnt);
   {
     TimedScope ts(c, "power_bins");
-    if (NV == 2)
-      hipLaunchKernelGGL((k_power_bins<T, true>), dim3(nblocks), dim3(64 * waves),
-                         per_wave * waves, c->stream, a, gk, part, pcnt);
-    else
-      hipLaunchKernelGGL((k_power_bins<T, false>), dim3(nblocks), dim3(64 * waves),
-                         per_wave * waves, c->stream, a, gk, part, pcnt);
+    if (lines) {
+      auto k = ls == 1   ? (a.kbin == 4 ? k_power_lines<T, 1, 4> : k_power_lines<T, 1, 8>)
+               : ls == 2 ? (a.kbin == 4 ? k_power_lines<T, 2, 4> : k_power_lines<T, 2, 8>)
+                         : (a.kbin == 4 ? k_power_lines<T, 3, 4> : k_power_lines<T, 3, 8>);
+      hipLaunchKernelGGL(k, dim3(nblocks), dim3(64 * waves), per_wave * waves, c->stream, a, g, gk,
+                         part, pcnt);
+    } else {
+      hipLaunchKernelGGL(k_power_bins<T>, dim3(nblocks), dim3(64 * waves), per_wave * waves,
+                         c->stream, a, gk, part, pcnt);
+    }
     EXH_LAUNCH_CHECK();
   }
   {

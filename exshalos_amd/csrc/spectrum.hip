@@ -8,12 +8,16 @@
 //                order, accumulated per lattice tile in LDS (double) and
 //                flushed with one coalesced atomic per touched cell
 //  k_normalise   rho / rho_bar - 1 for unweighted grids (gridmodule.c:197-202)
-//  k_power_bins  one pass over the half-complex modes of all tracer grids:
+//  k_bin_*       the same weights for particles in any order, listed by grid
+//                tiles and summed per tile in LDS
+//  k_power_lines, k_power_bins  one pass over the half-complex modes of one
+//                tracer's or all tracers' grids:
 //                interlacing combine, window deconvolution and Normk
 //                (spectrum_h.c:112-157), the reference's mode mask and bin
 //                index (powermodule.c:47-55), and the pair products times
-//                P_2l(mu) (powermodule.c:66-72).  Each wavefront takes one
-//                (i, j) row at a time; along a row the bin index never
+//                P_2l(mu) (powermodule.c:66-72).  One tracer: each lane sums
+//                along j and adds where its bin changes.  Several: along a
+//                row the bin index never
 //                decreases, so bins are summed by a segmented scan across
 //                the 64 lanes and added by the segment's last lane into a
 //                wave-private LDS accumulator.  Waves and blocks are then
@@ -500,16 +504,13 @@ __global__ __launch_bounds__(TILE_THREADS) void k_deposit_tiles(
 // Window deposit: the tile's particles go into a fixed LDS window of
 // E = W + 2 h cells per axis (W = grid cells per tile side, margin h), placed at
 // the tile's mean displacement.  The mean is taken over one sampled
-// particle per wave, so no pass over all particles precedes the deposit;
-// each particle's wrap and division are evaluated once per sub-grid.  The
+// particle per wave, so no pass over all particles precedes the deposit.  The
 // rare stencil that leaves the window goes straight to the grid.  The
 // window is flushed row by row, lanes along z, one global atomic per
 // touched cell.
 //
 // A tile is PX x PY x PZ particles of the lattice and the window holds
-// ACC (float: ds_add_f32, or double: ds_add_f64) sums.  The flush's global
-// atomics scale with the window's cells per grid cell, (W + 2h)^3 / W^3 for
-// cubic tiles, so larger tiles in float windows issue fewer of them.
+// ACC sums (unsigned, float or double).
 static constexpr int WIN_THREADS = 1024;
 static constexpr int WIN_HALO = 4;  // default margin h
 
@@ -794,7 +795,7 @@ __global__ __launch_bounds__(WIN_THREADS, sizeof(ACC) == 4 ? 8 : 4) void k_depos
 // atomic per particle, cell and sub-grid, and those run at 26 G requests a
 // second whatever they touch (2 M particles, CIC, interlaced, 256^3 FP32:
 // 1.54 ms; binned 0.20 ms, of which the tiles' LDS atomics are the most).  Here
-// the grid is cut into tiles of at most BIN_EDGE^3 cells; every particle is
+// the grid is cut into tiles of at most 16 to 24 cells an edge; every particle is
 // listed with each tile that its stencils reach (1.4 on average for
 // interlaced CIC and 16^3 tiles), and one workgroup per tile sums its
 // particles in LDS, in double, and writes its own cells: no global atomic,
@@ -1757,48 +1758,46 @@ __device__ __forceinline__ void power_block_sums(const double* lds, int nw, int 
   }
 }
 
-// One tracer's combined, deconvolved mode, (f1 + f2 e^{-i theta}) / 2 over the
-// window: for the monopole of a float grid in float (the grid's precision),
-// else in double.
-template <typename T, bool FLT, bool RWIN>
-__device__ __forceinline__ void power_mode(const PowerArgs& a, int i, int j, int k,
-                                           const double2& e1d, const double2& e2d,
-                                           const double2& e3d,
-                                           const typename cplx<T>::type& f1,
-                                           const typename cplx<T>::type& f2, double& dr,
-                                           double& di) {
+// Phase e^{-i theta} = e1 e2 e3 of a mode and the factor that undoes the window
+// and normalises, the same for every tracer; F is the precision of the combine
+// (float for the monopole of a float grid, else double).
+template <typename F>
+struct ModePhase {
+  F er, ei, wk;
+};
+template <typename T, typename F, bool RWIN>
+__device__ __forceinline__ ModePhase<F> mode_phase(const PowerArgs& a, int i, int j, int k,
+                                                   const double2& e1d, const double2& e2d,
+                                                   const double2& e3d) {
   const int nd = a.nd;
-  const int fi = (2 * i < nd) ? i : i - nd, fj = (2 * j < nd) ? j : j - nd;
-  const int fk = (2 * k < nd) ? k : k - nd;
-  if constexpr (FLT) {
-    const float2 e1 = make_float2((float)e1d.x, (float)e1d.y);
-    const float2 e2 = make_float2((float)e2d.x, (float)e2d.y);
-    const float2 e3 = make_float2((float)e3d.x, (float)e3d.y);
-    const float wk = RWIN && a.rwin ? (float)(a.Normk / (double)window_r<T>(a, fi, fj, fk))
-                            : (float)a.wx[i] * (float)a.wx[j] * (float)a.wz[k] * (float)a.Normk;
-    const float pr = e1.x * e2.x - e1.y * e2.y, pi = e1.x * e2.y + e1.y * e2.x;
-    const float er = pr * e3.x - pi * e3.y, ei = pr * e3.y + pi * e3.x;
-    float re = (float)f1.x, im = (float)f1.y;
-    if (a.nsub == 2) {
-      re = (re + ((float)f2.x * er - (float)f2.y * ei)) * 0.5f;
-      im = (im + ((float)f2.x * ei + (float)f2.y * er)) * 0.5f;
-    }
-    dr = (double)(re * wk);
-    di = (double)(im * wk);
+  ModePhase<F> m;
+  if (RWIN && a.rwin) {
+    const int fi = (2 * i < nd) ? i : i - nd, fj = (2 * j < nd) ? j : j - nd;
+    const int fk = (2 * k < nd) ? k : k - nd;
+    m.wk = (F)(a.Normk / (double)window_r<T>(a, fi, fj, fk));
   } else {
-    const double wk = RWIN && a.rwin ? a.Normk / (double)window_r<T>(a, fi, fj, fk)
-                             : a.wx[i] * a.wx[j] * a.wz[k] * a.Normk;
-    // e^{-i theta} = e1 e2 e3
-    const double pr = e1d.x * e2d.x - e1d.y * e2d.y, pi = e1d.x * e2d.y + e1d.y * e2d.x;
-    const double er = pr * e3d.x - pi * e3d.y, ei = pr * e3d.y + pi * e3d.x;
-    double re = (double)f1.x, im = (double)f1.y;
-    if (a.nsub == 2) {
-      re = (re + ((double)f2.x * er - (double)f2.y * ei)) / 2.0;
-      im = (im + ((double)f2.x * ei + (double)f2.y * er)) / 2.0;
-    }
-    dr = re * wk;
-    di = im * wk;
+    m.wk = (F)a.wx[i] * (F)a.wx[j] * (F)a.wz[k] * (F)a.Normk;
   }
+  const F x1 = (F)e1d.x, y1 = (F)e1d.y, x2 = (F)e2d.x, y2 = (F)e2d.y, x3 = (F)e3d.x,
+          y3 = (F)e3d.y;
+  const F pr = x1 * x2 - y1 * y2, pi = x1 * y2 + y1 * x2;
+  m.er = pr * x3 - pi * y3;
+  m.ei = pr * y3 + pi * x3;
+  return m;
+}
+
+// A tracer's combined, deconvolved mode, (f1 + f2 e^{-i theta}) / 2 with two
+// sub-grids.
+template <typename F, typename C2>
+__device__ __forceinline__ void mode_combine(const ModePhase<F>& m, int nsub, const C2& f1,
+                                             const C2& f2, double& dr, double& di) {
+  F re = (F)f1.x, im = (F)f1.y;
+  if (nsub == 2) {
+    re = (re + ((F)f2.x * m.er - (F)f2.y * m.ei)) * (F)0.5;
+    im = (im + ((F)f2.x * m.ei + (F)f2.y * m.er)) * (F)0.5;
+  }
+  dr = (double)(re * m.wk);
+  di = (double)(im * m.wk);
 }
 
 // One tracer, LS multipoles, a window that is a product over the axes; KB is
@@ -1821,7 +1820,7 @@ __global__ __launch_bounds__(256) void k_power_lines(PowerArgs a, PowerLines g,
   extern __shared__ double lds[];
   using C2 = typename cplx<T>::type;
   constexpr int NV = LS + 1, U = 4;
-  constexpr bool FLT = LS == 1 && sizeof(T) == 4;
+  using F = typename std::conditional<LS == 1 && sizeof(T) == 4, float, double>::type;
   a.kbin = KB;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int Nk = a.Nk, nd = a.nd, nz = a.nz;
@@ -1889,7 +1888,8 @@ __global__ __launch_bounds__(256) void k_power_lines(PowerArgs a, PowerLines g,
         }
         if (b < 0) continue;
         double dr, di;
-        power_mode<T, FLT, false>(a, i, ju, k, e1, a.ex[ju], e3, f1[u], f2[u], dr, di);
+        mode_combine(mode_phase<T, F, false>(a, i, ju, k, e1, a.ex[ju], e3), a.nsub, f1[u], f2[u],
+                     dr, di);
         const double P = dr * dr + di * di;
 #pragma unroll
         for (int l = 0; l < LS; l++) cs[l] += P * legendre_d(2 * l, mu);
@@ -1963,10 +1963,13 @@ __global__ void k_power_bins(PowerArgs a, const typename cplx<T>::type* gk, doub
       double dr[8], di[8];
       if (valid) {
         const double2 e1 = a.ex[i], e2 = a.ex[j], e3 = a.ez[k];
+        const auto m = mode_phase<T, double, true>(a, i, j, k, e1, e2, e3);
         for (int t = 0; t < a.ntype; t++) {
           const C2* f = gk + (size_t)(t * a.nsub) * nh + id;
-          power_mode<T, false, true>(a, i, j, k, e1, e2, e3, f[0], a.nsub == 2 ? f[nh] : f[0], dr[t],
-                               di[t]);
+          const C2 f1 = f[0];
+          C2 f2 = f1;
+          if (a.nsub == 2) f2 = f[nh];
+          mode_combine(m, a.nsub, f1, f2, dr[t], di[t]);
         }
       }
       // values: pair products x P_2l(mu), then |k|

@@ -44,10 +44,12 @@ namespace exh {
 // reference's loop does not terminate for huge or infinite values).  Where L
 // is below the rounding of x / L * L (|x| beyond 1e7 boxes in float), the
 // difference may lie anywhere and says nothing of the position: 0 is taken.
-// Non-finite input returns -1, which the callers skip.
+// Non-finite input is returned as it is, and the callers skip the tracer: a
+// position that becomes so by the redshift-space shift is still seen by the
+// test that follows its wrap.
 template <typename T>
 __device__ inline T wrap_while(T x, T L) {
-  if (!isfinite(x)) return (T)-1;
+  if (!isfinite(x)) return x;
   if (x >= (T)2 * L || x < -L) {
     const T r = x - floor(x / L) * L;
     x = r >= -L && r < (T)2 * L ? r : (T)0;
@@ -64,6 +66,11 @@ __device__ inline T wrap_while(T x, T L) {
 template <typename T>
 __device__ inline void atomic_add_t(T* p, T v) {
   unsafeAtomicAdd(p, v);
+}
+
+template <typename T>
+__device__ __forceinline__ bool finite3(const T* x) {
+  return isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]);
 }
 
 template <typename T>
@@ -158,7 +165,7 @@ __global__ void k_deposit(const T* pos, const T* vel, const T* mass, const int* 
     T m = mass ? mass[j] : (T)1;
     T p[3];
     for (int a = 0; a < 3; a++) p[a] = wrap_while<T>(x[a], L);
-    if (p[0] < (T)0 || p[1] < (T)0 || p[2] < (T)0) continue;  // non-finite position
+    if (!finite3(p)) continue;
     T* g = grid + (size_t)t * nsub * ng;
     if (WIN == 1) dep_ngp(g, p, nd, Ld, m);
     if (WIN == 2) dep_cic(g, p, nd, Ld, m);
@@ -260,7 +267,7 @@ __global__ void k_deposit_sphere(const T* pos, const T* vel, const T* mass, cons
     const T m = mass ? mass[j] : (T)1;
     T p[3];
     for (int a = 0; a < 3; a++) p[a] = wrap_while<T>(x[a], L);
-    if (p[0] < (T)0 || p[1] < (T)0 || p[2] < (T)0) continue;  // non-finite position
+    if (!finite3(p)) continue;
     T* g = grid + (size_t)t * nsub * ng;
     atomicAdd(&sh[t * nsub], dep_sphere<T, EXPW>(g, p, nd, L, Ld, R, Rt, m));
     if (nsub == 2) {
@@ -419,7 +426,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_deposit_tiles(
     size_t j = ((size_t)(tx * TILE_L + a) * nL + (ty * TILE_L + b)) * nL + (tz * TILE_L + c);
     T x[3] = {pos[3 * j], pos[3 * j + 1], pos[3 * j + 2]};
     if (direction >= 0) x[direction] = wrap_while<T>(x[direction] + vel[3 * j + direction] * rsd, L);
-    ok[p] = isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]);
+    ok[p] = finite3(x);
     for (int q = 0; q < 3; q++) xs[p][q] = x[q];
     ms[p] = mass ? mass[j] : (T)1;
     myvalid += ok[p];
@@ -626,7 +633,6 @@ __device__ __forceinline__ void deposit_window_tile(
     }
     m = mass ? mass[j] : (T)1;
   };
-  auto valid = [](const T* x) { return isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]); };
   unsigned myvalid = 0;
   // displacement (in cells) of each wave's first particle: its cell relative
   // to the tile centre minus its lattice point's offset from the centre
@@ -638,7 +644,7 @@ __device__ __forceinline__ void deposit_window_tile(
 #pragma unroll
     for (int q = 0; q < 3; q++) {
       float r = 1e30f;
-      if (valid(x)) {
+      if (finite3(x)) {
         int cc = (int)floor(wrap_while<T>(x[q], L) / Ld);
         cc = cc < nd ? cc : nd - 1;
         r = (float)rel_cell(cc, qc[q], nd) -
@@ -689,7 +695,7 @@ __device__ __forceinline__ void deposit_window_tile(
       for (int p = 0; p < PPT; p++) {
         const T px[3] = {x[0], x[1], x[2]}, pm = m;
         if (p + 1 < PPT) load(p + 1, x, m);
-        if (!valid(px)) continue;
+        if (!finite3(px)) continue;
         if constexpr (!decltype(again)::value) myvalid += s == 0;
         int b[3], l[3];
         T w[3][NW];
@@ -859,7 +865,7 @@ __device__ __forceinline__ bool bin_particle(const BinParticles<T>& a, const Bin
       if (q == a.direction) x[q] = wrap_while<T>(x[q] + v, a.L);
   }
   t = a.type ? a.type[j] : 0;
-  return isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]) && (unsigned)t < (unsigned)g.ntype;
+  return finite3(x) && (unsigned)t < (unsigned)g.ntype;
 }
 
 // The one or two tiles per axis that the particle's stencils reach (at most
@@ -2325,7 +2331,7 @@ __global__ void k_deposit_adjoint(const T* S, int nL, double Lc, int nd, double 
     for (int a = 0; a < 3; a++) {
       D v = ((D)q[a] * Lc + Lc / 2.0) + (D)S[3 * p + a];
       x[a] = wrap_while<D>(v, L);
-      ok = ok && x[a] >= 0.0;
+      ok = ok && isfinite(x[a]);
     }
     double gx[3] = {0.0, 0.0, 0.0};
     if (ok && WIN == 2) {

@@ -559,8 +559,9 @@ struct WinAcc<unsigned> {
 // First cell (possibly -1) and weights of the window along one axis: the
 // values of stencil_q, in cell order.  CIC and TSC scale by the reciprocal of
 // the cell size (their weights are continuous in the position, so the
-// rounding of x / Ld against x * (1 / Ld) moves them by an ulp); NGP divides
-// as the reference does.
+// rounding of x / Ld against x * (1 / Ld) moves them by an ulp), TSC of a float
+// grid in double, far below a float weight's rounding; NGP and TSC of a double
+// grid divide as the reference does.
 template <typename T, int WIN>
 __device__ __forceinline__ int axis_window(T x, T Ld, T inv, double invd, int nd, T* w) {
   if constexpr (WIN == 1) {
@@ -577,7 +578,11 @@ __device__ __forceinline__ int axis_window(T x, T Ld, T inv, double invd, int nd
     w[1] = dx >= (T)0 ? far : near;
     return dx >= (T)0 ? xt : xt - 1;
   } else {
-    const double u = (double)x * invd - 0.5;
+    double u;
+    if constexpr (sizeof(T) == 8)
+      u = x / Ld - 0.5;
+    else
+      u = (double)x * invd - 0.5;
     const double cf = floor(u + 0.5);
     const double d = u - cf;
     w[0] = (T)(0.5 * (0.5 - d) * (0.5 - d));

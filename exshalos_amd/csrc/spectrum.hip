@@ -595,10 +595,11 @@ __device__ __forceinline__ int axis_window(T x, T Ld, T inv, double invd, int nd
 // Bound by vector instructions (204 a particle and sub-grid for TSC) and LDS
 // adds (6 cycles each with conflicts), with the flush's atomics close behind.
 // One cell and one range test per axis, the fixed-point scale folded into the
-// weights, adds without return values, the double division of TSC as a
-// product, and 64 registers in place of more than 64 (two workgroups per CU
-// instead of one): 775 -> 637 us for 256^3 particles, TSC, interlaced, FP32.
-template <typename T, int WIN, typename ACC, int PX, int PY, int PZ>
+// weights, adds without return values, the double division of a float grid's
+// TSC as a product, and 64 registers in place of more than 64 (two workgroups
+// per CU instead of one): 775 -> 637 us for 256^3 particles, TSC, interlaced,
+// FP32.
+template <typename T, int WIN, typename ACC, int PX, int PY, int PZ, bool KEEP>
 __device__ __forceinline__ void deposit_window_tile(
     int tile, const T* pos, const T* vel, const T* mass, int nL, int nd, int Wx, int Wy, int Wz,
     int wh, T L, T Lb, int direction, T rsd, int nsub, T* grid, unsigned long long* counts) {
@@ -621,9 +622,8 @@ __device__ __forceinline__ void deposit_window_tile(
   // tile centre in grid cells: the middle of the grid tile of the same index
   const int qc[3] = {tx * Wx + Wx / 2, ty * Wy + Wy / 2, tz * Wz + Wz / 2};
   if (threadIdx.x == 0) nvalid = 0;
-  // particle p of this thread, after the redshift-space shift.  Positions are
-  // read again for every filling (48 KB a tile, from the L2): kept in registers
-  // they cost the second workgroup of a CU.
+  // particle p of this thread, after the redshift-space shift: kept in
+  // registers, or read again for every filling (48 KB a tile, from the L2)
   auto load = [&](int p, T* x, T& m) {
     const int lin = threadIdx.x + p * WIN_THREADS;
     const int c = lin % PZ, b = (lin / PZ) % PY, a = lin / (PZ * PY);
@@ -638,14 +638,19 @@ __device__ __forceinline__ void deposit_window_tile(
     }
     m = mass ? mass[j] : (T)1;
   };
+  T xk[KEEP ? PPT : 1][3], mk[KEEP ? PPT : 1];
+  if constexpr (KEEP) {
+#pragma unroll
+    for (int p = 0; p < PPT; p++) load(p, xk[p], mk[p]);
+  }
   unsigned myvalid = 0;
   // displacement (in cells) of each wave's first particle: its cell relative
   // to the tile centre minus its lattice point's offset from the centre
   if ((threadIdx.x & 63) == 0) {
     const int lin = threadIdx.x;
     const int lat[3] = {lin / (PZ * PY), (lin / PZ) % PY, lin % PZ};
-    T x[3], m;
-    load(0, x, m);
+    T x[3] = {xk[0][0], xk[0][1], xk[0][2]}, m;
+    if constexpr (!KEEP) load(0, x, m);
 #pragma unroll
     for (int q = 0; q < 3; q++) {
       float r = 1e30f;
@@ -695,11 +700,16 @@ __device__ __forceinline__ void deposit_window_tile(
       for (int v = threadIdx.x; v < vol; v += WIN_THREADS) box[v] = (ACC)0;
       __syncthreads();
       T x[3], m;
-      load(0, x, m);
-#pragma unroll 1
+      if constexpr (!KEEP) load(0, x, m);
+#pragma unroll(KEEP ? PPT : 1)
       for (int p = 0; p < PPT; p++) {
+        if constexpr (KEEP) {
+          x[0] = xk[p][0], x[1] = xk[p][1], x[2] = xk[p][2], m = mk[p];
+        }
         const T px[3] = {x[0], x[1], x[2]}, pm = m;
-        if (p + 1 < PPT) load(p + 1, x, m);
+        if constexpr (!KEEP) {
+          if (p + 1 < PPT) load(p + 1, x, m);
+        }
         if (!finite3(px)) continue;
         if constexpr (!decltype(again)::value) myvalid += s == 0;
         int b[3], l[3];
@@ -790,13 +800,14 @@ __device__ __forceinline__ void deposit_window_tile(
 
 // One workgroup per tile, or (EXH_DEPOSIT_WG) fewer workgroups that walk the
 // tiles, leaving CUs to the kernels of other streams.
-template <typename T, int WIN, typename ACC, int PX, int PY, int PZ>
-__global__ __launch_bounds__(WIN_THREADS, sizeof(ACC) == 4 ? 8 : 4) void k_deposit_window(
+template <typename T, int WIN, typename ACC, int PX, int PY, int PZ, bool KEEP, int WAVES>
+__global__ __launch_bounds__(WIN_THREADS, WAVES) void k_deposit_window(
     const T* pos, const T* vel, const T* mass, int nL, int nd, int Wx, int Wy, int Wz, int wh,
     T L, T Lb, int direction, T rsd, int nsub, T* grid, unsigned long long* counts, int ntiles) {
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    deposit_window_tile<T, WIN, ACC, PX, PY, PZ>(tile, pos, vel, mass, nL, nd, Wx, Wy, Wz, wh, L,
-                                                 Lb, direction, rsd, nsub, grid, counts);
+    deposit_window_tile<T, WIN, ACC, PX, PY, PZ, KEEP>(tile, pos, vel, mass, nL, nd, Wx, Wy, Wz,
+                                                       wh, L, Lb, direction, rsd, nsub, grid,
+                                                       counts);
     __syncthreads();
   }
 }
@@ -1256,12 +1267,12 @@ void* noalloc_grid_scratch(int device) {
 // accumulator (EXH_DEPOSIT_ACC: 1 fixed point, the default for float grids
 // without masses; 8 double; 4 float).  Two 16^3 workgroups of 55 KB and 64
 // registers share a CU.  The whole call (zero, deposit, normalise) at nd = nL
-// = 512, CIC, interlaced, takes 3.28 ms with 16^3 tiles; longer ones in z,
-// which issue up to a third fewer atomics, take 3.41 (16 x 16 x 32, one
-// workgroup per CU), 3.74 (16 x 8 x 32) and 3.84 ms (8 x 8 x 64).  Float sums
-// are no choice: ds_add_f32 runs far slower than ds_add_u32 or ds_add_f64
-// here (16^3: 12.6 ms against 3.6).  Beside the halo finder's sort larger
-// workgroups hold CUs long enough to slow the sort.
+// = 512, FP32, CIC, interlaced, LPT positions, takes 3.28 ms with 16^3 tiles,
+// 3.28 with 32 x 16 x 16 and 3.02 with 32 x 32 x 16, whose windows issue the
+// fewest atomics; small boxes leave CUs without one of the larger tiles (64^3:
+// 52, 63 and 84 us), and beside the halo finder's sort larger workgroups hold
+// CUs long enough to slow the sort.  16^3 tiles summed in double take 4.33 ms,
+// in float 12.1 (ds_add_f32 runs far slower than ds_add_u32 or ds_add_f64).
 struct WinShape {
   int px, py, pz;
 };
@@ -1302,14 +1313,32 @@ struct DepositWinArgs {
   int ntiles;
 };
 
+// Positions stay in registers where every CU has one tile at most, and with
+// two sub-grids, which read them twice, also where one workgroup fills a CU
+// anyway and there are few tiles a CU; else they are read again, in 64
+// registers (WAVES = 8) where the window lets two workgroups share a CU.
+// Whole call, read again against kept, us: FP32, CIC, two sub-grids, 96^3
+// (216 tiles) 69.6 and 65.0; TSC, 256^3 638 and 664.  FP64, CIC, two
+// sub-grids, 160^3 (1000 tiles) 206 and 193, 256^3 (4096) 671 and 681; one
+// sub-grid, with weights, 256^3 326 and 372.  32 x 32 x 16 particles, FP32,
+// CIC, two sub-grids, 192^3 (432 tiles) 246 and 239; one, 320^3 472 and 517.
 template <typename T, int WN, typename ACC, int PX, int PY, int PZ>
 static void launch_window(exh_ctx* c, unsigned nwg, int lds, const DepositWinArgs<T>& a) {
-  auto k = k_deposit_window<T, WN, ACC, PX, PY, PZ>;
-  EXH_CHECK_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    lds));
-  hipLaunchKernelGGL(k, dim3(nwg), dim3(WIN_THREADS), lds, c->stream, a.pos, a.vel, a.mass, a.nL,
-                     a.nd, a.Wx, a.Wy, a.Wz, a.wh, a.L, a.Lb, a.direction, a.rsd, a.nsub, a.grid,
-                     a.counts, a.ntiles);
+  constexpr bool MAY = sizeof(ACC) == 4 && PX * PY * PZ == 4 * WIN_THREADS;
+  const bool two = MAY && lds <= WIN_LDS_MAX / 2;
+  auto go = [&](auto k) {
+    EXH_CHECK_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      lds));
+    hipLaunchKernelGGL(k, dim3(nwg), dim3(WIN_THREADS), lds, c->stream, a.pos, a.vel, a.mass, a.nL,
+                       a.nd, a.Wx, a.Wy, a.Wz, a.wh, a.L, a.Lb, a.direction, a.rsd, a.nsub, a.grid,
+                       a.counts, a.ntiles);
+  };
+  const bool keep = nwg <= 256 || (!two && a.nsub == 2 && nwg <= 2048);
+  if (keep) return go(k_deposit_window<T, WN, ACC, PX, PY, PZ, true, 4>);
+  if constexpr (MAY) {
+    if (two) return go(k_deposit_window<T, WN, ACC, PX, PY, PZ, false, 8>);
+  }
+  go(k_deposit_window<T, WN, ACC, PX, PY, PZ, false, 4>);
 }
 
 template <typename T, int WN>

@@ -187,6 +187,13 @@ int exh_ctx_set_tunable(exh_ctx* c, int key, int value) {
     EXH_REQUIRE(value == 0 || value == 64, EXH_ERR_ARG, "halo claims must be 0 or 64 (got %d)",
                 value);
     c->tune_halo_claims = value;
+  } else if (key >= EXH_TUNE_BIN_MAX && key <= EXH_TUNE_BIN_ENTRIES) {
+    EXH_REQUIRE(value >= 0 && (key != EXH_TUNE_BIN_ENTRIES || value <= 128), EXH_ERR_ARG,
+                "bad limit of the binned deposit: %d", value);
+    (key == EXH_TUNE_BIN_MAX    ? c->tune_bin_max
+     : key == EXH_TUNE_BIN_READ ? c->tune_bin_read
+     : key == EXH_TUNE_BIN_ROOM ? c->tune_bin_room
+                                : c->tune_bin_entries) = value;
   } else {
     EXH_REQUIRE(false, EXH_ERR_ARG, "unknown tunable %d", key);
   }
@@ -201,6 +208,18 @@ int exh_ctx_halo_stats(exh_ctx* c, long long* out5) {
   out5[2] = c->stat_rounds;
   out5[3] = c->stat_sort_levels;
   out5[4] = c->stat_sort_doubling;
+  EXH_API_END
+}
+
+int exh_ctx_deposit_path(exh_ctx* c) {
+  EXH_API_BEGIN
+  check_ctx(c);
+  if (c->deposit_path != EXH_DEPOSIT_BINNED) return c->deposit_path;
+  EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
+  if (c->aux) EXH_CHECK_HIP(hipStreamSynchronize(c->aux));
+  int n = 0;
+  EXH_CHECK_HIP(hipMemcpy(&n, c->bin_total, sizeof(n), hipMemcpyDeviceToHost));
+  return n > c->bin_cap ? EXH_DEPOSIT_ATOMICS : EXH_DEPOSIT_BINNED;
   EXH_API_END
 }
 

@@ -174,6 +174,7 @@ struct exh_ctx {
   int tune_deposit_tile = 0;
   int tune_deposit_acc = 0;
   int tune_halo_claims = 0;
+  int tune_bin_max = 0, tune_bin_read = 0, tune_bin_room = 0, tune_bin_entries = 0;
   void* buf[exh::BUF_NSLOTS] = {};
   size_t cap[exh::BUF_NSLOTS] = {};
   // allocation number of each slot's current buffer (0: none yet)
@@ -212,6 +213,11 @@ struct exh_ctx {
   // halo finder statistics of the last run
   long long stat_peaks = 0, stat_candidates = 0, stat_rounds = 0, stat_sort_levels = 0,
             stat_sort_doubling = 0, stat_sort_async_open = 0;
+  // the last grid deposit: EXH_DEPOSIT_*; of a binned one the entries counted
+  // (on the device) and those set aside
+  int deposit_path = 0;
+  const int* bin_total = nullptr;
+  long long bin_cap = 0;
 };
 
 namespace exh {

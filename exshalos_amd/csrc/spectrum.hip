@@ -142,10 +142,19 @@ __device__ inline void dep_tsc(T* g, const T* x, int nd, T Ld, T m) {
   }
 }
 
+// Entries that were counted against those set aside: where there are more,
+// nothing is listed and the atomics of k_deposit run in its place.
+struct BinRoom {
+  const int* total = nullptr;
+  long long cap = 0;
+  __device__ __forceinline__ bool over() const { return total && *total > cap; }
+};
+
 template <typename T, int WIN>
 __global__ void k_deposit(const T* pos, const T* vel, const T* mass, const int* type,
                           long long np, int nd, T L, T Lb, int direction, T rsd, int nsub,
-                          T* grid, unsigned long long* counts) {
+                          T* grid, unsigned long long* counts, BinRoom room) {
+  if (room.total && !room.over()) return;  // the bins have done it
   const size_t ng = (size_t)nd * nd * nd;
   const T Ld = L / (T)nd;
   // particle counts per type (the normalisation's total mass): registers
@@ -835,8 +844,7 @@ static constexpr int BIN_PART = 16384;  // entries of a part
 static constexpr long long BIN_ATOMICS = 1 << 20;  // fewest atomics to bin for
 static constexpr long long BIN_NP = 1 << 27;       // particles (entries fit an int)
 static constexpr long long BIN_READ = 4 << 20;     // most particles with 8 entries set aside for each
-                                                   // where the host may read the count instead
-static constexpr size_t BIN_BYTES = 8ull << 30;    // most bytes of entries set aside unread
+static constexpr size_t BIN_BYTES = 8ull << 30;    // most bytes set aside for a count not read
 
 struct BinGeom {
   int nd, nt, ntile;  // cells and tiles per axis, tiles
@@ -962,8 +970,10 @@ __global__ __launch_bounds__(1024) void k_bin_count(BinParticles<T> a, BinGeom g
 template <typename T, int WIN>
 __global__ __launch_bounds__(1024) void k_bin_scatter(BinParticles<T> a, BinGeom g,
                                                       long long chunk, const int* off,
-                                                      const int* place, BinEntry<T>* out) {
+                                                      const int* place, BinRoom room,
+                                                      BinEntry<T>* out) {
   extern __shared__ int bin_lds[];
+  if (room.over()) return;
   const int* pl = place + (size_t)blockIdx.x * g.bins;
   for (int b = threadIdx.x; b < g.bins; b += blockDim.x) bin_lds[b] = off[b] + pl[b];
   __syncthreads();
@@ -1020,8 +1030,10 @@ __global__ __launch_bounds__(256) void k_bin_deposit(BinGeom g, const BinEntry<T
                                                      const int* off, const int* slot, T L, T Lb,
                                                      int nsub, bool norm,
                                                      const unsigned long long* nvalid,
-                                                     double* partial, int pitch, T* grid) {
+                                                     double* partial, int pitch, BinRoom room,
+                                                     T* grid) {
   extern __shared__ double bin_sum[];
+  if (room.over()) return;
   constexpr int NW = WIN == 1 ? 1 : (WIN == 2 ? 2 : 3);
   int b = blockIdx.x, e0, e1, sl = -1;
   if (b < g.bins) {
@@ -1097,8 +1109,10 @@ __global__ __launch_bounds__(256) void k_bin_deposit(BinGeom g, const BinEntry<T
 template <typename T>
 __global__ __launch_bounds__(256) void k_bin_merge(BinGeom g, const int* slot, int nsub, bool norm,
                                                    const unsigned long long* nvalid,
-                                                   const double* partial, int pitch, T* grid) {
+                                                   const double* partial, int pitch, BinRoom room,
+                                                   T* grid) {
   const int sl = blockIdx.x;
+  if (room.over()) return;
   if (sl >= slot[g.bins]) return;
   int lo = 0, hi = g.bins;
   while (hi - lo > 1) {
@@ -1140,9 +1154,20 @@ __global__ void k_zero16(T* g, size_t n) {
   for (size_t i = nv * 16 / sizeof(T) + t0; i < n; i += st) g[i] = (T)0;
 }
 
+// The grids of a deposit whose entries found no room, zeroed for the atomics.
+template <typename T>
+__global__ void k_zero_over(T* g, size_t n, BinRoom room) {
+  if (!room.over()) return;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
+       i += (size_t)gridDim.x * blockDim.x)
+    g[i] = (T)0;
+}
+
 // grid (blockIdx.y) of ngrids: delta = rho / (M / ng) - 1
 template <typename T>
-__global__ void k_normalise(T* grid, size_t ng, int nsub, const unsigned long long* counts) {
+__global__ void k_normalise(T* grid, size_t ng, int nsub, const unsigned long long* counts,
+                            BinRoom room) {
+  if (room.total && !room.over()) return;
   const double M = (double)counts[blockIdx.y / nsub];
   const double mean = M / (double)ng;
   T* g = grid + (size_t)blockIdx.y * ng;
@@ -1373,14 +1398,15 @@ static void launch_window_any(exh_ctx* c, int window, int acc, const WinShape& w
 
 // Tiles of the binned deposit: the smallest edge (16, 20 or 24 cells) whose
 // bins fit the LDS counters; 0 bins where none does.
-static BinGeom bin_geom(int nd, int ntype) {
+static BinGeom bin_geom(const exh_ctx* c, int nd, int ntype) {
+  const int most = c->tune_bin_max ? std::min(c->tune_bin_max, BIN_MAX) : BIN_MAX;
   BinGeom g{};
   g.nd = nd;
   g.ntype = ntype;
   for (int edge = 16; edge <= 24; edge += 4) {
     g.nt = (nd + edge - 1) / edge;
     const long long bins = (long long)g.nt * g.nt * g.nt * ntype;
-    if (bins > BIN_MAX) continue;
+    if (bins > most) continue;
     g.ntile = g.nt * g.nt * g.nt;
     g.bins = (int)bins;
     g.dnd = fast_div((unsigned)nd);
@@ -1389,30 +1415,48 @@ static BinGeom bin_geom(int nd, int ntype) {
   return g;
 }
 
-// The host may wait for the number of entries: not while the stream is
-// captured, nor on the aux stream, where it must run ahead of the halo finder.
-static bool may_read_counts(const exh_ctx* c) {
-  if (c->stream == c->aux) return false;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(c->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
-}
-
-// The entries' buffer; null where it would take more than a quarter of the
-// memory that is free, and the atomics then need none.
-static char* bin_entries_buf(exh_ctx* c, size_t bytes) {
-  if (c->cap[BUF_BIN_ENT] < bytes) {
-    size_t avail = 0, total = 0;
-    if (hipMemGetInfo(&avail, &total) != hipSuccess ||
-        bytes > (avail + c->cap[BUF_BIN_ENT]) / 4)
-      return nullptr;
-  }
-  return (char*)ctx_buf(c, BUF_BIN_ENT, bytes);
+// Whether the entries' buffer may take `bytes`: it has them, or they are at
+// most a quarter of the memory that is free (the atomics need none).
+static bool bin_fits(const exh_ctx* c, size_t bytes) {
+  if (c->tune_bin_room) return bytes <= (size_t)c->tune_bin_room << 20;
+  if (bytes <= c->cap[BUF_BIN_ENT]) return true;
+  size_t avail = 0, total = 0;
+  return hipMemGetInfo(&avail, &total) == hipSuccess &&
+         bytes <= (avail + c->cap[BUF_BIN_ENT]) / 4;
 }
 
 // False where the entries find no room: nothing of the grid is written then.
+//
+// Up to BIN_READ particles, room for the most entries there can be (8 each) is
+// set aside.  Above, the host reads their number, unless the call runs on the
+// second stream, where it must go ahead of the halo finder: there 2 a particle
+// are set aside (LPT particles of 4 Mpc/h cells have 1.3 with CIC and 1.6 with
+// TSC), and the device goes over to the atomics where they do not suffice
+// (200^3 chain, FP32, CIC: 3.3 ms in bins, 7.2 after an overflow, 8.0 with
+// atomics alone).  Whether there is room is decided before the first launch,
+// except for a number that is read where one entry a particle would fit.
+// Chains of sides that the tiles do not divide, 8 entries a particle counted
+// first against 2: FP64, 330^3 30.6 -> 13.1 ms (refused after the count), FP32,
+// 350^3 10.2 ms both, 9.1 -> 5.0 GB held.
 template <typename T, int WIN>
 static bool run_binned(exh_ctx* c, const BinParticles<T>& a, const BinGeom& g, T* grid,
                        unsigned long long* counts) {
+  const bool all = a.np <= (c->tune_bin_read ? c->tune_bin_read : BIN_READ);
+  const bool read = !all && !(c->aux && c->stream == c->aux);
+  const int edge = (g.nd + g.nt - 1) / g.nt, pitch = edge * edge * edge;
+  long long most = 8 * a.np;  // a particle's stencils reach at most 8 tiles
+  // a split bin has more than BIN_PART entries, so its parts hold at least
+  // half of BIN_PART on average
+  auto slots = [&]() { return (int)(2 * most / BIN_PART); };
+  auto entry_bytes = [&]() { return ((size_t)most * sizeof(BinEntry<T>) + 255) & ~(size_t)255; };
+  auto bytes = [&]() { return entry_bytes() + (size_t)slots() * a.nsub * pitch * 8; };
+  if (read) {
+    most = a.np;
+  } else if (!all) {
+    most = a.np * (c->tune_bin_entries ? c->tune_bin_entries : 32) / 16;
+    if (bytes() > BIN_BYTES) return false;
+  }
+  if (!bin_fits(c, bytes())) return false;
   // particles per workgroup of the counting passes: at least 4 a thread, and
   // at least as many as there are counters to clear
   const long long chunk =
@@ -1446,38 +1490,49 @@ static bool run_binned(exh_ctx* c, const BinParticles<T>& a, const BinGeom& g, T
                      g.bins, parts);
   EXH_LAUNCH_CHECK();
   exclusive_scan<int>(c, parts, slot, g.bins, BUF_BIN_SCAN);
-  long long most = 8 * a.np;  // a particle's stencils reach at most 8 tiles
-  if (a.np > BIN_READ && may_read_counts(c)) {
+  if (read) {
     int* h = (int*)ctx_pinned(c, 256);
     EXH_CHECK_HIP(hipMemcpyAsync(h, off + g.bins, 4, hipMemcpyDeviceToHost, c->stream));
     EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
     most = h[0];
+    if (!bin_fits(c, bytes())) return false;
   }
-  // a split bin has more than BIN_PART entries, so its parts hold at least
-  // half of BIN_PART on average
-  const int nslot = (int)(2 * most / BIN_PART);
-  const int edge = (g.nd + g.nt - 1) / g.nt, pitch = edge * edge * edge;
-  const size_t eb = ((size_t)most * sizeof(BinEntry<T>) + 255) & ~(size_t)255;
-  if (a.np > BIN_READ && eb > BIN_BYTES && !may_read_counts(c)) return false;
-  char* ebuf = bin_entries_buf(c, eb + (size_t)nslot * a.nsub * pitch * 8);
-  if (!ebuf) return false;
+  const int nslot = slots();
+  const size_t eb = entry_bytes();
+  const BinRoom lim{off + g.bins, most};
+  char* ebuf = (char*)ctx_buf(c, BUF_BIN_ENT, bytes());
   BinEntry<T>* ent = (BinEntry<T>*)ebuf;
   double* partial = (double*)(ebuf + eb);
   auto ks = k_bin_scatter<T, WIN>;
   EXH_CHECK_HIP(hipFuncSetAttribute((const void*)ks, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     lds));
-  hipLaunchKernelGGL(ks, dim3(nb), dim3(1024), lds, c->stream, a, g, chunk, off, place, ent);
+  hipLaunchKernelGGL(ks, dim3(nb), dim3(1024), lds, c->stream, a, g, chunk, off, place, lim, ent);
   const int dlds = pitch * 8;
   const bool norm = !a.mass;
   auto kd = k_bin_deposit<T, WIN>;
   EXH_CHECK_HIP(hipFuncSetAttribute((const void*)kd, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     dlds));
   hipLaunchKernelGGL(kd, dim3((unsigned)(g.bins + nslot)), dim3(256), dlds, c->stream, g, ent, off,
-                     slot, a.L, a.Lb, a.nsub, norm, counts, partial, pitch, grid);
+                     slot, a.L, a.Lb, a.nsub, norm, counts, partial, pitch, lim, grid);
   if (nslot > 0)
     hipLaunchKernelGGL(k_bin_merge<T>, dim3((unsigned)nslot), dim3(256), 0, c->stream, g, slot,
-                       a.nsub, norm, counts, partial, pitch, grid);
+                       a.nsub, norm, counts, partial, pitch, lim, grid);
   EXH_LAUNCH_CHECK();
+  c->deposit_path = EXH_DEPOSIT_BINNED;
+  c->bin_total = off + g.bins;
+  c->bin_cap = most;
+  if (!all && !read) {
+    const size_t ng = (size_t)g.nd * g.nd * g.nd;
+    hipLaunchKernelGGL(k_zero_over<T>, dim3(2048), dim3(256), 0, c->stream, grid,
+                       ng * g.ntype * a.nsub, lim);
+    hipLaunchKernelGGL((k_deposit<T, WIN>), dim3(std::min(grid_for(a.np, 256), 8192u)), dim3(256),
+                       0, c->stream, a.pos, a.vel, a.mass, a.type, a.np, g.nd, a.L, a.Lb,
+                       a.direction, a.rsd, a.nsub, grid, (unsigned long long*)nullptr, lim);
+    if (norm)
+      hipLaunchKernelGGL(k_normalise<T>, dim3(1024, g.ntype * a.nsub), dim3(256), 0, c->stream,
+                         grid, ng, a.nsub, counts, lim);
+    EXH_LAUNCH_CHECK();
+  }
   return true;
 }
 
@@ -1502,6 +1557,7 @@ void run_grid(exh_ctx* c, const T* pos, const T* vel, const T* mass, const int* 
   unsigned long long* counts = scratch_dev ? (unsigned long long*)scratch_dev
                                            : (unsigned long long*)ctx_buf(c, BUF_GCNT, 64 * 8);
   EXH_REQUIRE(ntype <= 64, EXH_ERR_ARG, "at most 64 tracer types");
+  c->deposit_path = 0;
   const int nL = window == 3 || window == 4 ? 0 : lattice_side(np);
   const int nt = nL / TILE_L;
   const bool tiles = type == nullptr && nL >= TILE_L && nL % TILE_L == 0 && nd % nt == 0 &&
@@ -1518,7 +1574,7 @@ void run_grid(exh_ctx* c, const T* pos, const T* vel, const T* mass, const int* 
   const long long atomics = np * stencil * nsub;
   if (window != 3 && window != 4 && !tiles && !scratch_dev && np <= BIN_NP &&
       atomics >= (nL > 0 ? 3 * BIN_ATOMICS : BIN_ATOMICS)) {
-    const BinGeom g = bin_geom(nd, ntype);
+    const BinGeom g = bin_geom(c, nd, ntype);
     if (g.bins > 0) {
       TimedScope ts(c, window == 2 ? "cic_deposit" : (window == 1 ? "ngp_deposit" : "tsc_deposit"));
       hipLaunchKernelGGL(k_zero<unsigned long long>, dim3(1), dim3(64), 0, c->stream, counts,
@@ -1553,6 +1609,7 @@ void run_grid(exh_ctx* c, const T* pos, const T* vel, const T* mass, const int* 
     // spherical / exponential windows: normalised by the deposited weight
     double* wsum = scratch_dev ? (double*)scratch_dev : (double*)ctx_buf(c, BUF_GCNT, 128 * 8);
     hipLaunchKernelGGL(k_zero<double>, dim3(1), dim3(128), 0, c->stream, wsum, (size_t)128);
+    c->deposit_path = EXH_DEPOSIT_SPHERES;
     {
       TimedScope ts(c, window == 3 ? "sphere_deposit" : "exp_deposit");
       const unsigned gs = std::min(grid_for(np, 256), 65536u);
@@ -1619,7 +1676,9 @@ void run_grid(exh_ctx* c, const T* pos, const T* vel, const T* mass, const int* 
       const DepositWinArgs<T> da{pos, vel, mass, nL, nd, Wq[0], Wq[1], Wq[2], wh, Lf, Lb,
                                  direction, rsd, nsub, grid, counts, (int)nblk};
       launch_window_any<T>(c, window, acc, ws, nwg, win_lds, da);
+      c->deposit_path = EXH_DEPOSIT_WINDOWS;
     } else if (tiles) {
+      c->deposit_path = EXH_DEPOSIT_TILES;
       const int lds = deposit_lds_bytes();
       const int cap = lds / (int)sizeof(double);
       const unsigned nblk = (unsigned)nt * nt * nt;
@@ -1636,9 +1695,10 @@ void run_grid(exh_ctx* c, const T* pos, const T* vel, const T* mass, const int* 
       if (window == 5) EXH_DEPT(5);
 #undef EXH_DEPT
     } else {
+      c->deposit_path = EXH_DEPOSIT_ATOMICS;
 #define EXH_DEP(W)                                                                         \
   hipLaunchKernelGGL((k_deposit<T, W>), dim3(gsz), dim3(256), 0, c->stream, pos, vel, mass, \
-                     type, np, nd, Lf, Lb, direction, rsd, nsub, grid, counts)
+                     type, np, nd, Lf, Lb, direction, rsd, nsub, grid, counts, BinRoom{})
       if (window == 1) EXH_DEP(1);
       if (window == 2) EXH_DEP(2);
       if (window == 5) EXH_DEP(5);
@@ -1654,7 +1714,7 @@ void run_grid(exh_ctx* c, const T* pos, const T* vel, const T* mass, const int* 
                          dim3(256), 0, c->stream, grid, ng, nsub, counts);
     else
       hipLaunchKernelGGL(k_normalise<T>, dim3(grid_for(ng, 256 * 8), ntype * nsub), dim3(256),
-                         0, c->stream, grid, ng, nsub, counts);
+                         0, c->stream, grid, ng, nsub, counts, BinRoom{});
     EXH_LAUNCH_CHECK();
   }
 }

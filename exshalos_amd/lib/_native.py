@@ -29,6 +29,8 @@ ERRORS = {
 
 SRC_MODES, SRC_DELTA, SRC_DELTAK = 0, 1, 2
 TUNE_DEPOSIT_TILE, TUNE_DEPOSIT_ACC, TUNE_HALO_CLAIMS = 1, 2, 3
+TUNE_BIN_MAX, TUNE_BIN_READ, TUNE_BIN_ROOM, TUNE_BIN_ENTRIES = 4, 5, 6, 7
+DEPOSIT_ATOMICS, DEPOSIT_TILES, DEPOSIT_WINDOWS, DEPOSIT_BINNED, DEPOSIT_SPHERES = 1, 2, 3, 4, 5
 
 
 class Box(C.Structure):
@@ -68,6 +70,7 @@ _SIGS = {
     "exh_ctx_set_timing": (C.c_int, [_P, C.c_int]),
     "exh_ctx_timings": (C.c_int, [_P, C.c_char_p, C.c_int, _P, C.c_int]),
     "exh_ctx_halo_stats": (C.c_int, [_P, _P]),
+    "exh_ctx_deposit_path": (C.c_int, [_P]),
     "exh_ctx_set_tunable": (C.c_int, [_P, C.c_int, C.c_int]),
     "exh_box_init": (C.c_int, [C.POINTER(Box), C.c_int, C.c_int, C.c_int, C.c_double,
                                C.c_double, C.c_double, C.c_double, C.c_int]),

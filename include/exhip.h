@@ -127,15 +127,35 @@ int exh_ctx_timings(exh_ctx* ctx, char* names, int names_len, double* ms, int ma
  * grids without masses), 4 (float) or 8 (double).  Results agree to the
  * deposit's float rounding whatever the setting.  EXH_TUNE_HALO_CLAIMS: the
  * width of the halo growth rounds' per-cell claims, 0 (32 bits below 2^24
- * candidates, else 64) or 64; the catalogue is the same either way. */
+ * candidates, else 64) or 64; the catalogue is the same either way.
+ * EXH_TUNE_BIN_*: limits of the binned deposit of particles in any order.  MAX:
+ * most bins (tiles times types); tiles grow from 16 to 20 and 24 cells an edge
+ * to keep to it.  READ: most particles with room set aside for every entry
+ * there can be (above, the host reads their number, or, beside the halo
+ * finder, ENTRIES of them are set aside).  ROOM: most MiB of entries (0: a
+ * quarter of the free memory).  ENTRIES: per 16 particles. */
 #define EXH_TUNE_DEPOSIT_TILE 1
 #define EXH_TUNE_DEPOSIT_ACC 2
 #define EXH_TUNE_HALO_CLAIMS 3
+#define EXH_TUNE_BIN_MAX 4
+#define EXH_TUNE_BIN_READ 5
+#define EXH_TUNE_BIN_ROOM 6
+#define EXH_TUNE_BIN_ENTRIES 7
 int exh_ctx_set_tunable(exh_ctx* ctx, int key, int value);
 /* Halo-finder statistics of the last run (5 values): peaks, candidates,
  * growth rounds, device-wide sort levels, sort levels that needed pointer
  * doubling. */
 int exh_ctx_halo_stats(exh_ctx* ctx, long long* out5);
+/* How the context's last grid deposit was summed (0: none yet): atomics on the
+ * grid, lattice tiles in LDS boxes or in windows, bins of particles in any
+ * order, or the spherical and exponential windows' cubes.  Bins that found no
+ * room for their entries count as the atomics that took their place. */
+#define EXH_DEPOSIT_ATOMICS 1
+#define EXH_DEPOSIT_TILES 2
+#define EXH_DEPOSIT_WINDOWS 3
+#define EXH_DEPOSIT_BINNED 4
+#define EXH_DEPOSIT_SPHERES 5
+int exh_ctx_deposit_path(exh_ctx* ctx);
 
 /* set_cosmology + set_box (exshalos_h.c:43-106).  Lc_or_Mc < 100 is a cell
  * size in Mpc/h, > 1e5 a cell mass in Msun/h, anything else EXH_ERR_ARG. */

@@ -269,14 +269,6 @@ __host__ __device__ inline int isqrt_floor(int s) {
   return t;
 }
 
-// periodic single wrap (exshalos_h.c:22-30)
-__host__ __device__ inline int wrap1(int i, int j, int n) {
-  int r = i + j;
-  if (r >= n) r -= n;
-  if (r < 0) r += n;
-  return r;
-}
-
 // Division by a fixed divisor 1 <= d < 2^31 through a 64-bit reciprocal
 // m = ceil(2^64 / d): for 0 <= x < 2^31 the high 64 bits of x m are
 // exactly floor(x / d) (the error x (m - 2^64/d) / 2^64 < 2^-33 cannot

@@ -13,8 +13,9 @@
 //    lies inside that ball).  A candidate of one cell (G = 1) claims nothing:
 //    its centre's flag names its rank.  A candidate whose read ball
 //    (r^2 <= G) holds no claim and no centre of a denser pending candidate
-//    has seen its final flags: it commits.  The densest pending candidate always commits, so the rounds
-//    terminate; the result equals the sequential loop.
+//    has seen its final flags: it commits.  The densest pending candidate
+//    always commits, so the rounds terminate; the result equals the
+//    sequential loop.
 // 4. masses: taus uniforms by GF(2) jump-ahead, Tinker-integral splines
 //    (find_halos.c:442-476);
 // 5. halo positions from the displacement field (lpt.c:70-74, 245-255).
@@ -82,8 +83,8 @@ __device__ inline bool is_peak_at(const T* d, unsigned c, T v, int i, int j, int
 }
 
 // Peak flags of the thread's PK_ITEMS cells (cells past the grid: false), and
-// in the second byte those of its peaks below Bmin.  The pass also copies those cells of delta to eff, the growth rounds'
-// effective density.
+// in the second byte those of its peaks below Bmin.  The pass also copies
+// those cells of delta to eff, the growth rounds' effective density.
 template <typename T>
 __device__ inline unsigned peak_bits(const T* d, unsigned c0, unsigned ng, const PeakGeom& g,
                                      T Bmin, T* eff) {
@@ -476,7 +477,9 @@ __device__ __forceinline__ bool claimed(const unsigned long long* claim, unsigne
 // the kernel is vector issue in large boxes and that chain of loads and
 // ordered additions in small ones.
 static constexpr int GROW_MIN = 56;
-static constexpr int GROW_SHELLS = 9;  // last shell of the threads
+// Last shell of the threads.  The smallest table (sides of at least 4: 14
+// shells) holds their starts and those that the rows read ahead.
+static constexpr int GROW_SHELLS = 9;
 
 template <typename T, bool C32, int CPB>
 __global__ __launch_bounds__(256) void k_grow(GrowArgs<T> a, RoundLists rl,
@@ -738,7 +741,9 @@ __global__ __launch_bounds__(256) void k_grow(GrowArgs<T> a, RoundLists rl,
 // larger one.  The others are appended to their XCD's list of the next round
 // (in the order of the workgroups' atomics: the order of a list does not
 // change the result), in place of a count, a scan and a write pass (12 us a
-// round).  All rounds of the two boxes above: 283 -> 60 us, 2.6 -> 0.6 ms.
+// round).  All rounds, against one thread per candidate and those passes: a
+// 64^3 mock 283 -> 51 us, a 256^3 grid of 2 Mpc/h cells with an ellipsoidal
+// barrier 2640 -> 430 us.
 template <typename T, bool C32, int CPB>
 __global__ __launch_bounds__(256) void k_commit(GrowArgs<T> a, RoundLists rl,
                                                 unsigned long long tag_hi, int tmax) {
@@ -1058,7 +1063,10 @@ __global__ void k_flag_out(const int* flag, long long ng, const int* hidx, long 
 // larger one a row of 16 lanes that share its cells, so that no wave waits
 // for one thread's chain of loads through hundreds of cells.  The halos stand
 // in order of density, so a workgroup's are of similar size: HPB = 16 of them
-// (one a row) where there are few halos, else 256.
+// (one a row) where there are few halos, else 256.  A row adds 16 partial sums
+// (cells l, l + 16, ..) in a tree, not the cells in order: FP64 positions and
+// velocities of halos of several cells differ from a sum in order in the last
+// bits, like any two orders of a double sum.
 template <typename T, bool VEL>
 __device__ __forceinline__ void posh_store(const double* s, const double* v, int hc, int ci,
                                            int cj, int ck, T Lc, T L0, T L1, T L2, T* posh,
@@ -1603,9 +1611,9 @@ void run_halo_posh(exh_ctx* c, const exh_box* b, const T* S, const T* V, int lag
   const bool few = c->nh < 256 * 1024;
   auto kern = few ? (V ? k_halo_posh<T, true, 16> : k_halo_posh<T, false, 16>)
                   : (V ? k_halo_posh<T, true, 256> : k_halo_posh<T, false, 256>);
-  hipLaunchKernelGGL(kern, dim3(grid_for(c->nh, few ? 16 : 256)), dim3(256), 0, c->stream, st.hx, st.hcount,
-                     st.hr2, c->nh, st.sh, b->nd[0], b->nd[1], b->nd[2], S, V, (T)b->Lc,
-                     (T)b->L[0], (T)b->L[1], (T)b->L[2], lagrangian, (T*)st.posh,
+  hipLaunchKernelGGL(kern, dim3(grid_for(c->nh, few ? 16 : 256)), dim3(256), 0, c->stream, st.hx,
+                     st.hcount, st.hr2, c->nh, st.sh, b->nd[0], b->nd[1], b->nd[2], S, V,
+                     (T)b->Lc, (T)b->L[0], (T)b->L[1], (T)b->L[2], lagrangian, (T*)st.posh,
                      V ? (T*)st.velh : nullptr);
   EXH_LAUNCH_CHECK();
 }

@@ -149,7 +149,8 @@ __device__ inline long long wave_min_ll(long long v) {
 // Block 0 also clears the per-level counters (read by the host after the
 // previous level).
 template <typename K>
-__global__ __launch_bounds__(256) void k_tile_count(const K* keys, LevelBufs b, long long* tile_le) {
+__global__ __launch_bounds__(256) void k_tile_count(const K* keys, LevelBufs b,
+                                                    long long* tile_le) {
   __shared__ int shc[4];
   __shared__ long long shj[4];
   const long long t = blockIdx.x;
@@ -238,8 +239,9 @@ __device__ inline void push_child(const LevelBufs& b, long long cl, long long ch
 // queues the two children.
 template <typename K>
 __global__ __launch_bounds__(256) void k_tile_scatter(const K* keysA, const int* valsA, K* keysB,
-                                                      int* valsB, int* perm, LevelBufs b, const long long* tile_pre,
-                                                      int* arot, int* s0) {
+                                                      int* valsB, int* perm, LevelBufs b,
+                                                      const long long* tile_pre, int* arot,
+                                                      int* s0) {
   __shared__ int shw[4];
   const long long t = blockIdx.x;
   const int sg = b.tseg[t];
@@ -309,8 +311,8 @@ static constexpr int S0_DONE = 0x7fffffff;
 
 template <typename K>
 __global__ __launch_bounds__(256) void k_tile_chase(const K* keysA, const int* valsA, K* keysB,
-                                                    int* valsB, int* perm, LevelBufs b, const int* arot, int* s0,
-                                                    int* jmp, int cap) {
+                                                    int* valsB, int* perm, LevelBufs b,
+                                                    const int* arot, int* s0, int* jmp, int cap) {
   const long long t = blockIdx.x;
   const int sg = b.tseg[t];
   const SegInfo g = b.info[sg];
@@ -419,7 +421,8 @@ static int chase_cap() {
 // converged, since every pointer leads forward along its own chain.
 template <typename K>
 __global__ __launch_bounds__(256) void k_double_walk(const K* keysA, const int* valsA, K* keysB,
-                                                     int* valsB, int* perm, LevelBufs b, int* jmp, const int* s0, int guard) {
+                                                     int* valsB, int* perm, LevelBufs b, int* jmp,
+                                                     const int* s0, int guard) {
   const long long t = blockIdx.x;
   const int sg = b.tseg[t];
   if (!b.seg_need[sg]) return;
@@ -479,7 +482,8 @@ __global__ __launch_bounds__(256) void k_double_walk(const K* keysA, const int* 
 
 // Synchronous doubling round k (in place, same invariant as above); a
 // round whose predecessor left no entry open returns at once.
-__global__ __launch_bounds__(256) void k_double_round(LevelBufs b, int* jmp, int* round_open, int k) {
+__global__ __launch_bounds__(256) void k_double_round(LevelBufs b, int* jmp, int* round_open,
+                                                      int k) {
   if (k > 0 && !round_open[k - 1]) return;
   const long long t = blockIdx.x;
   const int sg = b.tseg[t];

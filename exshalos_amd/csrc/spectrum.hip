@@ -843,7 +843,7 @@ static constexpr int BIN_MAX = 36864;   // bins (tiles x types): counters in LDS
 static constexpr int BIN_PART = 16384;  // entries of a part
 static constexpr long long BIN_ATOMICS = 1 << 20;  // fewest atomics to bin for
 static constexpr long long BIN_NP = 1 << 27;       // particles (entries fit an int)
-static constexpr long long BIN_READ = 4 << 20;     // most particles with 8 entries set aside for each
+static constexpr long long BIN_READ = 4 << 20;     // most particles with 8 entries each
 static constexpr size_t BIN_BYTES = 8ull << 30;    // most bytes set aside for a count not read
 
 struct BinGeom {
@@ -1905,8 +1905,11 @@ __device__ __forceinline__ void mode_combine(const ModePhase<F>& m, int nsub, co
 // sum of every 64 modes and value (k_power_bins) the sums took most of them.
 // Here a lane keeps one k and steps along j, sums the modes of its current bin
 // in registers (a bin holds a few steps) and adds them to its wave's LDS sums
-// when the bin changes; a wave's sums are its own, so the order of the adds
-// does not depend on timing.  A wave takes 64 neighbouring k and `jlen` steps;
+// when the bin changes; a wave's sums are its own, so the order of its
+// instructions does not depend on timing.  Lanes that change to one bin at the
+// same step meet in one ds_add_f64: that equal calls give equal bits rests on
+// the LDS adding the lanes of an instruction in a fixed order, as it has in
+// every run.  A wave takes 64 neighbouring k and `jlen` steps;
 // the nz % 64 last k share a wave `rpw` rows at a time.  512^3, FP32,
 // interlaced: monopole, binned in double, 620 -> 464 us; l_max = 4, binned in
 // float, 1158 -> 520 us.
@@ -2023,77 +2026,75 @@ __global__ void k_power_bins(PowerArgs a, const typename cplx<T>::type* gk, doub
   const long long nchunks = (long long)((nh + 63) / 64);
   const long long gw = (long long)blockIdx.x * nw + wave, tw = (long long)gridDim.x * nw;
   for (long long ch = gw; ch < nchunks; ch += tw) {
-    {
-      const size_t id = (size_t)ch * 64 + lane;
-      int i = 0, j = 0, k = nz;  // k = nz: no mode
-      long long row = (long long)((nh - 1) / nz);
-      if (id < nh) {
-        if (nh < (1ull << 31)) {
-          const unsigned r = fdiv((unsigned)id, a.dz);
-          k = (int)((unsigned)id - r * (unsigned)nz);
-          i = (int)fdiv(r, a.dnd);
-          j = (int)(r - (unsigned)i * (unsigned)nd);
-          row = r;
-        } else {
-          k = (int)(id % nz);
-          const size_t r = id / nz;
-          j = (int)(r % nd);
-          i = (int)(r / nd);
-          row = (long long)r;
-        }
+    const size_t id = (size_t)ch * 64 + lane;
+    int i = 0, j = 0, k = nz;  // k = nz: no mode
+    long long row = (long long)((nh - 1) / nz);
+    if (id < nh) {
+      if (nh < (1ull << 31)) {
+        const unsigned r = fdiv((unsigned)id, a.dz);
+        k = (int)((unsigned)id - r * (unsigned)nz);
+        i = (int)fdiv(r, a.dnd);
+        j = (int)(r - (unsigned)i * (unsigned)nd);
+        row = r;
+      } else {
+        k = (int)(id % nz);
+        const size_t r = id / nz;
+        j = (int)(r % nd);
+        i = (int)(r / nd);
+        row = (long long)r;
       }
-      // the chunk's rows: within one row bins never decrease, so a bin has
-      // at most one segment per row; tails update the accumulators one row
-      // at a time (deterministically, without two lanes on one address)
-      const long long row0 = __shfl(row, 0, 64);
-      const int part = (int)(row - row0);
-      const int nparts = (int)(__shfl(row, 63, 64) - row0) + 1;
-      double kmod = 0, mu = 0;
-      const int b = k < nz ? mode_bin(a, i, j, k, kmod, mu) : -1;
-      const bool valid = b >= 0;
-      // segment bookkeeping
-      const int bprev = __shfl_up(b, 1, 64);
-      const bool head = valid && (lane == 0 || bprev != b);
-      const unsigned long long heads = __ballot(head);
-      const unsigned long long upto = heads & (lane == 63 ? ~0ull : ((2ull << lane) - 1));
-      const int sstart = upto ? 63 - __clzll((long long)upto) : 0;
-      const int bnext = __shfl_down(b, 1, 64);
-      const bool tail = valid && (lane == 63 || bnext != b);
-      // combined modes of every tracer
-      double dr[8], di[8];
-      if (valid) {
-        const double2 e1 = a.ex[i], e2 = a.ex[j], e3 = a.ez[k];
-        const auto m = mode_phase<T, double, true>(a, i, j, k, e1, e2, e3);
-        for (int t = 0; t < a.ntype; t++) {
-          const C2* f = gk + (size_t)(t * a.nsub) * nh + id;
-          const C2 f1 = f[0];
-          C2 f2 = f1;
-          if (a.nsub == 2) f2 = f[nh];
-          mode_combine(m, a.nsub, f1, f2, dr[t], di[t]);
-        }
-      }
-      // values: pair products x P_2l(mu), then |k|
-      for (int v = 0; v < NV; v++) {
-        double x = 0.0;
-        if (valid) {
-          if (v == NV - 1) {
-            x = kmod;
-          } else {
-            int pair = v / LS, l2 = 2 * (v % LS);
-            // pair index -> (l, m <= l) in the reference's order
-            int l = 0;
-            while ((l + 1) * (l + 2) / 2 <= pair) l++;
-            int m = pair - l * (l + 1) / 2;
-            x = (dr[l] * dr[m] + di[l] * di[m]) * legendre_d(l2, mu);
-          }
-        }
-        x = seg_scan_d(x, lane, sstart);
-        for (int p = 0; p < nparts; p++)
-          if (tail && part == p) acc[(size_t)b * NV + v] += x;
-      }
-      for (int p = 0; p < nparts; p++)
-        if (tail && part == p) cacc[b] += (unsigned)(lane - sstart + 1);
     }
+    // the chunk's rows: within one row bins never decrease, so a bin has
+    // at most one segment per row; tails update the accumulators one row
+    // at a time (deterministically, without two lanes on one address)
+    const long long row0 = __shfl(row, 0, 64);
+    const int part = (int)(row - row0);
+    const int nparts = (int)(__shfl(row, 63, 64) - row0) + 1;
+    double kmod = 0, mu = 0;
+    const int b = k < nz ? mode_bin(a, i, j, k, kmod, mu) : -1;
+    const bool valid = b >= 0;
+    // segment bookkeeping
+    const int bprev = __shfl_up(b, 1, 64);
+    const bool head = valid && (lane == 0 || bprev != b);
+    const unsigned long long heads = __ballot(head);
+    const unsigned long long upto = heads & (lane == 63 ? ~0ull : ((2ull << lane) - 1));
+    const int sstart = upto ? 63 - __clzll((long long)upto) : 0;
+    const int bnext = __shfl_down(b, 1, 64);
+    const bool tail = valid && (lane == 63 || bnext != b);
+    // combined modes of every tracer
+    double dr[8], di[8];
+    if (valid) {
+      const double2 e1 = a.ex[i], e2 = a.ex[j], e3 = a.ez[k];
+      const auto m = mode_phase<T, double, true>(a, i, j, k, e1, e2, e3);
+      for (int t = 0; t < a.ntype; t++) {
+        const C2* f = gk + (size_t)(t * a.nsub) * nh + id;
+        const C2 f1 = f[0];
+        C2 f2 = f1;
+        if (a.nsub == 2) f2 = f[nh];
+        mode_combine(m, a.nsub, f1, f2, dr[t], di[t]);
+      }
+    }
+    // values: pair products x P_2l(mu), then |k|
+    for (int v = 0; v < NV; v++) {
+      double x = 0.0;
+      if (valid) {
+        if (v == NV - 1) {
+          x = kmod;
+        } else {
+          int pair = v / LS, l2 = 2 * (v % LS);
+          // pair index -> (l, m <= l) in the reference's order
+          int l = 0;
+          while ((l + 1) * (l + 2) / 2 <= pair) l++;
+          int m = pair - l * (l + 1) / 2;
+          x = (dr[l] * dr[m] + di[l] * di[m]) * legendre_d(l2, mu);
+        }
+      }
+      x = seg_scan_d(x, lane, sstart);
+      for (int p = 0; p < nparts; p++)
+        if (tail && part == p) acc[(size_t)b * NV + v] += x;
+    }
+    for (int p = 0; p < nparts; p++)
+      if (tail && part == p) cacc[b] += (unsigned)(lane - sstart + 1);
   }
   power_block_sums(lds, nw, Nk, NV, part, pcnt);
 }

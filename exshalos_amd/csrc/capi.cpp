@@ -214,7 +214,7 @@ int exh_ctx_halo_stats(exh_ctx* c, long long* out5) {
 int exh_ctx_deposit_path(exh_ctx* c) {
   EXH_API_BEGIN
   check_ctx(c);
-  if (c->deposit_path != EXH_DEPOSIT_BINNED) return c->deposit_path;
+  if (c->deposit_path != EXH_DEPOSIT_BINNED || !c->bin_total) return c->deposit_path;
   EXH_CHECK_HIP(hipStreamSynchronize(c->stream));
   if (c->aux) EXH_CHECK_HIP(hipStreamSynchronize(c->aux));
   int n = 0;

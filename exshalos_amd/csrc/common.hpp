@@ -213,8 +213,8 @@ struct exh_ctx {
   // halo finder statistics of the last run
   long long stat_peaks = 0, stat_candidates = 0, stat_rounds = 0, stat_sort_levels = 0,
             stat_sort_doubling = 0, stat_sort_async_open = 0;
-  // the last grid deposit: EXH_DEPOSIT_*; of a binned one the entries counted
-  // (on the device) and those set aside
+  // the last grid deposit: EXH_DEPOSIT_*; of a binned one that may overflow,
+  // the entries counted (on the device) and those set aside
   int deposit_path = 0;
   const int* bin_total = nullptr;
   long long bin_cap = 0;

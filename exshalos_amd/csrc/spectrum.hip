@@ -1499,7 +1499,10 @@ static bool run_binned(exh_ctx* c, const BinParticles<T>& a, const BinGeom& g, T
   }
   const int nslot = slots();
   const size_t eb = entry_bytes();
-  const BinRoom lim{off + g.bins, most};
+  // tested on the device only where the entries may exceed it (every block of
+  // the passes would wait for the number: 244 -> 249 us for 2 M tracers)
+  const bool test = !all && !read;
+  const BinRoom lim = test ? BinRoom{off + g.bins, most} : BinRoom{};
   char* ebuf = (char*)ctx_buf(c, BUF_BIN_ENT, bytes());
   BinEntry<T>* ent = (BinEntry<T>*)ebuf;
   double* partial = (double*)(ebuf + eb);
@@ -1519,9 +1522,9 @@ static bool run_binned(exh_ctx* c, const BinParticles<T>& a, const BinGeom& g, T
                        a.nsub, norm, counts, partial, pitch, lim, grid);
   EXH_LAUNCH_CHECK();
   c->deposit_path = EXH_DEPOSIT_BINNED;
-  c->bin_total = off + g.bins;
-  c->bin_cap = most;
-  if (!all && !read) {
+  c->bin_total = lim.total;
+  c->bin_cap = lim.cap;
+  if (test) {
     const size_t ng = (size_t)g.nd * g.nd * g.nd;
     hipLaunchKernelGGL(k_zero_over<T>, dim3(2048), dim3(256), 0, c->stream, grid,
                        ng * g.ntype * a.nsub, lim);

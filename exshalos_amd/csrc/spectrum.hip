@@ -22,7 +22,8 @@
 //                the 64 lanes and added by the segment's last lane into a
 //                wave-private LDS accumulator.  Waves and blocks are then
 //                reduced in a fixed order: the double sums are bit-for-bit
-//                reproducible.
+//                reproducible (of one tracer as far as the LDS adds the lanes
+//                of one instruction in a fixed order).
 #include "common.hpp"
 #include "kernels.hpp"
 #include "util.hpp"
@@ -1499,8 +1500,8 @@ static bool run_binned(exh_ctx* c, const BinParticles<T>& a, const BinGeom& g, T
   }
   const int nslot = slots();
   const size_t eb = entry_bytes();
-  // tested on the device only where the entries may exceed it (every block of
-  // the passes would wait for the number: 244 -> 249 us for 2 M tracers)
+  // tested on the device only where the entries may exceed it: every block of
+  // the passes waits for the number first
   const bool test = !all && !read;
   const BinRoom lim = test ? BinRoom{off + g.bins, most} : BinRoom{};
   char* ebuf = (char*)ctx_buf(c, BUF_BIN_ENT, bytes());
